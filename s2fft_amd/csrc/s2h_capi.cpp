@@ -130,7 +130,7 @@ extern "C" int s2h_version(void) { return 1; }
 
 extern "C" size_t s2h_workspace_bytes(const s2h_plan* p, int batch) {
   if (!p || batch < 0) return 0;
-  size_t rows = (size_t)std::max(p->fwd_rows, p->inv_rows);
+  size_t rows = (size_t)std::max(p->pc_rows, p->inv_rows);
   if (p->fwd_kind != 0) rows += (size_t)p->fwd_in_rows;
   // + one flm-sized buffer for the adjoint of the conjugate fill
   const size_t flm = (size_t)p->d.L * (2 * p->d.L - 1);
@@ -340,32 +340,24 @@ int lat_inverse_stage(const s2h_plan* p, const void* flm, cplx* ftm, int batch, 
   return S2H_OK;
 }
 
-// Resampling arguments (MW / MWSS forward): phi-spectra of the input rows in
-// `spec`, the MWSS-at-2L grid into `ftm`.
-ResampleArgs resample_args(const s2h_plan* p, const cplx* spec, cplx* ftm, const PlaneSet* ps) {
-  const int L = p->d.L;
-  ResampleArgs ra{};
-  ra.in = spec;
-  ra.in_map_stride = (int64_t)p->fwd_in_rows * p->Mc;
-  ra.out = ftm;
-  ra.out_map_stride = (int64_t)p->fwd_rows * p->Mc;
-  ra.ncol = p->Mc;
-  ra.m_lo = p->m_lo;
-  ra.nm = p->nm;
-  ra.L = L;
-  ra.spin = ps ? ps->spin0 : p->d.spin;
-  ra.spin_step = ps ? ps->spin_step : 0;
-  ra.mw = p->fwd_kind == 1;
-  ra.nyq_split = p->d.reality ? 1 : 0;
-  ra.weights = p->fwd_weights;
-  ra.phi_factor = ra.mw ? (2.0 * L) / (2.0 * L - 1.0) : 1.0;
-  ra.lds = p->rs_info[3];
-  for (int i = 0; i < 3; ++i) {
-    ra.conv[i] = p->rs_info[i];
-    ra.chirp_off[i] = p->rs_chirp[i];
-  }
-  ra.pool = p->chirp;
-  return ra;
+// The theta step of the MW / MWSS forward: phi-spectra of the input rows
+// `spec` to the projection's rows `ftm` (or, adjoint, back).
+int theta_mix_stage(const s2h_plan* p, const PlaneSet* ps, cplx* spec, cplx* ftm, int batch,
+                    bool adjoint, hipStream_t s) {
+  const int64_t spec_map = (int64_t)p->fwd_in_rows * p->Mc, ftm_map = (int64_t)p->fwd_rows * p->Mc;
+  ThetaMixArgs t{};
+  t.in = adjoint ? ftm : spec;
+  t.in_map_stride = adjoint ? ftm_map : spec_map;
+  t.out = adjoint ? spec : ftm;
+  t.out_map_stride = adjoint ? spec_map : ftm_map;
+  t.ncol = p->Mc;
+  t.m_lo = p->m_lo;
+  t.spin = ps ? ps->spin0 : p->d.spin;
+  t.spin_step = ps ? ps->spin_step : 0;
+  t.adjoint = adjoint ? 1 : 0;
+  t.nyquist = p->d.reality ? 0 : 1;
+  ProfScope prof(S2H_KERNEL_RESAMPLE, s);
+  return hip_status(launch_theta_mix(p->mix.get(), t, batch, s));
 }
 
 // Plans whose forward and inverse share one ring grid without pole rows or
@@ -389,16 +381,12 @@ int forward_impl(const s2h_plan* p, const PlaneSet* ps, const void* f, int f_is_
   int st;
   cplx* ftm = static_cast<cplx*>(work);
   const bool resample = p->fwd_kind != 0;
-  // resampled forward: phi-spectrum of the input rows first, then the
-  // resampled MWSS-at-2L ftm after it in the workspace
+  // MW / MWSS: phi-spectrum of the input rows first, then the projection's
+  // rows after it in the workspace
   cplx* spec = ftm;
   if (resample) ftm = spec + (int64_t)batch * p->fwd_in_rows * p->Mc;
   if ((st = ring_analysis_stage(p, f, f_is_complex, resample ? spec : ftm, batch, s))) return st;
-  if (resample) {
-    const ResampleArgs ra = resample_args(p, spec, ftm, ps);
-    ProfScope prof(S2H_KERNEL_RESAMPLE, s);
-    if ((st = hip_status(launch_resample(ra, batch, s)))) return st;
-  }
+  if (resample && (st = theta_mix_stage(p, ps, spec, ftm, batch, false, s))) return st;
   return lat_forward_stage(p, ftm, flm, batch, precision, accumulate, s, false, ps);
 }
 
@@ -782,9 +770,8 @@ int forward_adjoint_impl(const s2h_plan* p, const PlaneSet* ps, const void* g, v
   }
   int64_t in_stride = ftm_stride;
   if (resample) {
-    const ResampleArgs ra = resample_args(p, spec, ftm, ps);
-    if ((st = hip_status(launch_resample_adjoint(ra, batch, s)))) return st;
-    in_stride = ra.in_map_stride;
+    if ((st = theta_mix_stage(p, ps, spec, ftm, batch, true, s))) return st;
+    in_stride = (int64_t)p->fwd_in_rows * p->Mc;
   }
 
   RingInvArgs r{};
@@ -1410,7 +1397,7 @@ extern "C" int s2h_compute_all_slices(const s2h_plan* p, const double* beta, int
 
 extern "C" size_t s2h_precompute_kernel_bytes(const s2h_plan* p, int forward) {
   if (!p || p->d.norm == S2H_NORM_NONE) return 0;
-  const size_t T = (size_t)(forward ? p->fwd_rows : p->inv_rows);
+  const size_t T = (size_t)(forward ? p->pc_rows : p->inv_rows);
   const size_t el = p->d.sampling == S2H_HEALPIX ? sizeof(cplx) : sizeof(double);
   return T * (size_t)p->d.L * (size_t)p->nm * el;
 }
@@ -1425,7 +1412,7 @@ extern "C" int s2h_precompute_kernel(const s2h_plan* p, int forward, double scal
   a.mstart = forward ? p->fwd_mstart : p->inv_mstart;
   a.coef = forward ? p->fwd_coef : p->inv_coef;
   a.theta = forward ? p->fwd_theta : p->inv_theta;
-  a.T = forward ? p->fwd_rows : p->inv_rows;
+  a.T = forward ? p->pc_rows : p->inv_rows;
   a.L = p->d.L;
   a.m_lo = p->m_lo;
   a.nm = p->nm;
@@ -1457,19 +1444,37 @@ extern "C" int s2h_precompute_forward(const s2h_plan* p, const void* kernel, int
   if ((st = ring_analysis_stage(p, f, f_is_complex, resample ? spec : ftm, batch, s, true)))
     return st;
   if (resample) {
-    ResampleArgs ra = resample_args(p, spec, ftm, nullptr);
-    ra.weights = nullptr;  // the kernel carries the quadrature weights
+    const int L = p->d.L;
+    ResampleArgs ra{};
+    ra.in = spec;
+    ra.in_map_stride = (int64_t)p->fwd_in_rows * p->Mc;
+    ra.out = ftm;
+    ra.out_map_stride = (int64_t)p->pc_rows * p->Mc;
+    ra.ncol = p->Mc;
+    ra.m_lo = p->m_lo;
+    ra.nm = p->nm;
+    ra.L = L;
+    ra.spin = p->d.spin;
+    ra.mw = p->fwd_kind == 1;
+    ra.nyq_split = p->d.reality ? 1 : 0;
+    ra.phi_factor = ra.mw ? (2.0 * L) / (2.0 * L - 1.0) : 1.0;
+    ra.lds = p->rs_info[3];
+    for (int i = 0; i < 3; ++i) {
+      ra.conv[i] = p->rs_info[i];
+      ra.chirp_off[i] = p->rs_chirp[i];
+    }
+    ra.pool = p->chirp;
     if ((st = hip_status(launch_resample(ra, batch, s)))) return st;
   }
   PcArgs a{};
   a.kernel = kernel;
   a.kernel_complex = kernel_is_complex ? 1 : 0;
-  a.T = p->fwd_rows;
+  a.T = p->pc_rows;
   a.L = p->d.L;
   a.m_lo = p->m_lo;
   a.nm = p->nm;
   a.y = ftm;
-  a.y_map_stride = (int64_t)p->fwd_rows * p->Mc;
+  a.y_map_stride = (int64_t)p->pc_rows * p->Mc;
   a.flm = static_cast<cplx*>(flm);
   a.flm_map_stride = flm_stride(p);
   a.scale = scale;

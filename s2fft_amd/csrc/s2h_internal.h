@@ -70,6 +70,7 @@ struct LatRing {
   double x;             // cos(theta_a)
   double c2;            // cos(theta_a / 2)
   double s2;            // sin(theta_a / 2)
+  double c2r, s2r;      // relative errors of c2 and s2: cos(theta_a / 2) = c2 (1 + c2r)
 };
 
 struct cplx {

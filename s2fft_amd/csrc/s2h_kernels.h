@@ -382,17 +382,28 @@ struct ResampleArgs {
   int L, spin;
   int mw;                   // 1: MW input (L rows), 0: MWSS input (L+1 rows)
   int nyq_split;            // real signals: split the theta-Nyquist bin (see kernel)
-  const double* weights;    // 2L+1 quadrature weights of MWSS at 2L (null: none)
   double phi_factor;        // 2L/(2L-1) for MW, 1 for MWSS
   int lds;                  // LDS elements (complex) per workgroup
   int conv[3];              // Bluestein lengths of the DFTs 2L-1, 2L, 4L (0 = mixed)
   int64_t chirp_off[3];
   const cplx* pool;
-  int spin_step;            // map b has spin + spin_step b (multi-plane launches)
 };
 hipError_t launch_resample(const ResampleArgs& a, int batch, hipStream_t s);
 hipError_t allow_large_lds_resample();
-hipError_t launch_resample_adjoint(const ResampleArgs& a, int batch, hipStream_t s);
-hipError_t allow_large_lds_resample_adjoint();
+
+// MW / MWSS forward: input rows -> the L + 1 weighted rows the projection
+// takes (or, adjoint, back), columns of both parities (s2h_theta_mix.hip).
+struct ThetaMix;
+struct ThetaMixArgs {
+  const cplx* in;           // [b][row][col], col <-> m = m_lo + col
+  int64_t in_map_stride;
+  cplx* out;
+  int64_t out_map_stride;
+  int ncol, m_lo;           // columns of both arrays
+  int spin, spin_step;      // map b has spin + spin_step b
+  int adjoint;
+  int nyquist;              // complex signals: the theta-Nyquist term at q = -L
+};
+hipError_t launch_theta_mix(const ThetaMix* x, const ThetaMixArgs& a, int batch, hipStream_t s);
 
 }  // namespace s2h

@@ -25,7 +25,7 @@ constexpr int kGroup = 4;        // steps whose coefficients are read from LDS t
 
 using lat::m_of_block;
 using lat::rescale;
-using lat::start_value;
+using lat::start_value_fp64;
 
 }  // namespace
 
@@ -62,7 +62,7 @@ __global__ void __launch_bounds__(kThreads) lat_inverse_kernel(LatArgs a) {
   int lscale = 0;
   if (valid) {
     rg = a.rings[p];
-    start_value(st, rg.c2, rg.s2, d, lscale);
+    start_value_fp64(st, rg, d, lscale);
   }
   const double x = rg.x;
 
@@ -213,7 +213,7 @@ __global__ void __launch_bounds__(kThreads) lat_forward_kernel(LatArgs a) {
     if (p < a.nrings) {
       const LatRing rg = a.rings[p];
       x[r] = rg.x;
-      start_value(st, rg.c2, rg.s2, d[r], ls[r]);
+      start_value_fp64(st, rg, d[r], ls[r]);
       const cplx fa = ftm[spec_row(rg.ta, a.ftm_ncol, a.ftm_tiled)];
       cplx fb = {0.0, 0.0};
       if (PAIRED && rg.tb >= 0 && rg.tb != rg.ta) fb = ftm[spec_row(rg.tb, a.ftm_ncol, a.ftm_tiled)];

@@ -56,6 +56,54 @@ __device__ __forceinline__ void start_value(const MStart& st, double c2, double 
   d = ldexp(v.m, v.e - 512 * ls);
 }
 
+// m 2^e (1 + r): a product that carries its rounding errors along in r.
+struct ExtR {
+  double m;
+  int e;
+  double r;
+};
+__device__ __forceinline__ ExtR extr_mul(ExtR a, ExtR b) {
+  const double p = a.m * b.m;
+  int e;
+  const double m = frexp(p, &e);
+  const double err = fma(a.m, b.m, -p) * __builtin_amdgcn_rcp(p);
+  return {m, a.e + b.e + e, a.r + b.r + (p != 0.0 ? err : 0.0)};
+}
+__device__ __forceinline__ ExtR extr_pow(ExtR x, int k) {
+  ExtR r = {0.5, 1, 0.0};
+  while (k) {
+    if (k & 1) r = extr_mul(r, x);
+    k >>= 1;
+    if (k) x = extr_mul(x, x);
+  }
+  return r;
+}
+
+// start_value for the FP64 kernels.  c2 and s2 rounded to FP64 and multiplied
+// up carry a relative error of about j eps into every d of their ring and m
+// (the largest error of the transforms: 5e-14 at L = 512); here the rounding
+// errors of c2, s2 and of every product are kept.  One power of c2 s2 and one
+// of the difference of the exponents (at most 2 |n|) in place of two powers.
+__device__ __forceinline__ void start_value_fp64(const MStart& st, const LatRing& rg, double& d,
+                                                 int& lscale) {
+  const Ext c = ext_of(rg.c2), s = ext_of(rg.s2);
+  const ExtR cr = {c.m, c.e, rg.c2r}, sr = {s.m, s.e, rg.s2r};
+  const int k = st.ecos < st.esin ? st.ecos : st.esin;
+  ExtR v = {st.kmant, st.kexp, 0.0};
+  if (k) v = extr_mul(v, extr_pow(extr_mul(cr, sr), k));
+  if (st.ecos > k) v = extr_mul(v, extr_pow(cr, st.ecos - k));
+  if (st.esin > k) v = extr_mul(v, extr_pow(sr, st.esin - k));
+  if (v.m == 0.0) {
+    d = 0.0;
+    lscale = 0;
+    return;
+  }
+  int ls = -((256 - v.e) >> 9);
+  if (ls > 0) ls = 0;
+  lscale = ls;
+  d = ldexp(fma(v.m, v.r, v.m), v.e - 512 * ls);
+}
+
 // Moves (d, dm1) down by 2^512 once |d| passes 2^256.  The recursion grows
 // by less than 2.5 per step, so checks every 32 steps cannot overflow.
 __device__ __forceinline__ void rescale(double& d, double& dm1, int& lscale) {

@@ -109,7 +109,7 @@ __global__ void __launch_bounds__(kMT) lat_forward_f64_kernel(LatArgs a) {
     if (base + lane < a.nrings) {
       const LatRing rg = a.rings[base + lane];
       x = rg.x;
-      start_value(st, rg.c2, rg.s2, d, ls);
+      lat::start_value_fp64(st, rg, d, ls);
     }
     // A operands: tile t, row i = lane % 16 -> (map 8t + i/2, re/im i%2), pair base + 4c + lane/16.
     // The wave's ring rows are staged in LDS (its d tile is free here), then

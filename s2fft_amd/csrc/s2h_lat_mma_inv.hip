@@ -70,7 +70,10 @@ __global__ void __launch_bounds__(kIT, 2) lat_inverse_mma_kernel(LatArgs a) {
   if (p < a.nrings) {
     const LatRing rg = a.rings[p];
     x = rg.x;
-    start_value(st, rg.c2, rg.s2, d, ls);
+    if constexpr (sizeof(T) == 8)
+      lat::start_value_fp64(st, rg, d, ls);
+    else
+      start_value(st, rg.c2, rg.s2, d, ls);
   }
 
   // accumulators: [map tile][16-pair tile q], even / odd l + m

@@ -440,7 +440,9 @@ hipError_t launch_cg_finish(const CgFinishArgs& a, int batch, hipStream_t s) {
 namespace s2h {
 
 // ------------------------------------------------------------------ resampling
-// MW / MWSS forward resampling in (theta, m) space, one workgroup per (m, map).
+// MW / MWSS resampling to the 2L + 1 rows that a stored precompute kernel
+// contracts, in (theta, m) space, one workgroup per (m, map) (the forward
+// transforms take the composed operators of s2h_theta_mix.hip instead).
 // s2fft/utils/resampling.py: mw_to_mwss (248-355) followed by
 // upsample_by_two_mwss (64-160).  Every step there is linear along theta per
 // phi-Fourier column m (the phi-rolls of the mirrored rows are (-1)^m), so
@@ -449,8 +451,8 @@ namespace s2h {
 //         phase e^{-i p pi/(2L-1)}, IDFT_{2L} -> rows 0..L of MWSS
 //   MWSS: extend L+1 rows to 2L with (-1)^(m+s) mirror, DFT_{2L}/(2L),
 //         zero-pad, IDFT_{4L} -> rows 0..2L of MWSS at 2L
-// then the quadrature weight of each output row and, for MW, the 2L/(2L-1)
-// of the phi zero-padding.
+// then, for MW, the 2L/(2L-1) of the phi zero-padding (the stored kernel
+// carries the quadrature weights).
 __device__ __forceinline__ void col_dft(double* re, double* im, int n, int conv, int64_t off,
                                         const cplx* pool, int sign) {
   if (conv == 0)
@@ -467,8 +469,7 @@ __global__ void __launch_bounds__(kThreads) resample_kernel(ResampleArgs a) {
   const int64_t b = blockIdx.y;
   double* re = smem;
   double* im = smem + a.lds;
-  const int spin_b = a.spin + a.spin_step * (int)b;
-  const double msgn = (((m + spin_b) % 2) + 2) % 2 ? -1.0 : 1.0;
+  const double msgn = (((m + a.spin) % 2) + 2) % 2 ? -1.0 : 1.0;
   const cplx* g = a.in + b * a.in_map_stride + col;
 
   int nrow;  // rows of the MWSS column at L now held in LDS
@@ -589,8 +590,7 @@ __global__ void __launch_bounds__(kThreads) resample_kernel(ResampleArgs a) {
   col_dft(re, im, 4 * L, a.conv[2], a.chirp_off[2], a.pool, +1);
   cplx* out = a.out + b * a.out_map_stride + col;
   for (int t = threadIdx.x; t <= 2 * L; t += kThreads) {
-    const double w = (a.weights ? a.weights[t] : 1.0) * a.phi_factor;
-    out[(int64_t)t * a.ncol] = {re[t] * w, im[t] * w};
+    out[(int64_t)t * a.ncol] = {re[t] * a.phi_factor, im[t] * a.phi_factor};
   }
 }
 
@@ -657,149 +657,6 @@ hipError_t launch_scale_pos_m(cplx* flm, int64_t map_stride, int L, int batch, d
   hipLaunchKernelGGL(scale_pos_m_kernel, dim3((L - 1 + kThreads - 1) / kThreads, L, batch),
                      dim3(kThreads), 0, s, flm, map_stride, L, factor);
   return hipGetLastError();
-}
-
-}  // namespace s2h
-
-namespace s2h {
-
-// Adjoint of resample_kernel (same column-per-workgroup layout, steps in
-// reverse with each step's adjoint): weights, zero-extension of the kept
-// rows, DFT for every IDFT, bin extraction for every zero-pad, IDFT/n for
-// every DFT/n, and folding of the mirrored rows.
-__global__ void __launch_bounds__(kThreads) resample_adjoint_kernel(ResampleArgs a) {
-  extern __shared__ double smem[];
-  const int L = a.L;
-  const int col = blockIdx.x;
-  const int m = a.m_lo + col;
-  const int64_t b = blockIdx.y;
-  double* re = smem;
-  double* im = smem + a.lds;
-  const int spin_b = a.spin + a.spin_step * (int)b;
-  const double msgn = (((m + spin_b) % 2) + 2) % 2 ? -1.0 : 1.0;
-  constexpr int kPer = kMaxConvLen / kThreads;
-
-  // rows 0..2L of the upsampled grid, weighted, zero-extended to 4L
-  const cplx* g = a.out + b * a.out_map_stride + col;
-  for (int t = threadIdx.x; t < 4 * L; t += kThreads) {
-    cplx v = {0.0, 0.0};
-    if (t <= 2 * L) {
-      const cplx u = g[(int64_t)t * a.ncol];
-      const double w = a.weights[t] * a.phi_factor;
-      v = {u.x * w, u.y * w};
-    }
-    re[t] = v.x;
-    im[t] = v.y;
-  }
-  __syncthreads();
-  col_dft(re, im, 4 * L, a.conv[2], a.chirp_off[2], a.pool, -1);
-  // keep bins q in [-L, L): index q (q >= 0) and 4L+q (q < 0) -> 2L layout
-  {
-    cplx v[kPer];
-#pragma unroll
-    for (int c = 0; c < kPer; ++c) {
-      const int k = threadIdx.x + c * kThreads;
-      if (k < 2 * L) {
-        const int src = k < L ? k : k + 2 * L;
-        v[c] = {re[src], im[src]};
-        if (a.nyq_split && k == L) v[c] = {0.5 * (re[3 * L] + re[L]), 0.5 * (im[3 * L] + im[L])};
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int c = 0; c < kPer; ++c) {
-      const int k = threadIdx.x + c * kThreads;
-      if (k < 2 * L) {
-        re[k] = v[c].x;
-        im[k] = v[c].y;
-      }
-    }
-    __syncthreads();
-  }
-  col_dft(re, im, 2 * L, a.conv[1], a.chirp_off[1], a.pool, +1);
-  // 1/(2L) and fold rows L+1..2L-1 onto L-1..1
-  {
-    cplx v[kPer];
-#pragma unroll
-    for (int c = 0; c < kPer; ++c) {
-      const int t = threadIdx.x + c * kThreads;
-      if (t >= 1 && t <= L - 1) v[c] = {re[t] + msgn * re[2 * L - t], im[t] + msgn * im[2 * L - t]};
-    }
-    __syncthreads();
-#pragma unroll
-    for (int c = 0; c < kPer; ++c) {
-      const int t = threadIdx.x + c * kThreads;
-      if (t >= 1 && t <= L - 1) {
-        re[t] = v[c].x;
-        im[t] = v[c].y;
-      }
-    }
-    __syncthreads();
-    for (int t = threadIdx.x; t <= L; t += kThreads) {
-      re[t] /= (2 * L);
-      im[t] /= (2 * L);
-    }
-    __syncthreads();
-  }
-  cplx* dst = const_cast<cplx*>(a.in) + b * a.in_map_stride + col;
-  if (!a.mw) {
-    for (int t = threadIdx.x; t <= L; t += kThreads) dst[(int64_t)t * a.ncol] = {re[t], im[t]};
-    return;
-  }
-  // MW part: rows 0..L zero-extended to 2L, DFT_{2L}, bins p in [-(L-1), L-1]
-  for (int t = L + 1 + threadIdx.x; t < 2 * L; t += kThreads) {
-    re[t] = 0.0;
-    im[t] = 0.0;
-  }
-  __syncthreads();
-  col_dft(re, im, 2 * L, a.conv[1], a.chirp_off[1], a.pool, -1);
-  const int n1 = 2 * L - 1;
-  {
-    cplx v[kPer];
-#pragma unroll
-    for (int c = 0; c < kPer; ++c) {
-      const int k = threadIdx.x + c * kThreads;
-      if (k < n1) {
-        const int p = k < L ? k : k - n1;
-        const int src = p >= 0 ? p : 2 * L + p;
-        cplx x = {re[src], im[src]};
-        x = cmul(x, expi_pi((int64_t)p, n1));
-        v[c] = {x.x / n1, x.y / n1};
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int c = 0; c < kPer; ++c) {
-      const int k = threadIdx.x + c * kThreads;
-      if (k < n1) {
-        re[k] = v[c].x;
-        im[k] = v[c].y;
-      }
-    }
-    __syncthreads();
-  }
-  col_dft(re, im, n1, a.conv[0], a.chirp_off[0], a.pool, +1);
-  for (int t = threadIdx.x; t < L; t += kThreads) {
-    cplx v = {re[t], im[t]};
-    if (t <= L - 2) {
-      v.x += msgn * re[2 * L - 2 - t];
-      v.y += msgn * im[2 * L - 2 - t];
-    }
-    dst[(int64_t)t * a.ncol] = v;
-  }
-}
-
-hipError_t launch_resample_adjoint(const ResampleArgs& a, int batch, hipStream_t s) {
-  if (batch == 0 || a.nm == 0) return hipSuccess;
-  const size_t lds = 2 * sizeof(double) * (size_t)a.lds;
-  hipLaunchKernelGGL(resample_adjoint_kernel, dim3(a.nm, batch), dim3(kThreads), lds, s, a);
-  return hipGetLastError();
-}
-
-hipError_t allow_large_lds_resample_adjoint() {
-  return hipFuncSetAttribute((const void*)resample_adjoint_kernel,
-                             hipFuncAttributeMaxDynamicSharedMemorySize,
-                             (int)(2 * sizeof(double) * kMaxConvLen));
 }
 
 }  // namespace s2h

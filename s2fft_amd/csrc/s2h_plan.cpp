@@ -405,16 +405,30 @@ int make_set(s2h_plan* p, std::vector<RingJob> jobs, JobSet* out) {
   return S2H_OK;
 }
 
-// Latitudinal ring list over rows [r0, r1] of a theta grid.
-std::vector<LatRing> lat_rings(const std::vector<double>& th, int r0, int r1, bool paired) {
+// Cosine of row t of the MW / MWSS forward's own grid (MWSS at L), the nearest
+// FP64 value, the same for a row and its mirror image up to sign.
+double mwss_cos(int t, int L) {
+  if (2 * t > L) return -mwss_cos(L - t, L);
+  return 2 * t == L ? 0.0 : (double)std::cos(kPi * t / L);
+}
+
+// Latitudinal ring list over rows [r0, r1] of a theta grid.  With xs the rings
+// are at the colatitudes with exactly those cosines, else at theta itself.
+std::vector<LatRing> lat_rings(const std::vector<double>& th, int r0, int r1, bool paired,
+                               const std::vector<double>* xs = nullptr) {
   std::vector<LatRing> out;
   auto mk = [&](int ta, int tb) {
     LatRing r{};
     r.ta = ta;
     r.tb = tb;
-    r.x = std::cos(th[ta]);
-    r.c2 = std::cos(th[ta] / 2.0);
-    r.s2 = std::sin(th[ta] / 2.0);
+    r.x = xs ? (*xs)[ta] : std::cos(th[ta]);
+    const long double half = (long double)th[ta] / 2;
+    const long double c = xs ? std::sqrt((1.0L + r.x) / 2) : std::cos(half);
+    const long double s = xs ? std::sqrt((1.0L - r.x) / 2) : std::sin(half);
+    r.c2 = xs ? (double)c : std::cos(th[ta] / 2.0);
+    r.s2 = xs ? (double)s : std::sin(th[ta] / 2.0);
+    r.c2r = r.c2 != 0.0 ? (double)((c - r.c2) / r.c2) : 0.0;
+    r.s2r = r.s2 != 0.0 ? (double)((s - r.s2) / r.s2) : 0.0;
     return r;
   };
   if (!paired) {
@@ -557,15 +571,18 @@ static int plan_build(s2h_plan* p) {
     fwd_j = inv_j;
     for (size_t t = 0; t < fwd_j.size(); ++t) fwd_j[t].weight = wf[t];
   } else {
-    // resampled to MWSS at 2L: rows 0..2L, poles at 0 and 2L
+    // the theta operators' output: MWSS at L, rows 0..L, poles at 0 and L; the
+    // operators absorb the rounding of the rows' cosines (delta)
     p->fwd_kind = d.sampling == S2H_MW ? 1 : 2;
-    p->fwd_rows = 2 * L + 1;
-    std::vector<double> thf;
-    for (int t = 0; t <= 2 * L; ++t) thf.push_back(2.0 * t * M_PI / (4.0 * L));
-    fwd_r = lat_rings(thf, 1, 2 * L - 1, pair_ok);
+    p->fwd_rows = L + 1;
+    std::vector<double> xs, delta(L + 1, 0.0);
+    for (int t = 0; t <= L; ++t) xs.push_back(mwss_cos(t, L));
+    for (int t = 1; t < L; ++t)
+      delta[t] = (double)((std::cos(kPi * t / L) - (long double)xs[t]) / std::sin(kPi * t / L));
+    fwd_r = lat_rings(thetas(S2H_MWSS, L, 0), 1, L - 1, pair_ok, &xs);
     p->fwd_paired = pair_ok;
     p->fwd_row_north = 0;
-    p->fwd_row_south = 2 * L;
+    p->fwd_row_south = L;
     wf = forward_weights(d.sampling, L, nside);
     p->fwd_in_rows = p->inv_rows;
     fwd_j = inv_j;  // phi-DFT of the input rows, weight 1
@@ -578,8 +595,12 @@ static int plan_build(s2h_plan* p) {
     if (need > kMaxConvLen) return S2H_ERR_UNSUPPORTED;
     p->rs_info[3] = need;
     if (allow_large_lds_resample() != hipSuccess) return S2H_ERR_HIP;
-    if (allow_large_lds_resample_adjoint() != hipSuccess) return S2H_ERR_HIP;
+    if (d.norm != S2H_NORM_NONE) {
+      const int st = theta_mix_get(p->device, d.sampling == S2H_MW, L, wf, delta, &p->mix);
+      if (st) return st;
+    }
   }
+  p->pc_rows = p->fwd_kind == 0 ? p->fwd_rows : 2 * L + 1;
 
   // ---------------- recursion tables
   std::vector<MStart> msf, msi;
@@ -663,9 +684,6 @@ static int plan_build(s2h_plan* p) {
   }
   if ((st = upload(p, nf, &p->fwd_norm))) return st;
   if ((st = upload(p, ni, &p->inv_norm))) return st;
-  if (!wf.empty() && p->fwd_kind != 0) {
-    if ((st = upload(p, wf, &p->fwd_weights))) return st;
-  }
   {
     std::vector<double> thf_rows;
     if (p->fwd_kind == 0) {

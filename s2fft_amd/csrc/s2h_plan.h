@@ -1,6 +1,7 @@
 // Host-side plan: constant tables for one (sampling, L, nside, spin, ...) set.
 #pragma once
 
+#include <memory>
 #include <vector>
 
 #include "s2h_kernels.h"
@@ -14,9 +15,11 @@ struct s2h_plan {
   double sign = 1;   // global sign folded into the recursion
 
   // forward
-  int fwd_kind = 0;  // 0 direct ring FFT, 1 MW resample, 2 MWSS resample
+  int fwd_kind = 0;  // 0 direct ring FFT, 1 MW, 2 MWSS (theta operators, s2h_theta_mix.hip)
   int fwd_rows = 0;  // rows of the internal forward ftm
-  int fwd_in_rows = 0;  // rows of the phi-spectrum before resampling (kinds 1, 2)
+  int fwd_in_rows = 0;  // rows of the phi-spectrum before the theta step (kinds 1, 2)
+  std::shared_ptr<s2h::ThetaMix> mix;  // kinds 1, 2
+  int pc_rows = 0;   // rows a stored forward kernel contracts: 2L + 1 (kinds 1, 2) or fwd_rows
   s2h::JobSet fwd_set;
   s2h::LatRing* fwd_rings = nullptr;
   int n_fwd_rings = 0;
@@ -26,8 +29,7 @@ struct s2h_plan {
   s2h::Coef* fwd_coef = nullptr;
   s2h::Coef* fwd_ucoef = nullptr;  // unit-c form (make_unit_coefs)
   double* fwd_norm = nullptr;
-  double* fwd_weights = nullptr;  // MWSS-at-2L weights (kinds 1, 2)
-  int rs_info[8] = {0};           // resampling DFT lengths / conv lengths
+  int rs_info[8] = {0};           // stored-kernel resampling: DFT lengths / conv lengths
   int64_t rs_chirp[4] = {0};
 
   // inverse
@@ -61,7 +63,7 @@ struct s2h_plan {
   double spec_belt_wn = 0.0;
   int spec_belt_row_lo = 0, spec_belt_row_hi = 0;
 
-  // per-row tables of the forward grid (fwd_rows) and the inverse grid
+  // per-row tables of the forward grid (pc_rows) and the inverse grid
   // (inv_rows), for the precompute kernels: colatitudes, the forward
   // quadrature weight of each forward row, the HEALPix first-pixel azimuth
   double* fwd_theta = nullptr;
@@ -94,6 +96,12 @@ struct HpTables {
 // S2H_ERR_INVALID for tables that were never prepared.
 int healpix_tables_prepare(int nside, int L);
 int healpix_tables(int nside, int L, HpTables* out);
+// Theta operators of the MW / MWSS forward (s2h_theta_mix.hip): built once per
+// (device, sampling, L) and shared by the plans alive; weights: the 2L + 1 rows
+// of MWSS at 2L; delta: the L + 1 shifts of the projection's colatitudes from
+// pi r / L.  Allocates, synchronises.
+int theta_mix_get(int device, bool mw, int L, const std::vector<double>& weights,
+                  const std::vector<double>& delta, std::shared_ptr<ThetaMix>* out);
 }  // namespace s2h
 
 // Wigner (SO(3)) transform plan: one spin plan per n (spin -n, Wigner
