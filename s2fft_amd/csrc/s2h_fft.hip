@@ -8,16 +8,16 @@ namespace s2h {
 
 constexpr int kFftMax = kMaxConvLen;
 
-// FFT_M(b)/M for Bluestein, b_j = exp(+i pi j^2 / n) for |j| < n, wrapped.
-__global__ void __launch_bounds__(kThreads) chirp_setup_kernel(const int* lengths,
-                                                               const int* conv_lens,
-                                                               const int64_t* offs,
+// The chirp pool's tables of one length per workgroup (ChirpEntry).
+__global__ void __launch_bounds__(kThreads) chirp_setup_kernel(const ChirpEntry* entries,
                                                                cplx* pool) {
   extern __shared__ double smem[];
-  const int n = lengths[blockIdx.x];
-  const int M = conv_lens[blockIdx.x];
+  const ChirpEntry en = entries[blockIdx.x];
+  const int n = en.n, M = en.M;
   double* re = smem;
   double* im = smem + M;
+  if (blockIdx.x == 0)
+    for (int j = threadIdx.x; j < kBlueTwiddles; j += kThreads) pool[j] = expi_pi(-j, kMaxConvLen / 2);
   for (int j = threadIdx.x; j < M; j += kThreads) {
     cplx v = {0.0, 0.0};
     if (j < n)
@@ -29,9 +29,15 @@ __global__ void __launch_bounds__(kThreads) chirp_setup_kernel(const int* length
   }
   __syncthreads();
   fft_mixed<kFftMax>(re, im, M, -1);
-  cplx* dst = pool + offs[blockIdx.x];
+  cplx* dst = pool + en.off;
   const double s = 1.0 / M;
-  for (int j = threadIdx.x; j < M; j += kThreads) dst[j] = {re[j] * s, im[j] * s};
+  for (int j = threadIdx.x; j < M; j += kThreads)
+    dst[en.ring ? blue_place(j, M) : j] = {re[j] * s, im[j] * s};
+  if (!en.ring) return;
+  for (int k = threadIdx.x; k < n; k += kThreads) {
+    dst[M + k] = expi_pi(-(int64_t)k * k, n);
+    dst[M + n + k] = expi_pi(-k, n);
+  }
 }
 
 // Direct DFT over gamma (G = 2N-1 <= 15 points) for every (beta, alpha)
@@ -129,12 +135,11 @@ __global__ void __launch_bounds__(kThreads) wigner_fill_adjoint_kernel(cplx* g, 
 }
 
 // ------------------------------------------------------------ launchers
-hipError_t launch_chirp_setup(const int* lengths, const int* conv_lens, const int64_t* offs,
-                              cplx* pool, int count, int max_conv, hipStream_t s) {
+hipError_t launch_chirp_setup(const ChirpEntry* entries, cplx* pool, int count, int max_conv,
+                              hipStream_t s) {
   if (count == 0) return hipSuccess;
   const size_t lds = 2 * sizeof(double) * (size_t)max_conv;
-  hipLaunchKernelGGL(chirp_setup_kernel, dim3(count), dim3(kThreads), lds, s, lengths, conv_lens,
-                     offs, pool);
+  hipLaunchKernelGGL(chirp_setup_kernel, dim3(count), dim3(kThreads), lds, s, entries, pool);
   return hipGetLastError();
 }
 
@@ -156,6 +161,7 @@ hipError_t launch_wigner_fill(cplx* flmn, int L, int N, hipStream_t s) {
 
 hipError_t allow_large_lds() {
   hipError_t e = allow_large_lds_rings();
+  if (e == hipSuccess) e = allow_large_lds_alias();
   if (e != hipSuccess) return e;
   const int bytes = 2 * sizeof(double) * kFftMax;
   return hipFuncSetAttribute((const void*)chirp_setup_kernel,

@@ -9,7 +9,7 @@
 namespace s2h {
 
 constexpr int kThreads = 256;        // workgroup size of every kernel here
-constexpr int kMaxRingLen = 4096;    // longest ring FFT held in LDS (Stockham)
+constexpr int kMaxRingLen = 4096;    // longest ring FFT
 constexpr int kMaxConvLen = 8192;    // longest Bluestein convolution held in LDS
 constexpr int kMaxL = 4096;           // ring phase tables cover |m| < kMaxL
 constexpr int kMlpHidden = 64;        // learned preconditioner: hidden width
@@ -23,26 +23,22 @@ struct RingJob {
   int32_t row;          // row of the ftm array this ring maps to
   double phi0_over_pi;  // azimuth of the first pixel / pi
   double weight;        // quadrature weight applied by the forward FFT
-  int32_t conv_len;     // 0: mixed-radix; else Bluestein length M (power of 2)
+  int32_t conv_len;     // 0: the power-of-two length; else Bluestein length M
   int32_t pad;
-  int64_t chirp_off;    // offset (complex elements) of FFT(chirp)/M in the chirp pool
+  int64_t chirp_off;    // offset (complex elements) of the length's tables in the chirp pool
 };
 
-// Ring jobs of one transform on the device, in three consecutive classes:
-// n_pow2 power-of-two lengths, n_smooth other lengths with prime factors
-// <= 13, n_blue Bluestein rings; each class sorted by decreasing length.
-// Bluestein rings whose convolution is longer than this launch separately:
-// the shorter ones then fit two workgroups' LDS per CU.
-constexpr int kBlueSplit = 4096;
+// Ring jobs of one transform on the device: n_pow2 rings of one power-of-two
+// length, then n_blue Bluestein rings (by decreasing convolution length).
+constexpr int kBlueLogMin = 6;   // convolutions of 64 ...
+constexpr int kBlueClasses = 8;  // ... to 8192 = kMaxConvLen points
 
 struct JobSet {
   RingJob* jobs = nullptr;
-  int n_pow2 = 0, n_smooth = 0, n_blue = 0;
-  int n_blue_long = 0;  // Bluestein rings with convolution > kBlueSplit (listed first)
-  int max_pow2 = 0;     // longest power-of-two ring
-  int max_smooth = 0;   // longest other mixed-radix ring
-  int max_conv = 0;     // longest Bluestein convolution
-  int max_conv_short = 0;  // longest Bluestein convolution <= kBlueSplit
+  int n_pow2 = 0, n_blue = 0;
+  int blue[kBlueClasses] = {};  // Bluestein rings by convolution length 64 << class
+  int log_pow2 = 0;     // log2 of the power-of-two length
+  int min_blue = 0;     // shortest Bluestein ring
   int max_nphi = 0;     // longest ring
 };
 

@@ -182,6 +182,7 @@ hipError_t launch_ring_fft_forward(const RingFwdArgs& a, const JobSet& js, int b
 hipError_t launch_ring_fft_inverse(const RingInvArgs& a, const JobSet& js, int batch,
                                    hipStream_t s);
 hipError_t allow_large_lds_rings();
+hipError_t allow_large_lds_alias();
 hipError_t launch_ring_alias(const RingAliasArgs& a, const JobSet& js, int batch, hipStream_t s);
 // pq[b] = sum_m c_m Re(conj(Y) A(Y)) over every ring of map b (part: batch x
 // ring_dot_jobs(js) doubles); alpha[b] = num[b] / pq[b] when alpha is given
@@ -205,8 +206,30 @@ hipError_t launch_ring_alias_sumsq(const RingAliasArgs& a, const JobSet& js, int
                                    double* part, double* sumsq, hipStream_t s);
 hipError_t launch_ring_dot(const RingAliasArgs& a, const JobSet& js, int batch, double* part,
                            const double* num, double* pq, double* alpha, hipStream_t s);
-hipError_t launch_chirp_setup(const int* lengths, const int* conv_lens, const int64_t* offs,
-                              cplx* pool, int count, int max_conv, hipStream_t s);
+// Chirp pool.  It starts with kBlueTwiddles twiddles e^{-2 pi i j / 8192}; then
+// per length n with convolution M either (ring 0: the stored-kernel resampling)
+// FFT_M(b) / M, b_j = e^{i pi j^2 / n}, or (ring 1: the Bluestein ring kernels)
+// FFT_M(b) / M at the places blue_place(k, M), the n chirps e^{-i pi k^2 / n} and
+// the n phases e^{-i pi k / n}.
+constexpr int kBlueTwiddles = 512;
+struct ChirpEntry {
+  int n, M, ring, pad;
+  int64_t off;
+};
+// Register order of the ring kernels' spectra: thread t of T = M / 16 holds
+// point i at i T + t (s2h_ring_fft.hip).
+__host__ __device__ inline int blue_place(int k, int M) {
+  const int T = M / 16;
+  const int k1 = k & 15;
+  if (T < 16) return ((k1 / T) * T + (k >> 4)) * T + k1 % T;
+  const int S = T / 16, k2 = (k >> 4) & 15, k3 = k >> 8;
+  const int g = k1 * 16 + k2;
+  if (S == 1) return k2 * T + k1;
+  if (S <= 16) return ((g / T) * S + k3) * T + g % T;
+  return (k3 & 15) * T + 2 * g + (k3 >> 4);
+}
+hipError_t launch_chirp_setup(const ChirpEntry* entries, cplx* pool, int count, int max_conv,
+                              hipStream_t s);
 hipError_t launch_gamma_dft(int N, int64_t npix, int mode, double scale, const void* in,
                             void* out, hipStream_t s);
 hipError_t launch_wigner_fill(cplx* flmn, int L, int N, hipStream_t s);

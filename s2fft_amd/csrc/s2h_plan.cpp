@@ -291,23 +291,28 @@ int next_pow2(int v) {
 }
 
 struct ChirpBuilder {
-  std::map<int, std::pair<int, int64_t>> table;  // n -> (M, offset)
-  int64_t total = 0;
+  std::map<std::tuple<int, int, int>, int64_t> table;  // (n, M, ring) -> offset
+  int64_t total = kBlueTwiddles;
   int max_conv = 0;
-  // Returns conv length (0 = mixed radix) and sets the chirp offset.
+  // Returns the convolution length of an n-point column DFT (0 = mixed radix)
+  // and sets the offset of its tables.
   int add(int n, int64_t* off) {
     *off = 0;
-    if (largest_prime_factor(n) <= 13) return 0;
-    auto it = table.find(n);
-    if (it != table.end()) {
-      *off = it->second.second;
-      return it->second.first;
+    return largest_prime_factor(n) <= 13 ? 0 : insert(n, next_pow2(2 * n - 1), 0, off);
+  }
+  // The same for an n-point ring, with at least min_m points.
+  int add_ring(int n, int64_t* off, int min_m) {
+    return insert(n, next_pow2(std::max(std::max(2 * n - 1, 1 << kBlueLogMin), min_m)), 1, off);
+  }
+  int insert(int n, int M, int ring, int64_t* off) {
+    const auto key = std::make_tuple(n, M, ring);
+    auto it = table.find(key);
+    if (it == table.end()) {
+      it = table.emplace(key, total).first;
+      total += M + (ring ? 2 * n : 0);
+      max_conv = std::max(max_conv, M);
     }
-    const int M = next_pow2(2 * n - 1);
-    table[n] = {M, total};
-    *off = total;
-    total += M;
-    max_conv = std::max(max_conv, M);
+    *off = it->second;
     return M;
   }
   // Allocates the chirp pool and fills it on the device (synchronously: plan
@@ -315,34 +320,26 @@ struct ChirpBuilder {
   // plan) or, with allocs null, owned by the caller; on failure nothing leaks.
   int build(cplx** pool, std::vector<void*>* allocs) {
     *pool = nullptr;
-    if (table.empty()) return S2H_OK;
-    std::vector<int> ns, Ms;
-    std::vector<int64_t> offs;
-    for (auto& kv : table) {
-      ns.push_back(kv.first);
-      Ms.push_back(kv.second.first);
-      offs.push_back(kv.second.second);
-    }
+    std::vector<ChirpEntry> en;
+    for (auto& kv : table)
+      en.push_back(ChirpEntry{std::get<0>(kv.first), std::get<1>(kv.first), std::get<2>(kv.first), 0,
+                              kv.second});
     // every temporary is freed on every path
     struct Tmp {
-      void* p[4] = {nullptr, nullptr, nullptr, nullptr};
+      void* p[2] = {nullptr, nullptr};
       ~Tmp() {
         for (void* q : p)
           if (q) (void)hipFree(q);
       }
     } t;
-    const size_t cnt = ns.size();
+    if (en.empty()) en.push_back(ChirpEntry{});  // twiddles only
+    const size_t bytes = sizeof(ChirpEntry) * en.size();
     if (hipMalloc(&t.p[0], sizeof(cplx) * total) != hipSuccess) return S2H_ERR_NOMEM;
-    if (hipMalloc(&t.p[1], sizeof(int) * cnt) != hipSuccess) return S2H_ERR_NOMEM;
-    if (hipMalloc(&t.p[2], sizeof(int) * cnt) != hipSuccess) return S2H_ERR_NOMEM;
-    if (hipMalloc(&t.p[3], sizeof(int64_t) * cnt) != hipSuccess) return S2H_ERR_NOMEM;
-    if (hipMemcpy(t.p[1], ns.data(), sizeof(int) * cnt, hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(t.p[2], Ms.data(), sizeof(int) * cnt, hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(t.p[3], offs.data(), sizeof(int64_t) * cnt, hipMemcpyHostToDevice) != hipSuccess)
+    if (hipMalloc(&t.p[1], bytes) != hipSuccess) return S2H_ERR_NOMEM;
+    if (hipMemcpy(t.p[1], en.data(), bytes, hipMemcpyHostToDevice) != hipSuccess)
       return S2H_ERR_HIP;
-    hipError_t e = launch_chirp_setup(static_cast<int*>(t.p[1]), static_cast<int*>(t.p[2]),
-                                      static_cast<int64_t*>(t.p[3]), static_cast<cplx*>(t.p[0]),
-                                      (int)cnt, max_conv, 0);
+    hipError_t e = launch_chirp_setup(static_cast<ChirpEntry*>(t.p[1]), static_cast<cplx*>(t.p[0]),
+                                      (int)en.size(), max_conv, 0);
     if (e == hipSuccess) e = hipDeviceSynchronize();
     if (e != hipSuccess) return S2H_ERR_HIP;
     *pool = static_cast<cplx*>(t.p[0]);
@@ -352,51 +349,49 @@ struct ChirpBuilder {
   }
 };
 
-RingJob make_job(int64_t off, int nphi, int row, double phi0, double w, ChirpBuilder& cb) {
+// A grid's one power-of-two length pow2 (0: none) runs as such from 64 points
+// on, every other ring by Bluestein.
+RingJob make_job(int64_t off, int nphi, int row, double phi0, double w, ChirpBuilder& cb, int pow2,
+                 int min_m = 0) {
   RingJob j{};
   j.pix_offset = off;
   j.nphi = nphi;
   j.row = row;
   j.phi0_over_pi = phi0;
   j.weight = w;
-  j.conv_len = cb.add(nphi, &j.chirp_off);
+  const bool direct = nphi == pow2 && (nphi & (nphi - 1)) == 0 && nphi >= 64;
+  if (!direct) j.conv_len = cb.add_ring(nphi, &j.chirp_off, min_m);
   return j;
 }
 
-// Orders the jobs (powers of two, other mixed-radix lengths, Bluestein;
-// longest first within a class so that the heavy workgroups start early) and
-// uploads them.
-int ring_class(const RingJob& j) {
-  if (j.conv_len) return 2;
-  return (j.nphi & (j.nphi - 1)) == 0 ? 0 : 1;
+// Convolution lengths of a ragged grid's Bluestein rings start at the number of
+// columns: M / 16 threads per ring then write (fold) a row in at most 16 columns
+// each, and the short rings share one launch.
+int ragged_min_conv(int ncol) { return std::min(next_pow2(ncol), kMaxConvLen); }
+
+// Orders the jobs (the power of two, then Bluestein by decreasing convolution
+// length, longest rings first) and uploads them.
+int blue_class(int M) {
+  int c = 0;
+  while ((1 << (kBlueLogMin + c)) < M) ++c;
+  return c;
 }
 
 int make_set(s2h_plan* p, std::vector<RingJob> jobs, JobSet* out) {
   std::stable_sort(jobs.begin(), jobs.end(), [](const RingJob& x, const RingJob& y) {
-    const int cx = ring_class(x), cy = ring_class(y);
-    if (cx != cy) return cx < cy;
-    const int kx = cx == 2 ? x.conv_len : x.nphi, ky = cy == 2 ? y.conv_len : y.nphi;
-    return kx > ky;
+    if ((x.conv_len == 0) != (y.conv_len == 0)) return x.conv_len == 0;
+    return x.conv_len != y.conv_len ? x.conv_len > y.conv_len : x.nphi > y.nphi;
   });
   JobSet js;
   for (auto& j : jobs) {
     js.max_nphi = std::max(js.max_nphi, j.nphi);
-    switch (ring_class(j)) {
-      case 0:
-        ++js.n_pow2;
-        js.max_pow2 = std::max(js.max_pow2, j.nphi);
-        break;
-      case 1:
-        ++js.n_smooth;
-        js.max_smooth = std::max(js.max_smooth, j.nphi);
-        break;
-      default:
-        ++js.n_blue;
-        js.max_conv = std::max(js.max_conv, j.conv_len);
-        if (j.conv_len > kBlueSplit)
-          ++js.n_blue_long;
-        else
-          js.max_conv_short = std::max(js.max_conv_short, j.conv_len);
+    if (j.conv_len == 0) {
+      ++js.n_pow2;
+      while ((1 << js.log_pow2) < j.nphi) ++js.log_pow2;
+    } else {
+      ++js.n_blue;
+      ++js.blue[blue_class(j.conv_len)];
+      js.min_blue = js.n_blue == 1 ? j.nphi : std::min(js.min_blue, j.nphi);
     }
   }
   const int st = upload<RingJob>(p, jobs, &js.jobs);
@@ -461,7 +456,8 @@ int healpix_tables_prepare(int nside, int L) {
   int64_t off = 0;
   for (int t = 0; t < 4 * nside - 1; ++t) {
     const int n = healpix_nphi(t, nside);
-    jobs.push_back(make_job(off, n, t, healpix_phi0_over_pi(t, nside), 1.0, cb));
+    jobs.push_back(make_job(off, n, t, healpix_phi0_over_pi(t, nside), 1.0, cb, 4 * nside,
+                            ragged_min_conv(2 * L)));
     off += n;
   }
   HpTables tb;
@@ -518,7 +514,8 @@ static int plan_build(s2h_plan* p) {
       int64_t off = 0;
       for (int t = 0; t < p->inv_rows; ++t) {
         const int np = healpix_nphi(t, nside);
-        inv_j.push_back(make_job(off, np, t, healpix_phi0_over_pi(t, nside), 1.0, cb));
+        inv_j.push_back(make_job(off, np, t, healpix_phi0_over_pi(t, nside), 1.0, cb, 4 * nside,
+                                 ragged_min_conv(p->Mc)));
         off += np;
       }
       p->npix = off;
@@ -529,7 +526,7 @@ static int plan_build(s2h_plan* p) {
       p->inv_rows = (int)thi.size();
       inv_r = lat_rings(thi, 0, p->inv_rows - 1, pair_ok);
       const int np = 2 * L - 1;
-      for (int t = 0; t < p->inv_rows; ++t) inv_j.push_back(make_job((int64_t)t * np, np, t, 0.0, 1.0, cb));
+      for (int t = 0; t < p->inv_rows; ++t) inv_j.push_back(make_job((int64_t)t * np, np, t, 0.0, 1.0, cb, np));
       p->npix = (int64_t)p->inv_rows * np;
       break;
     }
@@ -538,7 +535,7 @@ static int plan_build(s2h_plan* p) {
       inv_r = lat_rings(thi, 0, L - 2, false);  // theta_{L-1} = pi is the pole row
       p->inv_row_south = L - 1;
       const int np = 2 * L - 1;
-      for (int t = 0; t < L; ++t) inv_j.push_back(make_job((int64_t)t * np, np, t, 0.0, 1.0, cb));
+      for (int t = 0; t < L; ++t) inv_j.push_back(make_job((int64_t)t * np, np, t, 0.0, 1.0, cb, np));
       p->npix = (int64_t)L * np;
       break;
     }
@@ -548,7 +545,7 @@ static int plan_build(s2h_plan* p) {
       p->inv_row_north = 0;
       p->inv_row_south = L;
       const int np = 2 * L;
-      for (int t = 0; t <= L; ++t) inv_j.push_back(make_job((int64_t)t * np, np, t, 0.0, 1.0, cb));
+      for (int t = 0; t <= L; ++t) inv_j.push_back(make_job((int64_t)t * np, np, t, 0.0, 1.0, cb, np));
       p->npix = (int64_t)(L + 1) * np;
       break;
     }

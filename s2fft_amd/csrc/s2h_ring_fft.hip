@@ -1,5 +1,4 @@
-// Ragged ring FFT kernels: one workgroup per (ring, map or map pair), the
-// whole ring in LDS.
+// Ragged ring FFTs, every ring in the registers of its threads.
 //
 // Forward  (s2fft/utils/healpix_ffts.py:187-226 + spherical.py:533-546):
 //   out[row, col] = w_t * exp(-i m phi0_t) * F_t[m mod nphi_t],  m = m_first + col
@@ -7,1405 +6,1120 @@
 //   quadrature weight and the ring phase are fused into the store.
 // Inverse  (healpix_ffts.py:335-371 + spherical.py:183-200):
 //   F_t[q] = sum_{m = q mod nphi} exp(+i m phi0_t) c(m), f_t[p] = sum_q F_t[q] e^{2 pi i q p/nphi}
-//   the folding and the phase are fused into the LDS load.
+//   the folding and the phase are fused into the load.
 //
-// Rings fall in three classes launched separately so that each gets the LDS
-// and registers it needs: powers of two (radix-8 Stockham passes and one
-// radix 4 or 2), other lengths whose prime factors are all <= 13 (radices
-// 3, 5, 7, 11, 13 as well) and the rest (Bluestein's chirp-z over a
-// power-of-two convolution).  Twiddles, chirps and ring
-// phases come from two-level tables in LDS (e^{i a k} = hi[k / 64] lo[k % 64])
-// built once per workgroup, so no transcendental is evaluated per point.
+// Two kinds of rings: the grid's one power-of-two length as such, every other
+// length by Bluestein's chirp-z (Bluestein 1970).  Lengths with small prime
+// factors too: with a mixed-radix LDS kernel for those the grid of nside 192,
+// five maps, took 109 us and 62 without it.
 // Two real maps share one complex transform (z = x + i y, split by the
 // conjugate symmetry of the spectra), halving the transforms for real data.
+//
+// T = N / 16 threads per ring hold 16 points each, p = t + T e in the first pass
+// (coalesced loads straight into it), and run radix-16 passes with one LDS
+// exchange between passes: N = 4096: 16 x 16 x 16, 2048, 1024, 512: 16 x 16 x
+// 8, 4, 2, 256: 16 x 16, 128, 64: 16 x 8, 16 x 4.  An exchange writes the
+// positions its thread read last, so it needs one barrier.
+//
+// Powers of two: the last pass takes the sub-transforms so that thread t ends
+// up with X[t + T e]: coalesced stores, no exchange into natural order.
+//
+// Bluestein: X[k] = c_k sum_p (x_p c_p) conj(c_{k-p}), c_k = e^{-i pi k^2/n}, the
+// convolution by two FFTs of M >= 2n - 1 points (M = 8192: 16 x 16 x 16 x 2, the
+// radix 2 between neighbouring lanes).  Decimation in frequency forward and in
+// time back, so nothing is put into natural order in between: FFT(chirp) is
+// stored in the order of the registers.  Four barriers per convolution; the
+// zero upper half of the input and the unwanted upper half of the output are
+// left out of the first and last pass.
+// Chirps, FFT(chirp) and twiddles come from the plan's table.
+//
+// What bounds it: the large grids their HBM traffic (64 maps of L = 512 MW, 1.07
+// GB: 0.38 ms forward and 0.40 inverse, 2.8 TB/s; the former LDS kernels with
+// one barrier pair per radix-8 pass took 2.14 and 2.29), with two waves per SIMD
+// (the 16 points and their twiddles); single maps the latency of the passes (L =
+// 128, one map: 10 us, was 18; nside 512: 45, was 119; inverse 57, was 147).
+//
+// HEALPix ring phases are e^{-i m phi0} with phi0 = 0 or pi / n, so the phase of
+// column m = k + j n is (-1)^j e^{-i pi k / n}: one product per residue and a
+// sign per column, in both directions.
+#include <algorithm>
+
 #include "s2h_fft_lds.h"
 #include "s2h_kernels.h"
+#include "s2h_lat_common.h"
 
 namespace s2h {
 
 namespace {
 
-constexpr int kTabLo = 64;
+constexpr double kC8 = 0.92387953251128675613, kS8 = 0.38268343236508977173;  // cos, sin pi/8
+constexpr double kR2 = 0.70710678118654752440;
 
-// LDS word index of data point p: one pad word per 32 breaks the power-of-two
-// strides of the early Stockham passes across the LDS banks (their writes go
-// to stride R, then to runs of R at stride R^2).
-__device__ __forceinline__ int lx(int p) { return p + (p >> 5); }
-__host__ __device__ constexpr int lx_len(int n) { return n + (n >> 5) + 1; }
+__device__ __forceinline__ cplx cconj(cplx a) { return {a.x, -a.y}; }
+// a * w (INV: a * conj w)
+template <bool INV>
+__device__ __forceinline__ cplx tmul(cplx a, cplx w) {
+  return INV ? cplx{fma(a.x, w.x, a.y * w.y), fma(a.y, w.x, -(a.x * w.y))}
+             : cplx{fma(a.x, w.x, -(a.y * w.y)), fma(a.x, w.y, a.y * w.x)};
+}
+// -i a (INV: i a)
+template <bool INV>
+__device__ __forceinline__ cplx mul_mi(cplx a) {
+  return INV ? cplx{-a.y, a.x} : cplx{a.y, -a.x};
+}
 
-// e^{i pi num/den}-based two-level table: value(k) = hi[k >> 6] * lo[k & 63],
-// value(k) = e^{i pi s k / d} for 0 <= k < count.
-struct Tab2 {
-  const cplx* hi;
-  const cplx* lo;
-  __device__ cplx at(int k) const { return cmul(hi[k >> 6], lo[k & 63]); }
+template <bool INV>
+__device__ __forceinline__ void dft2(cplx& a, cplx& b) {
+  const cplx t = a;
+  a = cadd(t, b);
+  b = csub(t, b);
+}
+template <bool INV>
+__device__ __forceinline__ void dft4(cplx& a, cplx& b, cplx& c, cplx& d) {
+  const cplx s0 = cadd(a, c), d0 = csub(a, c), s1 = cadd(b, d), d1 = mul_mi<INV>(csub(b, d));
+  a = cadd(s0, s1);
+  b = cadd(d0, d1);
+  c = csub(s0, s1);
+  d = csub(d0, d1);
+}
+// w16^k a for the twiddles inside radix 8 and 16
+template <bool INV, int K>
+__device__ __forceinline__ cplx w16(cplx a) {
+  if constexpr (K == 0) return a;
+  if constexpr (K == 1) return tmul<INV>(a, cplx{kC8, -kS8});
+  if constexpr (K == 2) {
+    const cplx t = mul_mi<INV>(a);
+    return {kR2 * (a.x + t.x), kR2 * (a.y + t.y)};
+  }
+  if constexpr (K == 3) return tmul<INV>(a, cplx{kS8, -kC8});
+  if constexpr (K == 4) return mul_mi<INV>(a);
+  if constexpr (K == 6) {
+    const cplx t = mul_mi<INV>(a);
+    return {kR2 * (t.x - a.x), kR2 * (t.y - a.y)};
+  }
+  if constexpr (K == 9) return tmul<INV>(a, cplx{-kC8, kS8});
+  return a;
+}
+template <bool INV>
+__device__ __forceinline__ void dft8(cplx* v) {
+  dft4<INV>(v[0], v[2], v[4], v[6]);
+  dft4<INV>(v[1], v[3], v[5], v[7]);
+  const cplx o1 = w16<INV, 2>(v[3]), o2 = mul_mi<INV>(v[5]), o3 = w16<INV, 6>(v[7]);
+  const cplx e0 = v[0], e1 = v[2], e2 = v[4], e3 = v[6], o0 = v[1];
+  v[0] = cadd(e0, o0);
+  v[4] = csub(e0, o0);
+  v[1] = cadd(e1, o1);
+  v[5] = csub(e1, o1);
+  v[2] = cadd(e2, o2);
+  v[6] = csub(e2, o2);
+  v[3] = cadd(e3, o3);
+  v[7] = csub(e3, o3);
+}
+// 16 points, natural order in and out.  HALF_IN: v[8..15] are zero (not read);
+// HALF_OUT: only v[0..7] are wanted.
+template <bool INV, bool HALF_IN, bool HALF_OUT>
+__device__ __forceinline__ void dft16(cplx* v) {
+  // columns j: points j, j + 4, j + 8, j + 12 -> y[j][k]
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    if constexpr (HALF_IN) {
+      const cplx a = v[j], b = v[j + 4], t = mul_mi<INV>(b);
+      v[j] = cadd(a, b);
+      v[j + 4] = cadd(a, t);
+      v[j + 8] = csub(a, b);
+      v[j + 12] = csub(a, t);
+    } else {
+      dft4<INV>(v[j], v[j + 4], v[j + 8], v[j + 12]);
+    }
+  }
+  v[5] = w16<INV, 1>(v[5]);
+  v[6] = w16<INV, 2>(v[6]);
+  v[7] = w16<INV, 3>(v[7]);
+  v[9] = w16<INV, 2>(v[9]);
+  v[10] = w16<INV, 4>(v[10]);
+  v[11] = w16<INV, 6>(v[11]);
+  v[13] = w16<INV, 3>(v[13]);
+  v[14] = w16<INV, 6>(v[14]);
+  v[15] = w16<INV, 9>(v[15]);
+  // rows k: X[k + 4 m]
+  cplx x[16];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    cplx a = v[4 * k], b = v[4 * k + 1], c = v[4 * k + 2], d = v[4 * k + 3];
+    dft4<INV>(a, b, c, d);
+    x[k] = a;
+    x[k + 4] = b;
+    x[k + 8] = c;
+    x[k + 12] = d;
+  }
+#pragma unroll
+  for (int k = 0; k < (HALF_OUT ? 8 : 16); ++k) v[k] = x[k];
+}
+
+// v[k] *= w^k (INV: conj w^k), the powers by products of depth 4
+template <bool INV>
+__device__ __forceinline__ void twiddle16(cplx* v, cplx w) {
+  const cplx w2 = cmul(w, w), w4 = cmul(w2, w2), w8 = cmul(w4, w4);
+  v[1] = tmul<INV>(v[1], w);
+  v[2] = tmul<INV>(v[2], w2);
+  v[4] = tmul<INV>(v[4], w4);
+  v[8] = tmul<INV>(v[8], w8);
+  const cplx w3 = cmul(w2, w), w5 = cmul(w4, w), w6 = cmul(w4, w2), w9 = cmul(w8, w);
+  v[3] = tmul<INV>(v[3], w3);
+  v[5] = tmul<INV>(v[5], w5);
+  v[6] = tmul<INV>(v[6], w6);
+  v[9] = tmul<INV>(v[9], w9);
+  v[7] = tmul<INV>(v[7], cmul(w4, w3));
+  v[10] = tmul<INV>(v[10], cmul(w8, w2));
+  v[11] = tmul<INV>(v[11], cmul(w8, w3));
+  v[12] = tmul<INV>(v[12], cmul(w8, w4));
+  v[13] = tmul<INV>(v[13], cmul(w8, w5));
+  v[14] = tmul<INV>(v[14], cmul(w8, w6));
+  v[15] = tmul<INV>(v[15], cmul(w8, cmul(w4, w3)));
+}
+
+template <int LOGM>
+struct Shape {
+  static constexpr int M = 1 << LOGM, T = M / 16;
+  static constexpr int S = T >= 16 ? T / 16 : T;  // points per sub-transform of the last stage
+  static constexpr int LDS = M + (LOGM <= 9 ? M / 8 + 32 : 0);  // complex per ring
+  // LDS place of point q.  8 neighbouring lanes take 128 bytes per cycle: the
+  // passes access runs of consecutive q or one q per lane S apart, spread over
+  // the banks by an exclusive-or within each aligned group of 8 (no room for
+  // padding at the large M), by padding at the small ones.
+  __device__ static int at(int q) {
+    if constexpr (LOGM >= 13) return q ^ (((q >> 5) & 3) << 1);
+    if constexpr (LOGM == 12) return q ^ ((q >> 4) & 7);
+    if constexpr (LOGM == 11) return q ^ ((q >> 3) & 7);
+    if constexpr (LOGM == 10) return q ^ ((q >> 3) & 3) ^ (((q >> 6) & 1) << 2);
+    if constexpr (LOGM == 9) return q + (q >> 3) + (q >> 5) * 2;
+    if constexpr (LOGM == 8) return q + (q >> 4);
+    return q + (q >> 3);
+  }
 };
 
-// Builds hi[0..ceil(count/64)) and lo[0..64) for e^{i pi s k / d}.
-template <int TPB>
-__device__ void build_tab(cplx* hi, cplx* lo, int count, int s, int d) {
-  const int nhi = (count + kTabLo - 1) / kTabLo;
-  for (int k = threadIdx.x; k < nhi + kTabLo; k += TPB) {
-    if (k < nhi)
-      hi[k] = expi_pi((int64_t)s * kTabLo * k, d);
-    else
-      lo[k - nhi] = expi_pi((int64_t)s * (k - nhi), d);
-  }
+// A value the compiler takes for new: what is computed from it again (twiddle
+// powers, LDS places) is computed again and not held in registers meanwhile.
+__device__ __forceinline__ int renew(int x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
+__device__ __forceinline__ cplx renew(cplx x) {
+  asm volatile("" : "+v"(x.x), "+v"(x.y));
+  return x;
 }
 
-// Phase table e^{i sgn (m0 + c) phi0} for c in [0, count): double-precision
-// angles (the reference forms m * phi0 the same way).
-template <int TPB>
-__device__ void build_phase(cplx* hi, cplx* lo, int count, int m0, double phi0_over_pi,
-                            double sgn) {
-  const int nhi = (count + kTabLo - 1) / kTabLo;
-  for (int k = threadIdx.x; k < nhi + kTabLo; k += TPB) {
-    double s, c;
-    if (k < nhi) {
-      sincospi(sgn * (double)(m0 + kTabLo * k) * phi0_over_pi, &s, &c);
-      hi[k] = {c, s};
-    } else {
-      sincospi(sgn * (double)(k - nhi) * phi0_over_pi, &s, &c);
-      lo[k - nhi] = {c, s};
-    }
-  }
+__device__ __forceinline__ double swap_lane1(double x) {
+  // lane ^ 1 by a quad permute (1, 0, 3, 2)
+  const long long v = __double_as_longlong(x);
+  const int lo = __builtin_amdgcn_mov_dpp((int)(v & 0xffffffff), 0xB1, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(v >> 32), 0xB1, 0xF, 0xF, true);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
+// e^{-2 pi i k / 32}
+__device__ __constant__ const double kW32[16][2] = {
+    {1.0, 0.0},
+    {0.98078528040323044913, -0.19509032201612826785},
+    {0.92387953251128675613, -0.38268343236508977173},
+    {0.83146961230254523708, -0.55557023301960222474},
+    {0.70710678118654752440, -0.70710678118654752440},
+    {0.55557023301960222474, -0.83146961230254523708},
+    {0.38268343236508977173, -0.92387953251128675613},
+    {0.19509032201612826785, -0.98078528040323044913},
+    {0.0, -1.0},
+    {-0.19509032201612826785, -0.98078528040323044913},
+    {-0.38268343236508977173, -0.92387953251128675613},
+    {-0.55557023301960222474, -0.83146961230254523708},
+    {-0.70710678118654752440, -0.70710678118654752440},
+    {-0.83146961230254523708, -0.55557023301960222474},
+    {-0.92387953251128675613, -0.38268343236508977173},
+    {-0.98078528040323044913, -0.19509032201612826785}};
 
-__device__ __forceinline__ cplx conj_if(cplx v, bool c) { return c ? cplx{v.x, -v.y} : v; }
-
-// for (p = tid; p < n; p += TPB) use(p, load(p)), with the loads of U
-// consecutive iterations issued before any of their uses.  Without this each
-// iteration waits out one global-memory latency, and a ring workgroup has too
-// few waves beside it to hide that.
-template <int TPB, int U, typename T, typename Load, typename Use>
-__device__ __forceinline__ void batched_for(int n, Load load, Use use) {
-  for (int p0 = threadIdx.x; p0 < n; p0 += U * TPB) {
-    T v[U];
+template <int S, bool INV>
+__device__ __forceinline__ void dft_groups(cplx* v) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int p = p0 + u * TPB;
-      v[u] = p < n ? load(p) : T{};
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int p = p0 + u * TPB;
-      if (p < n) use(p, v[u]);
-    }
+  for (int g = 0; g < 16; g += S) {
+    if constexpr (S == 2) dft2<INV>(v[g], v[g + 1]);
+    if constexpr (S == 4) dft4<INV>(v[g], v[g + 1], v[g + 2], v[g + 3]);
+    if constexpr (S == 8) dft8<INV>(v + g);
+    if constexpr (S == 16) dft16<INV, false, false>(v + g);
   }
 }
 
-// Radix-R DFT in place.  Odd R uses the symmetric form: with s_k = v_k + v_{R-k},
-// d_k = v_k - v_{R-k} (k = 1..H, H = (R-1)/2) and c_m + i t_m = e^{sign 2 pi i m/R},
-//   X_j = v_0 + sum_k c_{jk} s_k + i t_{jk} d_k,  X_{R-j} = the same with -i,
-// so only R + 2H complex values are live.  cs[m] = (c_m, t_m), m = 1..H.
-template <int R>
-__device__ __forceinline__ void radix_dft(cplx* v, int sign, const cplx* cs) {
-  if constexpr (R == 2 || R == 4 || R == 8) {
-    SmallDft<R>::run(v, sign, nullptr);
+// v[e], e < 8: the chirped input at p = t + T e -> the convolution there.
+template <int LOGM>
+__device__ __forceinline__ void blue_conv(cplx* v, cplx* lds, int t0, const cplx* __restrict__ bhat,
+                                          const cplx* __restrict__ tw) {
+  typedef Shape<LOGM> P;
+  constexpr int T = P::T, S = P::S;
+  int t = t0;
+  const cplx w1 = tw[t << (13 - LOGM)];  // e^{-2 pi i t / M}
+  dft16<false, true, false>(v);
+  twiddle16<false>(v, w1);
+#pragma unroll
+  for (int k = 0; k < 16; ++k) lds[P::at(k * T + t)] = v[k];
+  __syncthreads();
+  if constexpr (T < 16) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] = lds[P::at((t + T * (i / S)) * S + i % S)];
+    dft_groups<S, false>(v);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] = cmul(v[i], bhat[i * T + t]);
+    dft_groups<S, true>(v);
+    t = renew(t);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) lds[P::at((t + T * (i / S)) * S + i % S)] = v[i];
   } else {
-    constexpr int H = (R - 1) / 2;
-    cplx sm[H], df[H];
-    const cplx x0 = v[0];
-    cplx tot = x0;
+    int nn = t % S, base = (t / S) * T + nn;
+    const cplx w2 = S > 1 ? tw[nn << (17 - LOGM)] : cplx{1.0, 0.0};  // e^{-2 pi i nn / T}
 #pragma unroll
-    for (int k = 1; k <= H; ++k) {
-      sm[k - 1] = cadd(v[k], v[R - k]);
-      df[k - 1] = csub(v[k], v[R - k]);
-      tot = cadd(tot, sm[k - 1]);
-    }
-    v[0] = tot;
+    for (int i = 0; i < 16; ++i) v[i] = lds[P::at(base + i * S)];
+    dft16<false, false, false>(v);
+    if constexpr (S == 1) {
 #pragma unroll
-    for (int j = 1; j <= H; ++j) {
-      cplx a = x0, b = {0.0, 0.0};
+      for (int i = 0; i < 16; ++i) v[i] = cmul(v[i], bhat[i * T + t]);
+    } else {
+      twiddle16<false>(v, w2);
 #pragma unroll
-      for (int k = 1; k <= H; ++k) {
-        const int m = (j * k) % R;
-        const double c = m <= H ? cs[m].x : cs[R - m].x;
-        const double t = m <= H ? cs[m].y : -cs[R - m].y;
-        a.x = fma(c, sm[k - 1].x, a.x);
-        a.y = fma(c, sm[k - 1].y, a.y);
-        b.x = fma(t, df[k - 1].x, b.x);
-        b.y = fma(t, df[k - 1].y, b.y);
+      for (int i = 0; i < 16; ++i) lds[P::at(base + i * S)] = v[i];
+      __syncthreads();
+      if constexpr (S <= 16) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v[i] = lds[P::at((t + T * (i / S)) * S + i % S)];
+        dft_groups<S, false>(v);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v[i] = cmul(v[i], bhat[i * T + t]);
+        dft_groups<S, true>(v);
+        t = renew(t);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) lds[P::at((t + T * (i / S)) * S + i % S)] = v[i];
+      } else {
+        // S = 32: 16 x 2, the radix 2 between lanes t and t ^ 1
+        const int odd = t & 1, b3 = (t >> 1) * 32 + odd;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v[i] = lds[P::at(b3 + 2 * i)];
+        dft16<false, false, false>(v);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const cplx w = odd ? cplx{kW32[i][0], kW32[i][1]} : cplx{1.0, 0.0};
+          const cplx a = cmul(v[i], w);
+          const cplx o = {swap_lane1(a.x), swap_lane1(a.y)};
+          // X = (even + odd, even - odd); times FFT(chirp); and back
+          cplx y = odd ? csub(o, a) : cadd(a, o);
+          y = cmul(y, bhat[i * T + t]);
+          const cplx q = {swap_lane1(y.x), swap_lane1(y.y)};
+          y = odd ? csub(q, y) : cadd(y, q);
+          v[i] = tmul<true>(y, w);
+        }
+        dft16<true, false, false>(v);
+        t = renew(t);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) lds[P::at((t >> 1) * 32 + (t & 1) + 2 * i)] = v[i];
       }
-      v[j] = {a.x - b.y, a.y + b.x};
-      v[R - j] = {a.x + b.y, a.y - b.x};
+      __syncthreads();
+      nn = t % S;
+      base = (t / S) * T + nn;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) v[i] = lds[P::at(base + i * S)];
+      twiddle16<true>(v, renew(w2));
+    }
+    dft16<true, false, false>(v);
+    base = renew(base);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) lds[P::at(base + i * S)] = v[i];
+  }
+  __syncthreads();
+  t = renew(t);
+#pragma unroll
+  for (int k = 0; k < 16; ++k) v[k] = lds[P::at(k * T + t)];
+  twiddle16<true>(v, renew(w1));
+  dft16<true, false, true>(v);
+}
+
+// ------------------------------------------------------------- powers of two
+template <int LOGN>
+struct Pow2Shape {
+  static constexpr int N = 1 << LOGN, T = N / 16, LOGT = LOGN - 4;
+  static constexpr int S = T >= 16 ? T / 16 : T;
+  // LDS place of point q: an exclusive-or with the row q / T, bits reversed,
+  // keeps all three access patterns (runs of lanes, runs of S, one row per
+  // lane) free of bank conflicts
+  __device__ static int at(int q) {
+    if constexpr (LOGT == 2) return q ^ ((q >> 3) & 3);
+    const int r = q >> LOGT;
+    return q ^ (((r & 1) << 2) | (r & 2) | ((r >> 2) & 1));
+  }
+};
+
+// v[e] = x[t + T e] -> X[t + T e] (INV: the unnormalised inverse).
+template <int LOGN, bool INV>
+__device__ __forceinline__ void pow2_fft(cplx* v, cplx* lds, int t, const cplx* __restrict__ tw) {
+  typedef Pow2Shape<LOGN> P;
+  constexpr int T = P::T, S = P::S;
+  dft16<INV, false, false>(v);
+  twiddle16<INV>(v, tw[t << (13 - LOGN)]);
+#pragma unroll
+  for (int k = 0; k < 16; ++k) lds[P::at(k * T + t)] = v[k];
+  __syncthreads();
+  if constexpr (T >= 16) {
+    const int nn = t % S, base = (t / S) * T + nn;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] = lds[P::at(base + i * S)];
+    dft16<INV, false, false>(v);
+    if constexpr (S > 1) {
+      twiddle16<INV>(v, tw[nn << (17 - LOGN)]);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) lds[P::at(base + i * S)] = v[i];
+      __syncthreads();
+    }
+  }
+  if constexpr (S > 1) {
+    // sub-transforms g = t + T i: k = g + R s, R = 256 (T < 16: 16)
+    constexpr int G = 16 / S;
+    cplx u[16];
+#pragma unroll
+    for (int i = 0; i < G; ++i) {
+      const int g = t + T * i;
+      const int q0 = T >= 16 ? (g & 15) * T + (g >> 4) * S : g * T;
+#pragma unroll
+      for (int s = 0; s < S; ++s) u[i * S + s] = lds[P::at(q0 + s)];
+    }
+    dft_groups<S, INV>(u);
+#pragma unroll
+    for (int i = 0; i < G; ++i)
+#pragma unroll
+      for (int s = 0; s < S; ++s) v[i + G * s] = u[i * S + s];
+  }
+}
+
+// ------------------------------------------------------------- rings in and out
+__device__ __forceinline__ double ring_scale(int mode, int n) {
+  return mode == 1 ? 1.0 / (double)n : mode == 2 ? 1.0 / sqrt((double)n) : 1.0;
+}
+__device__ __forceinline__ bool ring_phase(int apply, const RingJob& job) {
+  return apply && rint(job.nphi * job.phi0_over_pi) != 0.0;
+}
+
+// Loads through these take unconditional loads from clamped places (one basic
+// block: all of them in flight together) and drop the unwanted values afterwards.
+
+// v[e] = pixel t + T e of the ring (z = x + i y for a pair of real maps), zero
+// from n on.
+template <int T, int E>
+__device__ __forceinline__ void load_pixels(cplx* v, const RingFwdArgs& a, const RingJob& job,
+                                            int t, int64_t b0, int paired, bool two) {
+  const int n = job.nphi;
+  const int64_t off = b0 * a.map_stride + job.pix_offset;
+  const int64_t next = two ? a.map_stride : 0;
+  const auto at = [&](int e) { return t + T * e < n ? t + T * e : 0; };
+  bool real = a.real_only_all || (a.real_only_2L && n == 2 * a.L);
+  if (paired && !a.f_complex) {
+    const double* s0 = reinterpret_cast<const double*>(a.f) + off;
+#pragma unroll
+    for (int e = 0; e < E; ++e) v[e] = {s0[at(e)], s0[next + at(e)]};
+    real = !two;
+  } else if (paired) {
+    const cplx* s0 = reinterpret_cast<const cplx*>(a.f) + off;
+#pragma unroll
+    for (int e = 0; e < E; ++e) v[e] = {s0[at(e)].x, s0[next + at(e)].x};
+    real = !two;
+  } else if (a.in_single) {
+    const float2* s0 = reinterpret_cast<const float2*>(a.f) + off;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const float2 x = s0[at(e)];
+      v[e] = {(double)x.x, (double)x.y};
+    }
+  } else {
+    const cplx* s0 = reinterpret_cast<const cplx*>(a.f) + off;
+#pragma unroll
+    for (int e = 0; e < E; ++e) v[e] = s0[at(e)];
+  }
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const bool in = t + T * e < n;
+    v[e] = {in ? v[e].x : 0.0, in && !real ? v[e].y : 0.0};
+  }
+}
+
+// Stores a ring whose residues have at most one column each, from registers:
+// residue p = t + T e (phased) is column m = p or p - n.
+template <int T, int E>
+__device__ __forceinline__ void store_direct(const cplx* v, const RingFwdArgs& a,
+                                             const RingJob& job, int t, int64_t b0, bool ph) {
+  const int n = job.nphi;
+  cplx* d0 = a.out + b0 * a.out_map_stride + (int64_t)job.row * a.ncol;
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const int p = t + T * e;
+    int col = p - a.m_first;
+    const bool wrap = col >= n;
+    if (wrap) col -= n;
+    const double sg = wrap && ph ? -1.0 : 1.0;
+    if (p < n && col < a.ncol) d0[col] = {sg * v[e].x, sg * v[e].y};
+  }
+}
+
+// Stores a ring's columns from its residues in LDS: [0, n), real pairs the
+// second map's at [n, 2n).  Column m = k + j n is (-1)^j times residue k (ph).
+template <int T>
+__device__ __forceinline__ void store_columns(const cplx* lds, const RingFwdArgs& a,
+                                              const RingJob& job, int t, int64_t b0, bool two,
+                                              bool ph) {
+  const int n = job.nphi;
+  const int64_t o0 = b0 * a.out_map_stride + (int64_t)job.row * a.ncol;
+  cplx* d0 = a.out + o0;
+  float2* d0s = reinterpret_cast<float2*>(a.out) + o0;
+  int k = (a.m_first + t) % n;
+  if (k < 0) k += n;
+  int j = (a.m_first + t - k) / n;
+  const int dj = T / n, dk = T - dj * n;
+  for (int col = t; col < a.ncol; col += T) {
+    const bool zero = a.zero_neg_2L && n == 2 * a.L && a.m_first + col < 0;
+    const double sg = zero ? 0.0 : ph && (j & 1) ? -1.0 : 1.0;
+    const cplx z = lds[k];
+    if (a.out_single)
+      d0s[col] = make_float2((float)(sg * z.x), (float)(sg * z.y));
+    else
+      d0[col] = {sg * z.x, sg * z.y};
+    if (two) {
+      const cplx y = lds[n + k];
+      d0[a.out_map_stride + col] = {sg * y.x, sg * y.y};
+    }
+    k += dk;
+    j += dj;
+    if (k >= n) {
+      k -= n;
+      ++j;
     }
   }
 }
 
-// One radix-R Stockham pass over n points (Ns = product of the radices done).
-// tw.at(k) = e^{-2 pi i k / n}; the inverse (sign > 0) uses its conjugate.
-// The last pass (Ns R = n) writes exactly the points each butterfly read, so
-// it streams one butterfly at a time; earlier passes hold their butterflies
-// in registers across the barrier between the reads and the writes.
-// P2: Ns is a power of two (every pass of a power-of-two length).
-template <int R, bool P2>
-__device__ __forceinline__ void butterfly(cplx* v, const double* re, const double* im, int j,
-                                          int nb, int Ns, int step, bool cj, int sign,
-                                          const Tab2& tw, const cplx* cs) {
+// Natural-order residues v[e] (t + T e) into LDS for store_columns, times
+// phase(p); real pairs split into X = (z + conj z')/2, Y = (z - conj z')/(2i),
+// z' the residue n - p.  Called by every thread; ends on a barrier.
+template <int T, int E, typename Phase>
+__device__ __forceinline__ void residues_to_lds(cplx* v, cplx* lds, int n, int t, int paired,
+                                                Phase phase) {
+  __syncthreads();
 #pragma unroll
-  for (int r = 0; r < R; ++r) v[r] = {re[lx(j + r * nb)], im[lx(j + r * nb)]};
-  const int jl = P2 ? (j & (Ns - 1)) : j % Ns;
-  if (jl != 0) {
-    const cplx w1 = conj_if(tw.at(jl * step), cj);
-    cplx wr = w1;
-#pragma unroll
-    for (int r = 1; r < R; ++r) {
-      v[r] = cmul(v[r], wr);
-      if (r + 1 < R) wr = cmul(wr, w1);
-    }
+  for (int e = 0; e < E; ++e) {
+    const int p = t + T * e;
+    if (p < n) lds[p] = paired ? v[e] : phase(e, v[e]);
   }
-  radix_dft<R>(v, sign, cs);
+  __syncthreads();
+  if (!paired) return;
+  cplx zc[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const int p = t + T * e;
+    zc[e] = p < n ? lds[p == 0 ? 0 : n - p] : cplx{0.0, 0.0};
+  }
+  __syncthreads();
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const int p = t + T * e;
+    if (p >= n) continue;
+    const cplx X = {0.5 * (v[e].x + zc[e].x), 0.5 * (v[e].y - zc[e].y)};
+    const cplx Y = {0.5 * (v[e].y + zc[e].y), -0.5 * (v[e].x - zc[e].x)};
+    lds[p] = phase(e, X);
+    lds[n + p] = phase(e, Y);
+  }
+  __syncthreads();
 }
 
-template <int R, int TPB, int MAXN, bool P2>
-__device__ __forceinline__ void pass_t(double* re, double* im, int n, int Ns, int sign, const Tab2& tw) {
-  constexpr int MAXB = (MAXN / R + TPB - 1) / TPB;
-  constexpr int H = R / 2 + 1;
-  const int nb = n / R;
-  const bool cj = sign > 0;
-  const int step = n / (Ns * R);
-  cplx cs[H];
-  if constexpr (R != 2 && R != 4 && R != 8) {
-#pragma unroll
-    for (int k = 1; k < H; ++k) cs[k] = conj_if(tw.at(k * (n / R)), cj);
+// The folded spectrum F[q] = sum_{m = q mod n} (-1)^j c(m), m = q + j n in [lo, hi]
+// (the sign for ph), of a map or of z = c_x + i c_y of a pair of real maps.
+struct FoldIn {
+  const cplx* x;
+  const cplx* y;      // second map of a pair, or null
+  const float2* xs;   // complex64 spectra instead of x, or null
+  int m_first, lo, hi, n;
+  bool herm, ph;
+
+  __device__ FoldIn(const RingInvArgs& a, const RingJob& job, int64_t b0, bool two) {
+    const int64_t in0 = b0 * a.in_map_stride + (int64_t)job.row * a.ncol;
+    n = job.nphi;
+    herm = a.herm_mode == 1 || (a.herm_mode == 2 && n == 2 * a.L);
+    lo = herm ? -(a.L - 1) : a.m_lo;
+    hi = herm ? (a.L - 1) : a.m_hi;
+    x = a.in + in0;
+    y = two ? x + a.in_map_stride : nullptr;
+    xs = a.in_single ? reinterpret_cast<const float2*>(a.in) + in0 : nullptr;
+    m_first = a.m_first;
+    ph = ring_phase(a.apply_phase, job);
   }
-  // radices 2 and 4 only ever run as the last pass (see fft_t)
-  if (R == 2 || R == 4 || Ns * R == n) {
-    for (int j = threadIdx.x; j < nb; j += TPB) {
-      cplx v[R];
-      butterfly<R, P2>(v, re, im, j, nb, Ns, step, cj, sign, tw, cs);
+  // u[e] = c(m), or c_x(m) + i c_y(m), for m = at(e), zero where m is outside
+  // [lo, hi]; m < 0 of Hermitian spectra from conj c(-m)
+  template <int E, typename At>
+  __device__ __forceinline__ void gather(cplx* u, At at) const {
+    const auto place = [&](int e) {
+      const int m = at(e);
+      return (m < lo || m > hi) ? 0 : (herm && m < 0 ? -m : m) - m_first;
+    };
+    if (xs) {
 #pragma unroll
-      for (int k = 0; k < R; ++k) {
-        re[lx(j + k * Ns)] = v[k].x;
-        im[lx(j + k * Ns)] = v[k].y;
+      for (int e = 0; e < E; ++e) {
+        const float2 r = xs[place(e)];
+        u[e] = {(double)r.x, (double)r.y};
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < E; ++e) u[e] = x[place(e)];
+    }
+    if (y) {
+      cplx r[E];
+#pragma unroll
+      for (int e = 0; e < E; ++e) r[e] = y[place(e)];
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const double sg = herm && at(e) < 0 ? -1.0 : 1.0;
+        u[e] = {fma(-sg, r[e].y, u[e].x), fma(sg, u[e].y, r[e].x)};
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < E; ++e)
+        if (herm && at(e) < 0) u[e].y = -u[e].y;
+    }
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int m = at(e);
+      if (m < lo || m > hi) u[e] = {0.0, 0.0};
+    }
+  }
+  __device__ static int floor_div(int p, int q) { return p >= 0 ? p / q : -((q - 1 - p) / q); }
+
+  // v[e] = F[t + T e], for rings longer than T
+  template <int T, int E>
+  __device__ __forceinline__ void owned(cplx* v, int t) const {
+    if (hi - lo < n) {  // one m per residue
+#pragma unroll
+      for (int e0 = 0; e0 < E; e0 += 8)
+        gather<8>(v + e0, [&](int e) {
+          const int q = t + T * (e0 + e);
+          return q >= n ? hi + 1 : q <= hi ? q : q - n;
+        });
+      if (ph) {
+#pragma unroll
+        for (int e = 0; e < E; ++e)
+          if (t + T * e > hi) v[e] = {-v[e].x, -v[e].y};
+      }
+      return;
+    }
+    const int j0 = floor_div(lo, n), j1 = floor_div(hi, n);
+#pragma unroll
+    for (int e = 0; e < E; ++e) v[e] = {0.0, 0.0};
+    for (int j = j0; j <= j1; ++j) {
+      const double sg = ph && (j & 1) ? -1.0 : 1.0;
+#pragma unroll
+      for (int e0 = 0; e0 < E; e0 += 8) {
+        cplx u[8];
+        gather<8>(u, [&](int e) {
+          const int q = t + T * (e0 + e);
+          return q < n ? q + j * n : hi + 1;
+        });
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          v[e0 + e] = {fma(sg, u[e].x, v[e0 + e].x), fma(sg, u[e].y, v[e0 + e].y)};
       }
     }
-    __syncthreads();
+  }
+  // a thread's share of residue t % n, for rings of at most T points: the
+  // G = T / n threads of a residue take j = j0 + g, j0 + g + G, ...
+  template <int T>
+  __device__ __forceinline__ cplx shared(int t) const {
+    cplx part = {0.0, 0.0};
+    const int G = T / n, q = t % n, g = t / n;
+    if (g >= G) return part;
+    const int j1 = floor_div(hi, n);
+    for (int jb = floor_div(lo, n) + g; jb <= j1; jb += 8 * G) {
+      cplx u[8];
+      gather<8>(u, [&](int i) { return q + (jb + i * G) * n; });
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const double sg = ph && ((jb + i * G) & 1) ? -1.0 : 1.0;
+        part = {fma(sg, u[i].x, part.x), fma(sg, u[i].y, part.y)};
+      }
+    }
+    return part;
+  }
+};
+
+// Stores pixel t + T e from v[e]; with sub_from the result is subtracted from it.
+template <int T, int E>
+__device__ __forceinline__ void store_pixels(cplx* v, const RingInvArgs& a, const RingJob& job,
+                                             int t, int64_t b0, int paired, bool two, bool herm) {
+  const int n = job.nphi;
+  const int64_t off = b0 * a.map_stride + job.pix_offset;
+  if (paired && a.f_complex) {
+    // real maps as complex128 with a zero imaginary part
+    cplx* d0 = reinterpret_cast<cplx*>(a.f) + off;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int p = t + T * e;
+      if (p >= n) continue;
+      cplx r0 = {v[e].x, 0.0}, r1 = {v[e].y, 0.0};
+      if (a.sub_from) {
+        const cplx* u0 = reinterpret_cast<const cplx*>(a.sub_from) + off;
+        r0 = csub(u0[p], r0);
+        if (two) r1 = csub(u0[a.map_stride + p], r1);
+      }
+      d0[p] = r0;
+      if (two) d0[a.map_stride + p] = r1;
+    }
+  } else if (paired || !a.f_complex) {
+    double* d0 = reinterpret_cast<double*>(a.f) + off;
+    if (a.sub_from) {
+      const double* u0 = reinterpret_cast<const double*>(a.sub_from) + off;
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const int p = t + T * e;
+        if (p < n) v[e] = {u0[p] - v[e].x, two ? u0[a.map_stride + p] - v[e].y : 0.0};
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int p = t + T * e;
+      if (p >= n) continue;
+      d0[p] = v[e].x;
+      if (two) d0[a.map_stride + p] = v[e].y;
+    }
+  } else if (a.f_single) {
+    float2* d0 = reinterpret_cast<float2*>(a.f) + off;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int p = t + T * e;
+      if (p < n) d0[p] = make_float2((float)v[e].x, herm ? 0.0f : (float)v[e].y);
+    }
+  } else {
+    cplx* d0 = reinterpret_cast<cplx*>(a.f) + off;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      if (herm) v[e].y = 0.0;
+    }
+    if (a.sub_from) {
+      const cplx* u0 = reinterpret_cast<const cplx*>(a.sub_from) + off;
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const int p = t + T * e;
+        if (p < n) v[e] = csub(u0[p], v[e]);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int p = t + T * e;
+      if (p < n) d0[p] = v[e];
+    }
+  }
+}
+
+// Consecutive jobs of one kind within a launch: blocks [block0, ...) hold
+// blockDim / T rings each.
+struct RingSeg {
+  int body;      // log2 of the convolution (Bluestein), or kPow2Body + log2 n
+  int job0, count, block0;
+  int direct;    // forward: every residue has at most one column (ring_direct)
+  int lds_ring;  // complex of LDS per ring
+};
+constexpr int kPow2Body = 32;
+constexpr int kMaxSegs = kBlueClasses + 1;
+constexpr int kRingLdsMax = 160 * 1024;
+struct RingSegs {
+  RingSeg s[kMaxSegs];
+  int n;
+};
+
+// the ring of this thread, and its place in it
+template <int T>
+struct RingOf {
+  int t, sub;
+  bool valid, two;
+  int64_t b0;
+  RingJob job;
+  cplx* lds;
+  __device__ RingOf(const RingJob* jobs, const RingSeg& seg, int paired, int batch, void* raw) {
+    t = threadIdx.x % T;
+    sub = threadIdx.x / T;
+    const int r = (blockIdx.x - seg.block0) * (blockDim.x / T) + sub;
+    valid = r < seg.count;
+    job = jobs[seg.job0 + (valid ? r : seg.count - 1)];
+    b0 = paired ? 2 * (int64_t)blockIdx.y : (int64_t)blockIdx.y;
+    two = paired && b0 + 1 < batch;
+    lds = reinterpret_cast<cplx*>(raw) + sub * seg.lds_ring;
+  }
+};
+
+template <int LOGM>
+__device__ __forceinline__ void blue_fwd(const RingFwdArgs& a, const RingSeg& seg, int paired,
+                                         void* raw) {
+  typedef Shape<LOGM> P;
+  constexpr int T = P::T;
+  const RingOf<T> ring(a.jobs, seg, paired, a.batch, raw);
+  const RingJob& job = ring.job;
+  cplx* lds = ring.lds;
+  const int n = job.nphi;
+  int t = ring.t;
+  const cplx* __restrict__ bhat = a.chirp_pool + job.chirp_off;
+  const cplx* __restrict__ chirp = bhat + P::M;
+  const cplx* __restrict__ phase = chirp + n;
+
+  cplx v[16];
+  load_pixels<T, 8>(v, a, job, t, ring.b0, paired, ring.two);
+  cplx c[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const int p = t + T * e;
+    c[e] = p < n ? chirp[p] : cplx{0.0, 0.0};
+  }
+#pragma unroll
+  for (int e = 0; e < 8; ++e) v[e] = cmul(v[e], c[e]);
+  blue_conv<LOGM>(v, lds, t, bhat, a.chirp_pool);
+
+  const double w = (a.apply_weight ? job.weight : 1.0) * ring_scale(a.norm_mode, n);
+  t = renew(t);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const int p = t + T * e;
+    const cplx ch = p < n ? chirp[p] : cplx{0.0, 0.0};
+    v[e] = cmul(v[e], cplx{w * ch.x, w * ch.y});
+  }
+  const bool ph = ring_phase(a.apply_phase, job);
+  if (seg.direct) {
+    if (ring.valid) store_direct<T, 8>(v, a, job, t, ring.b0, false);
     return;
   }
-  if constexpr (R != 2 && R != 4) {
-    cplx v[MAXB][R];
-#pragma unroll
-    for (int c = 0; c < MAXB; ++c) {
-      const int j = threadIdx.x + c * TPB;
-      if (j < nb) butterfly<R, P2>(v[c], re, im, j, nb, Ns, step, cj, sign, tw, cs);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int c = 0; c < MAXB; ++c) {
-      const int j = threadIdx.x + c * TPB;
-      if (j < nb) {
-        const int jl = P2 ? (j & (Ns - 1)) : j % Ns;
-        const int base = (j - jl) * R + jl;
-#pragma unroll
-        for (int k = 0; k < R; ++k) {
-          re[lx(base + k * Ns)] = v[c][k].x;
-          im[lx(base + k * Ns)] = v[c][k].y;
-        }
-      }
-    }
-    __syncthreads();
-  }
+  residues_to_lds<T, 8>(v, lds, n, t, paired, [&](int e, cplx z) {
+    return ph ? cmul(z, phase[t + T * e]) : z;
+  });
+  if (ring.valid) store_columns<T>(lds, a, job, t, ring.b0, ring.two, ph);
 }
 
-// Out-of-line pass: the smooth and Bluestein kernels call their passes so
-// that each pass gets its own register allocation.
-template <int R, int TPB, int MAXN, bool P2>
-__device__ __noinline__ void pass_call(double* re, double* im, int n, int Ns, int sign,
-                                       const Tab2 tw) {
-  pass_t<R, TPB, MAXN, P2>(re, im, n, Ns, sign, tw);
-}
+template <int LOGM>
+__device__ __forceinline__ void blue_inv(const RingInvArgs& a, const RingSeg& seg, int paired,
+                                         void* raw) {
+  typedef Shape<LOGM> P;
+  constexpr int T = P::T;
+  const RingOf<T> ring(a.jobs, seg, paired, a.batch, raw);
+  const RingJob& job = ring.job;
+  cplx* lds = ring.lds;
+  const int n = job.nphi;
+  int t = ring.t;
+  const cplx* __restrict__ bhat = a.chirp_pool + job.chirp_off;
+  const cplx* __restrict__ chirp = bhat + P::M;
+  const cplx* __restrict__ phase = chirp + n;
+  const FoldIn in(a, job, ring.b0, ring.two);
 
-template <int R, int TPB, int MAXN, bool INL, bool P2>
-__device__ __forceinline__ void pass_any(double* re, double* im, int n, int Ns, int sign,
-                                         const Tab2& tw) {
-  if constexpr (INL)
-    pass_t<R, TPB, MAXN, P2>(re, im, n, Ns, sign, tw);
-  else
-    pass_call<R, TPB, MAXN, P2>(re, im, n, Ns, sign, tw);
-}
-
-template <int TPB, int MAXN, bool POW2, bool INL>
-__device__ __forceinline__ void run_pass(int R, double* re, double* im, int n, int Ns, int sign,
-                                         const Tab2& tw) {
-  switch (R) {
-    case 8: pass_any<8, TPB, MAXN, INL, POW2>(re, im, n, Ns, sign, tw); break;
-    case 4: pass_any<4, TPB, MAXN, INL, POW2>(re, im, n, Ns, sign, tw); break;
-    case 2: pass_any<2, TPB, MAXN, INL, POW2>(re, im, n, Ns, sign, tw); break;
-    default:
-      if constexpr (!POW2) {
-        switch (R) {
-          case 3: pass_any<3, TPB, MAXN, INL, false>(re, im, n, Ns, sign, tw); break;
-          case 5: pass_any<5, TPB, MAXN, INL, false>(re, im, n, Ns, sign, tw); break;
-          case 7: pass_any<7, TPB, MAXN, INL, false>(re, im, n, Ns, sign, tw); break;
-          case 11: pass_any<11, TPB, MAXN, INL, false>(re, im, n, Ns, sign, tw); break;
-          case 13: pass_any<13, TPB, MAXN, INL, false>(re, im, n, Ns, sign, tw); break;
-          default: break;
-        }
-      }
-  }
-}
-
-// Mixed-radix FFT in place (prime factors <= 13, or powers of two only when
-// POW2); sign -1 forward, +1 inverse.  Radices in the order: odd primes
-// ascending, 8s, then the one 4 or 2 -- so a 4 or 2 is always the last
-// (streamed) pass.
-template <int TPB, int MAXN, bool POW2, bool INL>
-__device__ void fft_t(double* re, double* im, int n, int sign, const Tab2& tw) {
-  int fac[16];
-  int nf = 0, rem = n;
-  if (!POW2) {
-    const int odd[5] = {3, 5, 7, 11, 13};
-    for (int q = 0; q < 5; ++q)
-      while (rem % odd[q] == 0 && nf < 16) { fac[nf++] = odd[q]; rem /= odd[q]; }
-  }
-  while (rem % 8 == 0 && nf < 16) { fac[nf++] = 8; rem /= 8; }
-  if (rem % 4 == 0) { fac[nf++] = 4; rem /= 4; }
-  if (rem % 2 == 0) { fac[nf++] = 2; rem /= 2; }
-  if (rem != 1) return;  // unreachable: the host routes other lengths to Bluestein
-  int Ns = 1;
-  for (int i = 0; i < nf; ++i) {
-    run_pass<TPB, MAXN, POW2, INL>(fac[i], re, im, n, Ns, sign, tw);
-    Ns *= fac[i];
-  }
-}
-
-// LDS layout of a ring workgroup: tables (576 complex) | re im, each
-// lx_len(N) words (points at lx(p)); the data region is at least 2 TPB
-// doubles (the inverse fold's partial sums).
-// Tables: FFT twiddles (hi <= 128, lo 64), chirp e^{-i pi k/n} for k < 2n
-// (hi <= 128, lo 64; Bluestein only), phase over <= 8192 values of m
-// (hi <= 128, lo 64).
-constexpr int kTabCplx = 576;
-
-struct RingLds {
-  double* re;
-  double* im;
-  cplx* tw_hi;
-  cplx* tw_lo;
-  cplx* ch_hi;
-  cplx* ch_lo;
-  cplx* ph_hi;
-  cplx* ph_lo;
-};
-
-__device__ __forceinline__ RingLds ring_lds(double* smem, int N) {
-  RingLds s;
-  s.re = smem + 2 * kTabCplx;
-  s.im = s.re + lx_len(N);
-  cplx* t = reinterpret_cast<cplx*>(smem);
-  s.tw_hi = t;
-  s.tw_lo = t + 128;
-  s.ch_hi = t + 192;
-  s.ch_lo = t + 320;
-  s.ph_hi = t + 384;
-  s.ph_lo = t + 512;
-  return s;
-}
-
-// The DFT of the n points in re/im (sign -1 forward, +1 inverse, unnormalised),
-// direct or by Bluestein; tables must be built.
-// KIND: kPow2 (power-of-two ring), kSmooth (prime factors <= 13), kBlue.
-constexpr int kPow2 = 0, kSmooth = 1, kBlue = 2;
-
-template <int TPB, int MAXN, int KIND>
-__device__ void ring_transform(const RingLds& s, int n, int M, const cplx* chirp_hat, int sign) {
-  const Tab2 tw = {s.tw_hi, s.tw_lo};
-  if constexpr (KIND != kBlue) {
-    fft_t<TPB, MAXN, KIND == kPow2, KIND == kPow2>(s.re, s.im, n, sign, tw);
+  cplx v[16];
+  cplx part = {0.0, 0.0};
+  if (n > T) {
+    in.template owned<T, 8>(v, t);
   } else {
-  const Tab2 ch = {s.ch_hi, s.ch_lo};  // e^{-i pi k / n}, k < 2n (n <= 4096: k^2 < 2^31)
-  const bool cj = sign > 0;
-  for (int p = threadIdx.x; p < M; p += TPB) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = {0.0, 0.0};
+    part = in.template shared<T>(t);
+  }
+  lds[t] = part;
+  __syncthreads();
+  if (n <= T && t < n) {
+    for (int g = 0; g < T / n; ++g) v[0] = cadd(v[0], lds[g * n + t]);
+  }
+  const double w = (a.apply_weight ? job.weight : 1.0) * ring_scale(a.norm_mode, n);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const int p = t + T * e;
     if (p < n) {
-      cplx x = {s.re[lx(p)], cj ? -s.im[lx(p)] : s.im[lx(p)]};
-      x = cmul(x, ch.at((int)(((unsigned)p * (unsigned)p) % (unsigned)(2 * n))));
-      s.re[lx(p)] = x.x;
-      s.im[lx(p)] = x.y;
-    } else {
-      s.re[lx(p)] = 0.0;
-      s.im[lx(p)] = 0.0;
+      const cplx ch = chirp[p];
+      // conj(F e^{i pi p / n}) c_p
+      cplx f = {w * v[e].x, -w * v[e].y};
+      if (in.ph) f = cmul(f, phase[p]);
+      v[e] = cmul(f, ch);
     }
   }
-  __syncthreads();
-  fft_t<TPB, MAXN, true, false>(s.re, s.im, M, -1, tw);
-  batched_for<TPB, 8, cplx>(
-      M, [&](int k) { return chirp_hat[k]; },
-      [&](int k, cplx c) {
-        const cplx a = cmul(cplx{s.re[lx(k)], s.im[lx(k)]}, c);
-        s.re[lx(k)] = a.x;
-        s.im[lx(k)] = a.y;
-      });
-  __syncthreads();
-  fft_t<TPB, MAXN, true, false>(s.re, s.im, M, +1, tw);
-  for (int k = threadIdx.x; k < n; k += TPB) {
-    const cplx a = cmul(cplx{s.re[lx(k)], s.im[lx(k)]}, ch.at((int)(((unsigned)k * (unsigned)k) % (unsigned)(2 * n))));
-    s.re[lx(k)] = a.x;
-    s.im[lx(k)] = cj ? -a.y : a.y;
+  __syncthreads();  // the partial sums are read
+  blue_conv<LOGM>(v, lds, t, bhat, a.chirp_pool);
+  if (!ring.valid) return;
+  t = renew(t);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const int p = t + T * e;
+    const cplx z = cmul(v[e], p < n ? chirp[p] : cplx{0.0, 0.0});
+    v[e] = {z.x, -z.y};
   }
-  __syncthreads();
-  }
+  store_pixels<T, 8>(v, a, job, t, ring.b0, paired, ring.two, in.herm);
 }
 
-template <int TPB, bool BLUE>
-__device__ void build_fft_tables(const RingLds& s, int n, int M) {
-  const int N = BLUE ? M : n;
-  build_tab<TPB>(s.tw_hi, s.tw_lo, N, -2, N);        // e^{-2 pi i k / N}
-  if (BLUE) build_tab<TPB>(s.ch_hi, s.ch_lo, 2 * n, -1, n);  // e^{-i pi k / n}
+// e^{-i pi (t + T e) / N} of a power-of-two ring: e^{-i pi t / N} from the
+// twiddle table times e^{-i pi e / 16}
+template <int LOGN>
+__device__ __forceinline__ cplx pow2_phase(cplx base, int e) {
+  return cmul(base, cplx{kW32[e][0], kW32[e][1]});
+}
+
+// direct, real pairs: the columns m in [0, n / 2)
+template <int LOGN>
+__device__ __forceinline__ void pow2_fwd(const RingFwdArgs& a, const RingSeg& seg, int paired,
+                                         void* raw) {
+  typedef Pow2Shape<LOGN> P;
+  constexpr int T = P::T, N = P::N;
+  const RingOf<T> ring(a.jobs, seg, paired, a.batch, raw);
+  const RingJob& job = ring.job;
+  cplx* lds = ring.lds;
+  const int t = ring.t;
+  const cplx* __restrict__ tw = a.chirp_pool;
+  cplx v[16];
+  load_pixels<T, 16>(v, a, job, t, ring.b0, paired, ring.two);
+  pow2_fft<LOGN, false>(v, lds, t, tw);
+  const double w = (a.apply_weight ? job.weight : 1.0) * ring_scale(a.norm_mode, N);
+#pragma unroll
+  for (int e = 0; e < 16; ++e) v[e] = {w * v[e].x, w * v[e].y};
+  const bool ph = ring_phase(a.apply_phase, job);
+  const cplx base = tw[t << (12 - LOGN)];
+  if (seg.direct && paired) {
+    // X and Y of the residues below N / 2 from z and the upper half's z'
+    __syncthreads();
+#pragma unroll
+    for (int e = 8; e < 16; ++e) lds[T * e + t] = v[e];
+    __syncthreads();
+    if (!ring.valid) return;
+    cplx* d0 = a.out + ring.b0 * a.out_map_stride + (int64_t)job.row * a.ncol;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int p = t + T * e;
+      const cplx z = v[e], zc = p == 0 ? z : lds[N - p];
+      cplx X = {0.5 * (z.x + zc.x), 0.5 * (z.y - zc.y)};
+      cplx Y = {0.5 * (z.y + zc.y), -0.5 * (z.x - zc.x)};
+      if (ph) {
+        const cplx f = pow2_phase<LOGN>(base, e);
+        X = cmul(X, f);
+        Y = cmul(Y, f);
+      }
+      if (p < a.ncol) {
+        d0[p] = X;
+        if (ring.two) d0[a.out_map_stride + p] = Y;
+      }
+    }
+    return;
+  }
+  if (seg.direct) {
+    if (ph) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) v[e] = cmul(v[e], pow2_phase<LOGN>(base, e));
+    }
+    if (ring.valid) store_direct<T, 16>(v, a, job, t, ring.b0, ph);
+    return;
+  }
+  residues_to_lds<T, 16>(v, lds, N, t, paired, [&](int e, cplx z) {
+    return ph ? cmul(z, pow2_phase<LOGN>(base, e)) : z;
+  });
+  if (ring.valid) store_columns<T>(lds, a, job, t, ring.b0, ring.two, ph);
+}
+
+template <int LOGN>
+__device__ __forceinline__ void pow2_inv(const RingInvArgs& a, const RingSeg& seg, int paired,
+                                         void* raw) {
+  typedef Pow2Shape<LOGN> P;
+  constexpr int T = P::T, N = P::N;
+  const RingOf<T> ring(a.jobs, seg, paired, a.batch, raw);
+  const RingJob& job = ring.job;
+  cplx* lds = ring.lds;
+  const int t = ring.t;
+  const cplx* __restrict__ tw = a.chirp_pool;
+  const FoldIn in(a, job, ring.b0, ring.two);
+  cplx v[16];
+  in.template owned<T, 16>(v, t);
+  const double w = (a.apply_weight ? job.weight : 1.0) * ring_scale(a.norm_mode, N);
+#pragma unroll
+  for (int e = 0; e < 16; ++e) v[e] = {w * v[e].x, w * v[e].y};
+  if (in.ph) {
+    const cplx base = tw[t << (12 - LOGN)];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) v[e] = tmul<true>(v[e], pow2_phase<LOGN>(base, e));
+  }
+  pow2_fft<LOGN, true>(v, lds, t, tw);
+  if (ring.valid) store_pixels<T, 16>(v, a, job, t, ring.b0, paired, ring.two, in.herm);
+}
+
+// Runs the body of this block's segment: those whose rings of T threads fit WG.
+template <int WG, int DIR, typename Args>
+__device__ __forceinline__ void ring_body(const Args& a, const RingSeg& seg, int paired,
+                                          void* raw) {
+#define S2H_BLUE(L)                                                             \
+  case L:                                                                       \
+    if constexpr (Shape<L>::T <= WG && Shape<L>::T * kSpan >= WG) {             \
+      if constexpr (DIR == 0) blue_fwd<L>(a, seg, paired, raw);                 \
+      else blue_inv<L>(a, seg, paired, raw);                                    \
+    }                                                                           \
+    break;
+#define S2H_POW2(L)                                                             \
+  case kPow2Body + L:                                                           \
+    if constexpr (Pow2Shape<L>::T <= WG && Pow2Shape<L>::T * kSpan >= WG) {     \
+      if constexpr (DIR == 0) pow2_fwd<L>(a, seg, paired, raw);                 \
+      else pow2_inv<L>(a, seg, paired, raw);                                    \
+    }                                                                           \
+    break;
+  constexpr int kSpan = WG == 64 ? 16 : 8;
+  switch (seg.body) {
+    S2H_BLUE(6) S2H_BLUE(7) S2H_BLUE(8) S2H_BLUE(9) S2H_BLUE(10) S2H_BLUE(11) S2H_BLUE(12)
+    S2H_BLUE(13)
+    S2H_POW2(6) S2H_POW2(7) S2H_POW2(8) S2H_POW2(9) S2H_POW2(10) S2H_POW2(11) S2H_POW2(12)
+    default: break;
+  }
+#undef S2H_BLUE
+#undef S2H_POW2
+}
+
+__device__ __forceinline__ RingSeg seg_of_block(const RingSegs& g) {
+  int i = 0;
+  while (i + 1 < g.n && (int)blockIdx.x >= g.s[i + 1].block0) ++i;
+  return g.s[i];
 }
 
 }  // namespace
 
-// Extra scale of one ring's transform: 1, 1/n or 1/sqrt(n) (the reference's
-// fft_norm modes, lib/src/s2fft_callbacks.cu:256-308).
-__device__ __forceinline__ double norm_scale(int mode, int n) {
-  return mode == 1 ? 1.0 / (double)n : mode == 2 ? 1.0 / sqrt((double)n) : 1.0;
-}
-
-// ------------------------------------------------------------------ forward
 // gridDim.y: maps (complex input) or map pairs (real input, `paired`).
-template <int TPB, int MAXN, int KIND>
-__global__ void __launch_bounds__(TPB) ring_fwd_kernel(RingFwdArgs a, int job0, int paired) {
-  constexpr bool BLUE = KIND == kBlue;
-  extern __shared__ double smem[];
-  const RingJob job = a.jobs[job0 + blockIdx.x];
-  const int n = job.nphi;
-  const int M = BLUE ? job.conv_len : n;
-  const RingLds s = ring_lds(smem, M);
-  const int64_t b0 = paired ? 2 * (int64_t)blockIdx.y : (int64_t)blockIdx.y;
-  const bool two = paired && b0 + 1 < a.batch;
-
-  build_fft_tables<TPB, BLUE>(s, n, M);
-  if (a.apply_phase) build_phase<TPB>(s.ph_hi, s.ph_lo, a.ncol, a.m_first, job.phi0_over_pi, -1.0);
-
-  const auto put = [&](int p, cplx v) {
-    s.re[lx(p)] = v.x;
-    s.im[lx(p)] = v.y;
-  };
-  if (paired) {
-    // real data: z = x_b0 + i x_b0+1
-    if (a.f_complex) {
-      const cplx* s0 = reinterpret_cast<const cplx*>(a.f) + b0 * a.map_stride + job.pix_offset;
-      batched_for<TPB, 8, cplx>(
-          n, [&](int p) { return cplx{s0[p].x, two ? s0[a.map_stride + p].x : 0.0}; }, put);
-    } else {
-      const double* s0 = reinterpret_cast<const double*>(a.f) + b0 * a.map_stride + job.pix_offset;
-      batched_for<TPB, 8, cplx>(
-          n, [&](int p) { return cplx{s0[p], two ? s0[a.map_stride + p] : 0.0}; }, put);
-    }
-  } else if (a.in_single) {
-    const bool real_only = a.real_only_all || (a.real_only_2L && n == 2 * a.L);
-    const float2* src = reinterpret_cast<const float2*>(a.f) + b0 * a.map_stride + job.pix_offset;
-    batched_for<TPB, 8, cplx>(
-        n,
-        [&](int p) {
-          const float2 v = src[p];
-          return cplx{(double)v.x, real_only ? 0.0 : (double)v.y};
-        },
-        put);
-  } else {
-    const bool real_only = a.real_only_all || (a.real_only_2L && n == 2 * a.L);
-    const cplx* src = reinterpret_cast<const cplx*>(a.f) + b0 * a.map_stride + job.pix_offset;
-    batched_for<TPB, 8, cplx>(
-        n,
-        [&](int p) {
-          const cplx v = src[p];
-          return cplx{v.x, real_only ? 0.0 : v.y};
-        },
-        put);
-  }
-  __syncthreads();
-  ring_transform<TPB, MAXN, KIND>(s, n, M, a.chirp_pool + job.chirp_off, -1);
-
-  const double w = (a.apply_weight ? job.weight : 1.0) * norm_scale(a.norm_mode, n);
-  const Tab2 ph = {s.ph_hi, s.ph_lo};
-  const int64_t o0 = b0 * a.out_map_stride + (int64_t)job.row * a.ncol;
-  cplx* d0 = a.out + o0;
-  float2* d0s = reinterpret_cast<float2*>(a.out) + o0;
-  for (int col = threadIdx.x; col < a.ncol; col += TPB) {
-    const int m = a.m_first + col;
-    int k = m % n;
-    if (k < 0) k += n;
-    const bool zero = a.zero_neg_2L && n == 2 * a.L && m < 0;
-    const cplx f = a.apply_phase ? ph.at(col) : cplx{1.0, 0.0};
-    const cplx z = {s.re[lx(k)], s.im[lx(k)]};
-    if (paired) {
-      const int k2 = k == 0 ? 0 : n - k;
-      const cplx zc = {s.re[lx(k2)], -s.im[lx(k2)]};
-      // X = (z + zc)/2, Y = (z - zc)/(2i)
-      const cplx X = {0.5 * (z.x + zc.x), 0.5 * (z.y + zc.y)};
-      const cplx Y = {0.5 * (z.y - zc.y), -0.5 * (z.x - zc.x)};
-      const cplx vx = cmul(cplx{X.x * w, X.y * w}, f);
-      d0[col] = zero ? cplx{0.0, 0.0} : vx;
-      if (two) {
-        const cplx vy = cmul(cplx{Y.x * w, Y.y * w}, f);
-        d0[a.out_map_stride + col] = zero ? cplx{0.0, 0.0} : vy;
-      }
-    } else {
-      const cplx v = zero ? cplx{0.0, 0.0} : cmul(cplx{z.x * w, z.y * w}, f);
-      if (a.out_single)
-        d0s[col] = make_float2((float)v.x, (float)v.y);
-      else
-        d0[col] = v;
-    }
-  }
-}
-
-// ------------------------------------------------------------------ inverse
-// The folded spectrum of one ring, F[q] = w sum_{m = q mod n} e^{i m phi0} c(m),
-// for a map (z = c) or a pair of real maps (z = c_x + i c_y, whose inverse is
-// x + i y), m over [lo, hi].
-struct FoldSrc {
-  const cplx* x;  // column 0 of the ring's row (m = m_first)
-  const cplx* y;  // second map of a pair, or null
-  const float2* xs;  // complex64 row instead of x (unpaired maps), or null
-  int m_first;
-  bool herm;      // m < 0 read as conj(c(-m))
-  bool phase;
-  Tab2 ph;        // e^{i (lo + k) phi0}
-  int lo;
-
-  __device__ __forceinline__ cplx one(const cplx* src, int m) const {
-    if (herm && m < 0) {
-      const cplx t = src[-m - m_first];
-      return {t.x, -t.y};
-    }
-    return src[m - m_first];
-  }
-  __device__ __forceinline__ cplx one_single(int m) const {
-    if (herm && m < 0) {
-      const float2 t = xs[-m - m_first];
-      return {(double)t.x, -(double)t.y};
-    }
-    const float2 t = xs[m - m_first];
-    return {(double)t.x, (double)t.y};
-  }
-  // z(m) with the phase applied
-  __device__ __forceinline__ cplx at(int m) const {
-    cplx z = xs ? one_single(m) : one(x, m);
-    if (y) {
-      const cplx v = one(y, m);
-      z = {z.x - v.y, z.y + v.x};
-    }
-    return phase ? cmul(z, ph.at(m - lo)) : z;
-  }
-};
-
-// Writes F[q] (times w) to re/im[q], q < n: the sum over m = q (mod n), i.e.
-// m = lo + r + c n with r = (q - lo) mod n, c = 0, 1, ...  The terms of one q
-// are summed in increasing m, so the result does not depend on the launch.
-// Two layouts:
-//  n >= TPB: thread t owns q = t, t + TPB, ... and adds their terms in LDS;
-//  n <  TPB: G = TPB / n threads share a q (thread t: q = t % n, g = t / n
-//            takes the chunks c = g, g + G, ...), their partial sums meet in
-//            LDS (part, 2 TPB doubles) in order of g.
-// Both issue U loads before using them: the loads are independent, and a
-// ring workgroup has too few waves to hide one latency per term.
-template <int TPB>
-__device__ void fold_ring(const FoldSrc& src, int n, int hi, double w, double* re, double* im,
-                          double* part) {
-  constexpr int U = 8;
-  const int t = threadIdx.x;
-  const int lo = src.lo;
-  const int nm = hi - lo + 1;
-  const int nc = (nm + n - 1) / n;  // chunks of n consecutive m
-  const int lo_mod = ((-lo) % n + n) % n;
-  const auto r_of = [&](int q) { return q + lo_mod >= n ? q + lo_mod - n : q + lo_mod; };
-  if (n >= TPB) {
-    for (int q = t; q < n; q += TPB) {
-      re[lx(q)] = 0.0;
-      im[lx(q)] = 0.0;
-    }
-    const int nq = (n + TPB - 1) / TPB;
-    const int nslot = nq * nc;  // slot = (qi, c): q = t + qi TPB, m = lo + q + c n
-    for (int s0 = 0; s0 < nslot; s0 += U) {
-      cplx v[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int sl = s0 + u, qi = sl / nc, q = t + qi * TPB;
-        const int m = lo + r_of(q) + (sl - qi * nc) * n;
-        v[u] = (sl < nslot && q < n && m <= hi) ? src.at(m) : cplx{0.0, 0.0};
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int sl = s0 + u, qi = sl / nc, q = t + qi * TPB;
-        const int m = lo + r_of(q) + (sl - qi * nc) * n;
-        if (sl < nslot && q < n && m <= hi) {
-          re[lx(q)] += v[u].x;
-          im[lx(q)] += v[u].y;
-        }
-      }
-    }
-    for (int q = t; q < n; q += TPB) {
-      re[lx(q)] *= w;
-      im[lx(q)] *= w;
-    }
-    return;
-  }
-  const int G = TPB / n;
-  const int q = t % n, g = t / n, r = r_of(q);
-  const int ns = (nc + G - 1) / G;  // chunks per thread
-  cplx acc = {0.0, 0.0};
-  if (g < G) {
-    for (int s0 = 0; s0 < ns; s0 += U) {
-      cplx v[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int m = lo + r + (g + (s0 + u) * G) * n;
-        v[u] = (s0 + u < ns && m <= hi) ? src.at(m) : cplx{0.0, 0.0};
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) acc = cadd(acc, v[u]);
-    }
-    part[2 * t] = acc.x;
-    part[2 * t + 1] = acc.y;
-  }
-  __syncthreads();
-  cplx tot = {0.0, 0.0};
-  if (t < n) {
-    for (int gg = 0; gg < G; ++gg) tot = cadd(tot, cplx{part[2 * (gg * n + t)], part[2 * (gg * n + t) + 1]});
-  }
-  __syncthreads();  // part overlaps re/im
-  if (t < n) {
-    re[lx(t)] = tot.x * w;
-    im[lx(t)] = tot.y * w;
-  }
-}
-
-template <int TPB, int MAXN, int KIND>
-__global__ void __launch_bounds__(TPB) ring_inv_kernel(RingInvArgs a, int job0, int paired) {
-  constexpr bool BLUE = KIND == kBlue;
-  extern __shared__ double smem[];
-  const RingJob job = a.jobs[job0 + blockIdx.x];
-  const int n = job.nphi;
-  const int M = BLUE ? job.conv_len : n;
-  const RingLds s = ring_lds(smem, M);
-  const int64_t b0 = paired ? 2 * (int64_t)blockIdx.y : (int64_t)blockIdx.y;
-  const bool two = paired && b0 + 1 < a.batch;
-  const bool herm = a.herm_mode == 1 || (a.herm_mode == 2 && n == 2 * a.L);
-  const int lo = herm ? -(a.L - 1) : a.m_lo;
-  const int hi = herm ? (a.L - 1) : a.m_hi;
-
-  build_fft_tables<TPB, BLUE>(s, n, M);
-  if (a.apply_phase) build_phase<TPB>(s.ph_hi, s.ph_lo, hi - lo + 1, lo, job.phi0_over_pi, 1.0);
-  __syncthreads();
-
-  const double w = (a.apply_weight ? job.weight : 1.0) * norm_scale(a.norm_mode, n);
-  FoldSrc fs;
-  fs.x = a.in + b0 * a.in_map_stride + (int64_t)job.row * a.ncol;
-  fs.y = two ? fs.x + a.in_map_stride : nullptr;
-  fs.xs = a.in_single ? reinterpret_cast<const float2*>(a.in) + b0 * a.in_map_stride +
-                            (int64_t)job.row * a.ncol
-                      : nullptr;
-  fs.m_first = a.m_first;
-  fs.herm = herm;
-  fs.phase = a.apply_phase;
-  fs.ph = {s.ph_hi, s.ph_lo};
-  fs.lo = lo;
-  fold_ring<TPB>(fs, n, hi, w, s.re, s.im, s.re);
-  __syncthreads();
-  ring_transform<TPB, MAXN, KIND>(s, n, M, a.chirp_pool + job.chirp_off, +1);
-
-  // store; with sub_from the result is subtracted from it (a residual)
-  const int64_t off = b0 * a.map_stride + job.pix_offset;
-  if (paired || !a.f_complex) {
-    double* d0 = reinterpret_cast<double*>(a.f) + off;
-    if (a.sub_from) {
-      const double* u0 = reinterpret_cast<const double*>(a.sub_from) + off;
-      batched_for<TPB, 8, cplx>(
-          n, [&](int p) { return cplx{u0[p], two ? u0[a.map_stride + p] : 0.0}; },
-          [&](int p, cplx u) {
-            d0[p] = u.x - s.re[lx(p)];
-            if (two) d0[a.map_stride + p] = u.y - s.im[lx(p)];
-          });
-    } else {
-      for (int p = threadIdx.x; p < n; p += TPB) {
-        d0[p] = s.re[lx(p)];
-        if (two) d0[a.map_stride + p] = s.im[lx(p)];
-      }
-    }
-  } else if (a.f_single) {
-    float2* dst = reinterpret_cast<float2*>(a.f) + off;
-    for (int p = threadIdx.x; p < n; p += TPB)
-      dst[p] = make_float2((float)s.re[lx(p)], herm ? 0.0f : (float)s.im[lx(p)]);
-  } else {
-    cplx* dst = reinterpret_cast<cplx*>(a.f) + off;
-    const cplx* u0 = a.sub_from ? reinterpret_cast<const cplx*>(a.sub_from) + off : nullptr;
-    batched_for<TPB, 8, cplx>(
-        n, [&](int p) { return u0 ? u0[p] : cplx{0.0, 0.0}; },
-        [&](int p, cplx u) {
-          const cplx v = {s.re[lx(p)], herm ? 0.0 : s.im[lx(p)]};
-          dst[p] = u0 ? csub(u, v) : v;
-        });
-  }
-}
-
-// ------------------------------------------------------------------ aliasing
-// R = G - A(Y) for one (ring, map), A = (ring FFT) . (ring iFFT) with the
-// FFTs cancelled: with m = q + j_m n (q = m mod n) and w = e^{i n phi0},
-//   A(Y)[m] = w_t n e^{-i m phi0} sum_{m' = q mod n} e^{i m' phi0} c(m')
-//           = w_t n w^{-j_m} T[q],   T[q] = sum_j w^j c(q + j n),
-// m' = q + j n over [-(L-1), L-1] (c(m') = conj c(-m') for Hermitian spectra).
-// On the supported grids n phi0 / pi is an integer, so w = +-1 (sgn).
-// Rings with n >= 2L - 1 have one m' per q: R = G - w_t n Y elementwise.
-// Otherwise thread t owns the residue q = t (mod n): with n >= TPB it sums
-// T[q] itself; with n < TPB the G = TPB / n threads of a residue split the j
-// (j = g, g + G, ... from the first) and meet in LDS in order of g.  Each
-// thread then writes the outputs of its residue (the same split over j).
-__device__ __forceinline__ cplx alias_term(const cplx* y, int m, int m_first, bool herm) {
-  if (herm && m < 0) {
-    const cplx t = y[-m - m_first];
-    return {t.x, -t.y};
-  }
-  return y[m - m_first];
-}
-
-// floor(a / n) by a multiply-high with mag = floor((2^32 - 1) / n) + 1: exact
-// for 0 <= a < 2^16 and 0 < n < 2^16 (the error a (n mag - 2^32) / 2^32 n stays
-// below 1/n), so one division per thread replaces one per residue
-struct FastDiv {
-  int n;
-  unsigned mag;
-  __device__ explicit FastDiv(int n_) : n(n_), mag(n_ > 1 ? 0xFFFFFFFFu / (unsigned)n_ + 1u : 0u) {}
-  __device__ __forceinline__ int floor(int a) const {
-    if (n == 1) return a;
-    return a >= 0 ? (int)__umulhi((unsigned)a, mag) : -(int)__umulhi((unsigned)(n - 1 - a), mag);
-  }
-};
-
-// DOT: instead of writing R, the workgroup adds up
-//   sum_m c_m Re(conj(Y[m]) A(Y)[m]),   c_m = 2 for m > 0 of Hermitian spectra, else 1,
-// and stores it in a.part[map * jobs + job]: summed over rings this is
-// <p, Lat_fwd(A(Lat_inv p))> for Y = Lat_inv(p) (the latitudinal transforms
-// are transposes of each other), the curvature a conjugate-gradient step needs
-// without projecting A(Y).  With a.alpha the written residual is
-// R = G - alpha[map] A(Y); with a.part in that mode the workgroup also stores
-// the sum of squares of the R it wrote (re^2 + im^2 over its columns).
-template <int TPB, bool DOT>
-__global__ void __launch_bounds__(TPB) ring_alias_kernel(RingAliasArgs a) {
-  __shared__ double part[2 * TPB];
-  const RingJob job = a.jobs[blockIdx.x];
-  const int n = job.nphi;
-  const int64_t off = (int64_t)blockIdx.y * a.map_stride + (int64_t)job.row * a.ncol;
-  const cplx* __restrict__ y = a.y + off;
-  const cplx* g = a.g + off;
-  cplx* r = a.r + off;
-  const double wn = job.weight * n * (a.alpha && !DOT ? a.alpha[blockIdx.y] : 1.0);
-  const int lo = -(a.L - 1), hi = a.L - 1;
-  const bool herm = a.herm != 0;
-  const int t = threadIdx.x;
-  double dsum = 0.0;
-  if (n > hi - lo) {
-    // no aliasing: the column's own m is the only term
-    if constexpr (DOT) {
-      batched_for<TPB, 8, cplx>(
-          a.ncol, [&](int col) { return y[col]; },
-          [&](int col, cplx yv) {
-            const int m = a.m_first + col;
-            if (m >= lo && m <= hi)
-              dsum += (herm && m > 0 ? 2.0 * wn : wn) * (yv.x * yv.x + yv.y * yv.y);
-          });
-    } else {
-      batched_for<TPB, 8, cplx>(
-          a.ncol, [&](int col) { return g[col]; },
-          [&](int col, cplx gv) {
-            const int m = a.m_first + col;
-            cplx v = {0.0, 0.0};
-            if (m >= lo && m <= hi) v = alias_term(y, m, a.m_first, herm);
-            const cplx rv = {gv.x - wn * v.x, gv.y - wn * v.y};
-            r[col] = rv;
-            dsum = fma(rv.x, rv.x, fma(rv.y, rv.y, dsum));
-          });
-      if (!a.part) return;
-    }
-  } else if (herm && a.m_first == 0 && n >= a.L) {
-    // Hermitian spectra stored for m in [0, L) on a ring with L <= n < 2L - 1:
-    // the only alias of m is m - n, whose coefficient is conj Y[n - m], so
-    // A(Y)[m] = w n (Y[m] + w^{-1} conj Y[n - m]) for m >= n - L + 1, else w n Y[m]
-    const int e = (int)rint(n * job.phi0_over_pi);
-    const double sgn = (a.apply_phase && (e & 1)) ? -1.0 : 1.0;
-    const int m_pair = n - a.L + 1;
-    for (int m = t; m < a.ncol; m += TPB) {
-      const cplx yv = y[m];
-      cplx av = yv;
-      if (m >= m_pair) {
-        const cplx yp = y[n - m];
-        av = {fma(sgn, yp.x, av.x), fma(-sgn, yp.y, av.y)};
-      }
-      if constexpr (DOT) {
-        dsum += (m > 0 ? 2.0 * wn : wn) * (yv.x * av.x + yv.y * av.y);
-      } else {
-        const cplx gv = g[m];
-        const cplx rv = {gv.x - wn * av.x, gv.y - wn * av.y};
-        r[m] = rv;
-        dsum = fma(rv.x, rv.x, fma(rv.y, rv.y, dsum));
-      }
-    }
-    if (!DOT && !a.part) return;
-  } else {
-    const int e = (int)rint(n * job.phi0_over_pi);
-    const double sgn = (a.apply_phase && (e & 1)) ? -1.0 : 1.0;
-    // the division's operands: |q - lo|, |hi - q|, |q - m_first| and
-    // |m_last - q| are below n + 2L (the host keeps n + 2L < 2^16)
-    const FastDiv dv(n);
-    const int G = n >= TPB ? 1 : TPB / n;
-    const int nq = n >= TPB ? (n + TPB - 1) / TPB : 1;  // residues per thread
-    const int gi = n >= TPB ? 0 : t / n;
-    const bool active = gi < G;
-    const int m_last = a.m_first + a.ncol - 1;
-    for (int qi = 0; qi < nq; ++qi) {
-      const int q = n >= TPB ? t + qi * TPB : t % n;
-      const bool own = active && q < n;
-      // T[q]: j from j0 = ceil((lo - q) / n) to floor((hi - q) / n), this
-      // thread's j = j0 + gi + k G
-      cplx acc = {0.0, 0.0};
-      int j0 = 0;
-      if (own) {
-        j0 = -dv.floor(q - lo);
-        const int j1 = dv.floor(hi - q);
-        const int cnt = j1 - j0 + 1;
-        for (int k0 = gi; k0 < cnt; k0 += 4 * G) {
-          cplx v[4];
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            const int k = k0 + u * G;
-            v[u] = k < cnt ? alias_term(y, q + (j0 + k) * n, a.m_first, herm) : cplx{0.0, 0.0};
-          }
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            const int k = k0 + u * G;
-            const double sj = ((j0 + k) & 1) && sgn < 0 ? -1.0 : 1.0;
-            acc = {fma(sj, v[u].x, acc.x), fma(sj, v[u].y, acc.y)};
-          }
-        }
-      }
-      if (G > 1) {
-        if (own) {
-          part[2 * t] = acc.x;
-          part[2 * t + 1] = acc.y;
-        }
-        __syncthreads();
-        cplx tot = {0.0, 0.0};
-        if (own)
-          for (int gg = 0; gg < G; ++gg)
-            tot = cadd(tot, cplx{part[2 * (gg * n + q)], part[2 * (gg * n + q) + 1]});
-        __syncthreads();
-        acc = tot;
-      }
-      if (!own) continue;
-      // outputs m = q + j n in [m_first, m_last], this thread's j = jo + gi + k G
-      const int jo = -dv.floor(q - a.m_first);
-      const int cnt = dv.floor(m_last - q) - jo + 1;
-      const cplx* src = DOT ? y : g;
-      for (int k0 = gi; k0 < cnt; k0 += 4 * G) {
-        cplx gv[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int k = k0 + u * G;
-          gv[u] = k < cnt ? src[q + (jo + k) * n - a.m_first] : cplx{0.0, 0.0};
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int k = k0 + u * G;
-          if (k < cnt) {
-            const double c = (((jo + k) & 1) && sgn < 0 ? -wn : wn);
-            if constexpr (DOT) {
-              const int m = q + (jo + k) * n;
-              dsum += (herm && m > 0 ? 2.0 * c : c) * (gv[u].x * acc.x + gv[u].y * acc.y);
-            } else {
-              const cplx rv = {gv[u].x - c * acc.x, gv[u].y - c * acc.y};
-              r[q + (jo + k) * n - a.m_first] = rv;
-              dsum = fma(rv.x, rv.x, fma(rv.y, rv.y, dsum));
-            }
-          }
-        }
-      }
-    }
-  }
-  // residue-owned columns: the written values of R in the no-alias branch
-  // when a.part is set (write mode) fall through to the same reduction
-  if (DOT || a.part) {
-    // fixed-order workgroup sum: waves by shuffles, then wave 0 over the waves
-    for (int o = 32; o > 0; o >>= 1) dsum += __shfl_xor(dsum, o);
-    __syncthreads();
-    if ((t & 63) == 0) part[t >> 6] = dsum;
-    __syncthreads();
-    if (t == 0) {
-      double tot = 0.0;
-      for (int w = 0; w < TPB / 64; ++w) tot += part[w];
-      a.part[(int64_t)blockIdx.y * gridDim.x + blockIdx.x] = tot;
-    }
-  }
-}
-
-// pq[b] = sum over the rings' partial sums in ring order; alpha[b] = num[b] / pq[b]
-__global__ void __launch_bounds__(256) ring_dot_final_kernel(const double* part, int njobs,
-                                                             const double* num, double* pq,
-                                                             double* alpha) {
-  __shared__ double red[4];
-  const int b = blockIdx.x;
-  double acc = 0.0;
-  for (int k = threadIdx.x; k < njobs; k += 256) acc += part[(int64_t)b * njobs + k];
-  for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const double tot = (red[0] + red[1]) + (red[2] + red[3]);
-    if (pq) pq[b] = tot;
-    if (alpha) alpha[b] = (num && tot != 0.0) ? num[b] / tot : 0.0;
-  }
-}
-
-// ------------------------------------------------------------------ aliasing, tiled
-// ring_alias_kernel's cases for real maps (Hermitian spectra stored for m in
-// [0, L)) on the tiled spectra (spec_row), per row block of 8 rows:
-//  * belt blocks (every row n >= 2L - 1, no alias: R = G - w n Y) by
-//    ring_alias_belt_kernel: kAliasSplit workgroups per block, lane 8 cg + r
-//    on row r and column group v = split NG + cg, so that a wave's access to
-//    8 columns of the 8 rows is one contiguous kilobyte;
-//  * the other blocks by ring_alias_polar_kernel: RW rows of the block per
-//    workgroup, their spectra staged in LDS by whole columns (RW 16 coalesced
-//    bytes each), then per row as in ring_alias_kernel:
-//      L <= n < 2L - 1: the one alias m - n of m >= n - L + 1, whose
-//        coefficient is conj Y[n - m]: A(Y)[m] = w n (Y[m] + sgn conj Y[n - m]);
-//      n < L: residue sums T[q] = sum_j s_j c(q + j n) over m' in
-//        [-(L-1), L-1] (c(m') = conj Y[-m'] for m' < 0, s_j = -1 for odd j
-//        when sgn < 0), then A(Y)[q + j n] = s_j w n T[q];  residues of rows
-//        with n below the lanes per row split their j over groups that meet
-//        in LDS in group order,
-//    A(Y) / (w n) written over the staged Y, and R = G - w n A written back
-//    by whole columns.
-// Every per-row sum runs in a fixed order, and each workgroup's partial sum
-// (dot or |R|^2) is reduced in a fixed order into part[map][block][slot]
-// (kAliasSlots slots per block; the unused ones are zeroed): deterministic.
-constexpr int kAliasSplit = 4;
-constexpr int kAliasSlots = 8;
-// polar workgroups: TPB threads staging up to LDSB bytes of spectra (8
-// columns per lane): 1024 threads and 128 KB (L <= 8192); the dot up to
-// L = 4096 as two workgroups of 512 threads and 64 KB per CU, so that one
-// stages while the other sums
-constexpr int kAliasPolarTpb = 1024;
-constexpr int kAliasPolarLds = 128 * 1024;
-constexpr int kAliasDotTpb = 512;
-constexpr int kAliasDotLds = 64 * 1024;
-
-// rows of a block per polar workgroup: the largest power of two <= 8 with
-// RW L 16 bytes within the LDS budget ldsb
-__host__ __device__ inline int alias_polar_rows(int L, int ldsb) {
-  int rw = kSpecBlock;
-  while (rw > 1 && (int64_t)rw * L * 16 > ldsb) rw >>= 1;
-  return rw;
-}
-
-// fixed-order workgroup sum of dsum into part[slot]; slot 0's workgroup
-// also zeroes the slots >= nslots
-template <int TPB>
-__device__ __forceinline__ void alias_block_sum(double dsum, double* red, double* part, int slot,
-                                                int nslots) {
-  const int t = threadIdx.x;
-  for (int o = 32; o > 0; o >>= 1) dsum += __shfl_xor(dsum, o);
-  __syncthreads();
-  if ((t & 63) == 0) red[t >> 6] = dsum;
-  __syncthreads();
-  if (t == 0) {
-    double tot = 0.0;
-    for (int w = 0; w < TPB / 64; ++w) tot += red[w];
-    part[slot] = tot;
-    if (slot == 0)
-      for (int k = nslots; k < kAliasSlots; ++k) part[k] = 0.0;
-  }
-}
-
-template <int TPB, bool DOT>
-__global__ void __launch_bounds__(TPB) ring_alias_belt_kernel(RingAliasTiledArgs a) {
-  constexpr int NG = TPB / kSpecBlock;  // column groups per workgroup
-  constexpr int NV = kAliasSplit * NG;  // column groups per row block
-  constexpr int U = 4;                  // loads in flight
-  __shared__ double red[TPB / 64];
-  const int t = threadIdx.x, r = t & 7, cg = t >> 3;
-  const int blk = a.belt_blocks[blockIdx.x], b = blockIdx.y, sp = blockIdx.z;
-  const int v = sp * NG + cg;
-  const int row = kSpecBlock * blk + r;
-  const RingJob job = a.rowjobs[row];
-  const int n = job.nphi;
-  const int L = a.L;
-  const int64_t tile = (int64_t)b * a.map_stride + (int64_t)blk * kSpecBlock * a.ncol;
-  const cplx* __restrict__ y = a.y + tile + r;  // column m at y[8 m]
-  cplx* rr = a.r + tile + r;
-  const cplx* g = a.g_tiled ? a.g + tile + r
-                            : a.g + (int64_t)b * a.map_stride + (int64_t)row * a.ncol;
-  const int gs = a.g_tiled ? kSpecBlock : 1;
-  const double wn = job.weight * n * (a.alpha && !DOT ? a.alpha[b] : 1.0);
-  double dsum = 0.0;
-  if (n > 0) {
-    for (int m0 = v; m0 < L; m0 += U * NV) {
-      cplx yv[U], gv[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int m = m0 + u * NV;
-        yv[u] = gv[u] = cplx{0.0, 0.0};
-        if (m < L) {
-          yv[u] = y[kSpecBlock * m];
-          if (!DOT) gv[u] = g[gs * m];
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int m = m0 + u * NV;
-        if (m >= L) continue;
-        if constexpr (DOT) {
-          dsum += (m > 0 ? 2.0 * wn : wn) * (yv[u].x * yv[u].x + yv[u].y * yv[u].y);
-        } else {
-          const cplx rv = {gv[u].x - wn * yv[u].x, gv[u].y - wn * yv[u].y};
-          rr[kSpecBlock * m] = rv;
-          dsum = fma(rv.x, rv.x, fma(rv.y, rv.y, dsum));
-        }
-      }
-    }
-  }
-  if (DOT || a.part)
-    alias_block_sum<TPB>(dsum, red,
-                         a.part + (int64_t)b * a.part_map_stride + a.belt_part_off +
-                             (int64_t)blockIdx.x * kAliasSlots,
-                         sp, kAliasSplit);
-}
-
-template <bool DOT, int TPB, int LDSB>
-__global__ void __launch_bounds__(TPB) ring_alias_polar_kernel(RingAliasTiledArgs a) {
-  constexpr int kAliasMaxCols = LDSB / 16 / TPB;  // staged columns per lane
+template <int WG>
+__global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(2)))
+ring_reg_fwd_kernel(RingFwdArgs a, RingSegs g, int paired) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
-  cplx* ys = reinterpret_cast<cplx*>(lds_raw);  // [column m][row of the workgroup]
-  __shared__ double xch[2 * TPB];                // residue groups' partial sums
-  __shared__ double red[TPB / 64];
-  const int L = a.L;
-  const int RW = alias_polar_rows(L, LDSB);
-  const int H = kSpecBlock / RW;                 // workgroups per block
-  // blockIdx.x -> (block, part z): the H parts of a block on one XCD
-  // (workgroups are dealt to the 8 XCDs round-robin), so that they read each
-  // 128-byte line of the block through that XCD's L2 at about the same time
-  const int i = blockIdx.x;
-  const int z = (i >> 3) % H;
-  const int bi = ((i >> 3) / H) * 8 + (i & 7);
-  if (bi >= a.n_polar) return;
-  const int blk = a.polar_blocks[bi], b = blockIdx.y;
-  const int t = threadIdx.x;
-  const int r0 = z * RW;
-  const int64_t tile = (int64_t)b * a.map_stride + (int64_t)blk * kSpecBlock * a.ncol;
-  const int ntot = L * RW;  // <= kAliasMaxCols TPB
-  // stage Y: element (m, q) of the workgroup's rows at ys[m RW + q]; every
-  // load of the thread in flight before the first LDS store (q = t % RW is
-  // the thread's own: TPB is a multiple of RW)
-  const int qt = t % RW;
-  {
-    cplx v[kAliasMaxCols];
-#pragma unroll
-    for (int k = 0; k < kAliasMaxCols; ++k) {
-      const int idx = t + k * TPB;
-      v[k] = idx < ntot ? a.y[tile + (int64_t)(idx / RW) * kSpecBlock + r0 + qt]
-                        : cplx{0.0, 0.0};
-    }
-#pragma unroll
-    for (int k = 0; k < kAliasMaxCols; ++k) {
-      const int idx = t + k * TPB;
-      if (idx < ntot) ys[idx] = v[k];
-    }
-  }
-  __syncthreads();
-
-  const int LPR = TPB / RW;                      // lanes per row
-  const int rq = t / LPR, li = t - rq * LPR;
-  const int row = kSpecBlock * blk + r0 + rq;
-  const RingJob job = a.rowjobs[row];
-  const int n = job.nphi;
-  const double wn = job.weight * n * (a.alpha && !DOT ? a.alpha[b] : 1.0);
-  const int e = (int)rint(n * job.phi0_over_pi);
-  const double sgn = (a.apply_phase && (e & 1)) ? -1.0 : 1.0;
-  auto Y = [&](int m) { return ys[m * RW + rq]; };
-  const int kind = n == 0 ? 0 : n > 2 * L - 2 ? 1 : n >= L ? 2 : 3;  // none, no alias, pair, fold
-  double dsum = 0.0;
-
-  // pair rows: A(Y) / (w n) of columns li + k LPR, fold rows: T of residues
-  // q = li + k LPR (n >= LPR) or of the one residue of a split, in registers
-  cplx av[kAliasMaxCols];
-  cplx* tq = av;
-  const bool splitf = kind == 3 && n < LPR;
-  const int G = splitf ? LPR / n : 1;
-  const int gi = splitf ? li / n : 0;
-  const int qs = splitf ? li % n : li;
-  const bool owns = kind == 3 && gi < G;
-  FastDiv dv(kind == 3 ? n : 1);
-#pragma unroll
-  for (int k = 0; k < kAliasMaxCols; ++k) av[k] = cplx{0.0, 0.0};
-  if (kind == 2) {
-    const int m_pair = n - L + 1;
-#pragma unroll
-    for (int k = 0; k < kAliasMaxCols; ++k) {
-      const int m = li + k * LPR;
-      if (m < L) {
-        const cplx y0 = Y(m);
-        cplx v = y0;
-        if (m >= m_pair) {
-          const cplx yp = Y(n - m);
-          v = {fma(sgn, yp.x, v.x), fma(-sgn, yp.y, v.y)};
-        }
-        av[k] = v;
-        if constexpr (DOT) dsum += (m > 0 ? 2.0 * wn : wn) * (y0.x * v.x + y0.y * v.y);
-      }
-    }
-  } else if (owns) {
-#pragma unroll
-    for (int k = 0; k < kAliasMaxCols; ++k) {
-      const int q = qs + k * (splitf ? 0 : LPR);
-      if ((splitf && k > 0) || q >= n) continue;
-      const int j0 = -dv.floor(q + L - 1);
-      const int cnt = dv.floor(L - 1 - q) - j0 + 1;
-      cplx acc = {0.0, 0.0};
-      for (int kk = gi; kk < cnt; kk += G) {
-        const int mp = q + (j0 + kk) * n;
-        cplx v = Y(mp < 0 ? -mp : mp);
-        if (mp < 0) v.y = -v.y;
-        const double sj = ((j0 + kk) & 1) && sgn < 0 ? -1.0 : 1.0;
-        acc = {fma(sj, v.x, acc.x), fma(sj, v.y, acc.y)};
-      }
-      tq[k] = acc;
-    }
-  }
-  // split residues: the groups' partial sums meet in LDS in group order
-  xch[2 * t] = tq[0].x;
-  xch[2 * t + 1] = tq[0].y;
-  __syncthreads();
-  if (splitf && owns) {
-    cplx T = {0.0, 0.0};
-    for (int gg = 0; gg < G; ++gg) {
-      const int src = rq * LPR + gg * n + qs;
-      T = {T.x + xch[2 * src], T.y + xch[2 * src + 1]};
-    }
-    tq[0] = T;
-  }
-  if constexpr (DOT) {
-    // a fold row's dot from its residues alone: the sum over m >= 0 of
-    // c_m Re(conj Y[m] A[m]) is the sum over all m' in (-L, L) of
-    // conj(c(m')) s_j T[q] (A(-m) = conj A(m) for a real ring), i.e.
-    // sum_q T[q] conj(sum_j s_j c(q + j n)) = sum_q |T[q]|^2
-    if (owns && (!splitf || gi == 0)) {
-#pragma unroll
-      for (int k = 0; k < kAliasMaxCols; ++k) {
-        const int q = qs + k * (splitf ? 0 : LPR);
-        if ((splitf && k > 0) || q >= n) continue;
-        dsum = fma(wn, tq[k].x * tq[k].x + tq[k].y * tq[k].y, dsum);
-      }
-    }
-  } else {
-    __syncthreads();  // every read of the staged Y is done
-  }
-
-  // columns of the row's outputs: A / (w n) over the staged Y (write mode),
-  // or the dot's terms c_m w n Re(conj Y[m] A[m]) (dot mode)
-  auto out = [&](int m, cplx A) {
-    if constexpr (DOT) {
-      const cplx yv = Y(m);
-      dsum += (m > 0 ? 2.0 * wn : wn) * (yv.x * A.x + yv.y * A.y);
-    } else {
-      ys[m * RW + rq] = A;
-    }
-  };
-  if (kind == 1) {
-    if constexpr (DOT)
-      for (int m = li; m < L; m += LPR) out(m, Y(m));
-  } else if (DOT) {
-    // pair and fold rows: summed above
-  } else if (kind == 2) {
-#pragma unroll
-    for (int k = 0; k < kAliasMaxCols; ++k) {
-      const int m = li + k * LPR;
-      if (m < L) out(m, av[k]);
-    }
-  } else if (owns) {
-#pragma unroll
-    for (int k = 0; k < kAliasMaxCols; ++k) {
-      const int q = qs + k * (splitf ? 0 : LPR);
-      if ((splitf && k > 0) || q >= n) continue;
-      const int cnt = dv.floor(L - 1 - q) + 1;
-      for (int kk = gi; kk < cnt; kk += G) {
-        const double sj = ((kk & 1) && sgn < 0) ? -1.0 : 1.0;
-        out(q + kk * n, cplx{sj * tq[k].x, sj * tq[k].y});
-      }
-    }
-  }
-
-  if constexpr (!DOT) {
-    __syncthreads();
-    // R = G - w n A by whole columns (this thread: row r0 + qt), the G loads
-    // in flight together
-    const int rw_row = kSpecBlock * blk + r0 + qt;
-    const RingJob jq = a.rowjobs[rw_row];
-    if (jq.nphi > 0) {
-      const double c = jq.weight * jq.nphi * (a.alpha ? a.alpha[b] : 1.0);
-      cplx gv[kAliasMaxCols];
-#pragma unroll
-      for (int k = 0; k < kAliasMaxCols; ++k) {
-        const int idx = t + k * TPB;
-        const int m = idx / RW;
-        gv[k] = idx >= ntot ? cplx{0.0, 0.0}
-                : a.g_tiled ? a.g[tile + (int64_t)m * kSpecBlock + r0 + qt]
-                            : a.g[(int64_t)b * a.map_stride + (int64_t)rw_row * a.ncol + m];
-      }
-#pragma unroll
-      for (int k = 0; k < kAliasMaxCols; ++k) {
-        const int idx = t + k * TPB;
-        if (idx >= ntot) continue;
-        const cplx A = ys[idx];
-        const cplx rv = {gv[k].x - c * A.x, gv[k].y - c * A.y};
-        a.r[tile + (int64_t)(idx / RW) * kSpecBlock + r0 + qt] = rv;
-        dsum = fma(rv.x, rv.x, fma(rv.y, rv.y, dsum));
-      }
-    }
-  }
-  if (DOT || a.part)
-    alias_block_sum<TPB>(dsum, red,
-                         a.part + (int64_t)b * a.part_map_stride + a.polar_part_off +
-                             (int64_t)bi * kAliasSlots,
-                         z, H);
+  ring_body<WG, 0>(a, seg_of_block(g), paired, lds_raw);
+}
+template <int WG>
+__global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(2)))
+ring_reg_inv_kernel(RingInvArgs a, RingSegs g, int paired) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
+  ring_body<WG, 1>(a, seg_of_block(g), paired, lds_raw);
 }
 
 // ------------------------------------------------------------------ launchers
 namespace {
 
-constexpr int kTpbPow2 = 512;
-constexpr int kTpbSmooth = 256;
-constexpr int kTpbBlue = 512;
-constexpr int kTpbAlias = 256;
-constexpr int kTabBytes = kTabCplx * sizeof(cplx);
-
-// tables + data region (2 lx_len(N) doubles, at least 2 TPB for the fold's partials)
-size_t ring_lds_bytes(int N, int tpb) {
-  const int w = lx_len(N);
-  const size_t nd = 2 * (size_t)(w > tpb ? w : tpb);
-  return nd * sizeof(double) + kTabBytes;
+// Whether every residue of an n-point ring has at most one column.
+bool ring_direct(const RingFwdArgs& a, int n, int paired) {
+  if (a.out_single || a.zero_neg_2L) return false;
+  if (paired) return a.m_first == 0 && a.ncol <= n / 2;
+  return a.ncol <= n && a.m_first <= 0 && -a.m_first < n;
 }
 
-bool fwd_paired(const RingFwdArgs& a) { return !a.f_complex || a.real_only_all; }
-bool inv_paired(const RingInvArgs& a) { return a.herm_mode == 1 && !a.f_complex; }
+int shape_lds(int logm) { return (1 << logm) + (logm <= 9 ? (1 << logm) / 8 + 32 : 0); }
+int seg_threads(const RingSeg& s) { return 1 << ((s.body & (kPow2Body - 1)) - 4); }
 
-}  // namespace
-
-hipError_t launch_ring_fft_forward(const RingFwdArgs& a0, const JobSet& js, int batch,
-                                   hipStream_t s) {
-  if (batch == 0 || js.n_pow2 + js.n_smooth + js.n_blue == 0) return hipSuccess;
-  RingFwdArgs a = a0;
-  a.jobs = js.jobs;
-  a.batch = batch;
-  const int paired = fwd_paired(a) ? 1 : 0;
-  const unsigned gy = paired ? (unsigned)((batch + 1) / 2) : (unsigned)batch;
-  if (js.n_pow2)
-    hipLaunchKernelGGL((ring_fwd_kernel<kTpbPow2, kMaxRingLen, kPow2>), dim3(js.n_pow2, gy),
-                       dim3(kTpbPow2), ring_lds_bytes(js.max_pow2, kTpbPow2), s, a, 0, paired);
-  if (js.n_smooth)
-    hipLaunchKernelGGL((ring_fwd_kernel<kTpbSmooth, kMaxRingLen, kSmooth>),
-                       dim3(js.n_smooth, gy), dim3(kTpbSmooth), ring_lds_bytes(js.max_smooth, kTpbSmooth), s,
-                       a, js.n_pow2, paired);
-  // Bluestein: the long convolutions (one workgroup per CU), then the short
-  // ones with their own, smaller LDS size
-  const int b0 = js.n_pow2 + js.n_smooth, nshort = js.n_blue - js.n_blue_long;
-  if (js.n_blue_long)
-    hipLaunchKernelGGL((ring_fwd_kernel<kTpbBlue, kMaxConvLen, kBlue>), dim3(js.n_blue_long, gy),
-                       dim3(kTpbBlue), ring_lds_bytes(js.max_conv, kTpbBlue), s, a, b0, paired);
-  if (nshort)
-    hipLaunchKernelGGL((ring_fwd_kernel<kTpbBlue, kMaxConvLen, kBlue>), dim3(nshort, gy),
-                       dim3(kTpbBlue), ring_lds_bytes(js.max_conv_short, kTpbBlue), s, a,
-                       b0 + js.n_blue_long, paired);
-  return hipGetLastError();
-}
-
-hipError_t launch_ring_fft_inverse(const RingInvArgs& a0, const JobSet& js, int batch,
-                                   hipStream_t s) {
-  if (batch == 0 || js.n_pow2 + js.n_smooth + js.n_blue == 0) return hipSuccess;
-  RingInvArgs a = a0;
-  a.jobs = js.jobs;
-  a.batch = batch;
-  const int paired = inv_paired(a) ? 1 : 0;
-  const unsigned gy = paired ? (unsigned)((batch + 1) / 2) : (unsigned)batch;
-  if (js.n_pow2)
-    hipLaunchKernelGGL((ring_inv_kernel<kTpbPow2, kMaxRingLen, kPow2>), dim3(js.n_pow2, gy),
-                       dim3(kTpbPow2), ring_lds_bytes(js.max_pow2, kTpbPow2), s, a, 0, paired);
-  if (js.n_smooth)
-    hipLaunchKernelGGL((ring_inv_kernel<kTpbSmooth, kMaxRingLen, kSmooth>),
-                       dim3(js.n_smooth, gy), dim3(kTpbSmooth), ring_lds_bytes(js.max_smooth, kTpbSmooth), s,
-                       a, js.n_pow2, paired);
-  const int b0 = js.n_pow2 + js.n_smooth, nshort = js.n_blue - js.n_blue_long;
-  if (js.n_blue_long)
-    hipLaunchKernelGGL((ring_inv_kernel<kTpbBlue, kMaxConvLen, kBlue>), dim3(js.n_blue_long, gy),
-                       dim3(kTpbBlue), ring_lds_bytes(js.max_conv, kTpbBlue), s, a, b0, paired);
-  if (nshort)
-    hipLaunchKernelGGL((ring_inv_kernel<kTpbBlue, kMaxConvLen, kBlue>), dim3(nshort, gy),
-                       dim3(kTpbBlue), ring_lds_bytes(js.max_conv_short, kTpbBlue), s, a,
-                       b0 + js.n_blue_long, paired);
-  return hipGetLastError();
-}
-
-hipError_t launch_ring_alias(const RingAliasArgs& a, const JobSet& js, int batch, hipStream_t s) {
-  const int njobs = js.n_pow2 + js.n_smooth + js.n_blue;
-  if (batch == 0 || njobs == 0) return hipSuccess;
-  RingAliasArgs b = a;
-  b.jobs = js.jobs;
-  hipLaunchKernelGGL((ring_alias_kernel<kTpbAlias, false>), dim3(njobs, batch), dim3(kTpbAlias), 0,
-                     s, b);
-  return hipGetLastError();
-}
-
-hipError_t launch_ring_alias_sumsq(const RingAliasArgs& a, const JobSet& js, int batch,
-                                   double* part, double* sumsq, hipStream_t s) {
-  const int njobs = ring_dot_jobs(js);
-  if (batch == 0 || njobs == 0) return hipSuccess;
-  RingAliasArgs b = a;
-  b.jobs = js.jobs;
-  b.part = part;
-  hipLaunchKernelGGL((ring_alias_kernel<kTpbAlias, false>), dim3(njobs, batch), dim3(kTpbAlias), 0,
-                     s, b);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(ring_dot_final_kernel, dim3(batch), dim3(256), 0, s, part, njobs, nullptr,
-                     sumsq, nullptr);
-  return hipGetLastError();
-}
-
-int ring_dot_jobs(const JobSet& js) { return js.n_pow2 + js.n_smooth + js.n_blue; }
-int ring_dot_tiled_parts(int nblocks) { return nblocks * kAliasSlots; }
-namespace {
-// both tiled alias kernels over their blocks (part: null, or the per-block slots)
-hipError_t launch_alias_tiled_pair(const RingAliasTiledArgs& a, int batch, bool dot,
-                                   hipStream_t s) {
-  if (a.n_belt > 0) {
-    const dim3 grid(a.n_belt, batch, kAliasSplit);
-    if (dot)
-      hipLaunchKernelGGL((ring_alias_belt_kernel<kTpbAlias, true>), grid, dim3(kTpbAlias), 0, s,
-                         a);
-    else
-      hipLaunchKernelGGL((ring_alias_belt_kernel<kTpbAlias, false>), grid, dim3(kTpbAlias), 0,
-                         s, a);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
+// The segments of a job set, longest convolutions first.
+RingSegs ring_segs(const JobSet& js) {
+  RingSegs g{};
+  int j0 = js.n_pow2;
+  for (int c = kBlueClasses - 1; c >= 0; --c) {
+    if (!js.blue[c]) continue;
+    g.s[g.n++] = RingSeg{c + kBlueLogMin, j0, js.blue[c], 0, 0, shape_lds(c + kBlueLogMin)};
+    j0 += js.blue[c];
   }
-  if (a.n_polar > 0) {
-    if ((int64_t)a.L * 16 > kAliasPolarLds) return hipErrorInvalidValue;
-    const bool small = dot && (int64_t)a.L * 16 <= kAliasDotLds;
-    const int RW = alias_polar_rows(a.L, small ? kAliasDotLds : kAliasPolarLds);
-    const int H = kSpecBlock / RW;
-    const dim3 grid((unsigned)((a.n_polar + 7) / 8 * 8 * H), batch);
-    const size_t lds = (size_t)RW * a.L * sizeof(cplx);
-    constexpr int T = kAliasPolarTpb, TD = kAliasDotTpb;
-    constexpr int B = kAliasPolarLds, BD = kAliasDotLds;
-    if (small)
-      hipLaunchKernelGGL((ring_alias_polar_kernel<true, TD, BD>), grid, dim3(TD), lds, s, a);
-    else if (dot)
-      hipLaunchKernelGGL((ring_alias_polar_kernel<true, T, B>), grid, dim3(T), lds, s, a);
-    else
-      hipLaunchKernelGGL((ring_alias_polar_kernel<false, T, B>), grid, dim3(T), lds, s, a);
-    const hipError_t e = hipGetLastError();
+  if (js.n_pow2)
+    g.s[g.n++] = RingSeg{kPow2Body + js.log_pow2, 0, js.n_pow2, 0, 0, 1 << js.log_pow2};
+  return g;
+}
+
+// Launches segments [i0, i1) together at the workgroup size of the largest.
+template <int DIR, typename Args>
+hipError_t launch_segs(const Args& a, const RingSegs& all, int i0, int i1, unsigned gy, int paired,
+                       hipStream_t s) {
+  RingSegs g{};
+  int wg = 64, lds = 0, blocks = 0;
+  for (int i = i0; i < i1; ++i) wg = std::max(wg, seg_threads(all.s[i]));
+  for (int i = i0; i < i1; ++i) {
+    RingSeg q = all.s[i];
+    const int rings = wg / seg_threads(q);
+    q.block0 = blocks;
+    blocks += (q.count + rings - 1) / rings;
+    lds = std::max(lds, rings * q.lds_ring * (int)sizeof(cplx));
+    g.s[g.n++] = q;
+  }
+  const dim3 grid(blocks, gy);
+#define S2H_LAUNCH(WG)                                                                     \
+  if constexpr (DIR == 0)                                                                  \
+    hipLaunchKernelGGL((ring_reg_fwd_kernel<WG>), grid, dim3(WG), lds, s, a, g, paired);   \
+  else                                                                                     \
+    hipLaunchKernelGGL((ring_reg_inv_kernel<WG>), grid, dim3(WG), lds, s, a, g, paired);
+  switch (wg) {
+    case 64: S2H_LAUNCH(64) break;
+    case 128: S2H_LAUNCH(128) break;
+    case 256: S2H_LAUNCH(256) break;
+    default: S2H_LAUNCH(512) break;
+  }
+#undef S2H_LAUNCH
+  return hipGetLastError();
+}
+
+// One launch for a whole ragged grid while it has at most kMergeBlocks
+// workgroups, else one per segment (each at its own workgroup size).  Together
+// against one launch per segment: nside 512, one map 44 against 75 us, four
+// maps 90 against 129, nside 1024, 16 maps (25 600 workgroups) 1434 against 1330.
+constexpr int kMergeBlocks = 16384;
+template <int DIR, typename Args>
+hipError_t launch_rings(const Args& a, const RingSegs& g, unsigned gy, int paired, hipStream_t s) {
+  int wg = 64, narrow = 512;
+  int64_t threads = 0;
+  for (int i = 0; i < g.n; ++i) {
+    wg = std::max(wg, seg_threads(g.s[i]));
+    narrow = std::min(narrow, seg_threads(g.s[i]));
+    threads += (int64_t)g.s[i].count * seg_threads(g.s[i]);
+  }
+  int lds = 0;
+  for (int i = 0; i < g.n; ++i)
+    lds = std::max(lds, wg / seg_threads(g.s[i]) * g.s[i].lds_ring * (int)sizeof(cplx));
+  const bool together = threads * gy <= (int64_t)kMergeBlocks * wg &&
+                        narrow * (wg == 64 ? 16 : 8) >= wg && lds <= kRingLdsMax;
+  if (together) return launch_segs<DIR>(a, g, 0, g.n, gy, paired, s);
+  for (int i = 0; i < g.n; ++i) {
+    const hipError_t e = launch_segs<DIR>(a, g, i, i + 1, gy, paired, s);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
 }
 
-// every row block's slots, polar blocks first
-void full_part_layout(RingAliasTiledArgs& b) {
-  b.part_map_stride = (int64_t)b.nblocks * kAliasSlots;
-  b.polar_part_off = 0;
-  b.belt_part_off = b.n_polar * kAliasSlots;
-}
+// real pairs: two maps share a complex transform
+bool fwd_paired(const RingFwdArgs& a) { return !a.f_complex || a.real_only_all; }
+bool inv_paired(const RingInvArgs& a) { return a.herm_mode == 1; }
+unsigned grid_y(int batch, int paired) { return (unsigned)(paired ? (batch + 1) / 2 : batch); }
+
 }  // namespace
 
-hipError_t launch_ring_alias_tiled(const RingAliasTiledArgs& a, int batch, hipStream_t s) {
-  if (batch == 0 || a.nblocks == 0) return hipSuccess;
-  RingAliasTiledArgs b = a;
-  b.part = nullptr;
-  return launch_alias_tiled_pair(b, batch, false, s);
+hipError_t launch_ring_fft_forward(const RingFwdArgs& a0, const JobSet& js, int batch,
+                                   hipStream_t s) {
+  if (batch == 0 || js.n_pow2 + js.n_blue == 0) return hipSuccess;
+  RingFwdArgs a = a0;
+  a.jobs = js.jobs;
+  a.batch = batch;
+  const int paired = fwd_paired(a) ? 1 : 0;
+  RingSegs g = ring_segs(js);
+  for (int i = 0; i < g.n; ++i) {
+    RingSeg& q = g.s[i];
+    if (q.body >= kPow2Body) {
+      q.direct = ring_direct(a, 1 << js.log_pow2, paired);
+      if (!q.direct && paired) q.lds_ring *= 2;  // the residues of both maps
+    } else {
+      q.direct = !paired && !a.apply_phase && ring_direct(a, js.min_blue, 0);
+    }
+  }
+  return launch_rings<0>(a, g, grid_y(batch, paired), paired, s);
 }
 
-hipError_t launch_ring_alias_tiled_sumsq(const RingAliasTiledArgs& a, int batch, double* part,
-                                         double* sumsq, hipStream_t s) {
-  if (batch == 0 || a.nblocks == 0) return hipSuccess;
-  RingAliasTiledArgs b = a;
-  b.part = part;
-  full_part_layout(b);
-  hipError_t e = launch_alias_tiled_pair(b, batch, false, s);
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(ring_dot_final_kernel, dim3(batch), dim3(256), 0, s, part,
-                     a.nblocks * kAliasSlots, nullptr, sumsq, nullptr);
-  return hipGetLastError();
-}
-
-hipError_t launch_ring_dot_tiled(const RingAliasTiledArgs& a, int batch, double* part,
-                                 const double* num, double* pq, double* alpha, hipStream_t s) {
-  if (batch == 0 || a.nblocks == 0) return hipSuccess;
-  RingAliasTiledArgs b = a;
-  b.part = part;
-  b.alpha = nullptr;
-  full_part_layout(b);
-  hipError_t e = launch_alias_tiled_pair(b, batch, true, s);
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(ring_dot_final_kernel, dim3(batch), dim3(256), 0, s, part,
-                     a.nblocks * kAliasSlots, num, pq, alpha);
-  return hipGetLastError();
-}
-
-hipError_t launch_ring_dot_tiled_polar(const RingAliasTiledArgs& a, int batch, double* part,
-                                       int n_head, const double* num, double* pq, double* alpha,
-                                       hipStream_t s) {
-  if (batch == 0) return hipSuccess;
-  RingAliasTiledArgs b = a;
-  b.part = part;
-  b.alpha = nullptr;
-  b.n_belt = 0;
-  b.part_map_stride = n_head + (int64_t)b.n_polar * kAliasSlots;
-  b.polar_part_off = n_head;
-  b.belt_part_off = 0;
-  hipError_t e = launch_alias_tiled_pair(b, batch, true, s);
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(ring_dot_final_kernel, dim3(batch), dim3(256), 0, s, part,
-                     (int)b.part_map_stride, num, pq, alpha);
-  return hipGetLastError();
-}
-
-hipError_t launch_ring_dot(const RingAliasArgs& a, const JobSet& js, int batch, double* part,
-                           const double* num, double* pq, double* alpha, hipStream_t s) {
-  const int njobs = ring_dot_jobs(js);
-  if (batch == 0 || njobs == 0) return hipSuccess;
-  RingAliasArgs b = a;
-  b.jobs = js.jobs;
-  b.part = part;
-  b.alpha = nullptr;
-  hipLaunchKernelGGL((ring_alias_kernel<kTpbAlias, true>), dim3(njobs, batch), dim3(kTpbAlias), 0,
-                     s, b);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(ring_dot_final_kernel, dim3(batch), dim3(256), 0, s, part, njobs, num, pq,
-                     alpha);
-  return hipGetLastError();
+hipError_t launch_ring_fft_inverse(const RingInvArgs& a0, const JobSet& js, int batch,
+                                   hipStream_t s) {
+  if (batch == 0 || js.n_pow2 + js.n_blue == 0) return hipSuccess;
+  RingInvArgs a = a0;
+  a.jobs = js.jobs;
+  a.batch = batch;
+  const int paired = inv_paired(a) ? 1 : 0;
+  return launch_rings<1>(a, ring_segs(js), grid_y(batch, paired), paired, s);
 }
 
 hipError_t allow_large_lds_rings() {
-  const int bytes = (int)ring_lds_bytes(kMaxConvLen, kTpbBlue);
-  const void* fns[] = {(const void*)ring_fwd_kernel<kTpbPow2, kMaxRingLen, kPow2>,
-                       (const void*)ring_fwd_kernel<kTpbSmooth, kMaxRingLen, kSmooth>,
-                       (const void*)ring_fwd_kernel<kTpbBlue, kMaxConvLen, kBlue>,
-                       (const void*)ring_inv_kernel<kTpbPow2, kMaxRingLen, kPow2>,
-                       (const void*)ring_inv_kernel<kTpbSmooth, kMaxRingLen, kSmooth>,
-                       (const void*)ring_inv_kernel<kTpbBlue, kMaxConvLen, kBlue>};
+  const int bytes = kRingLdsMax;
+  const void* fns[] = {(const void*)ring_reg_fwd_kernel<64>,  (const void*)ring_reg_fwd_kernel<128>,
+                       (const void*)ring_reg_fwd_kernel<256>, (const void*)ring_reg_fwd_kernel<512>,
+                       (const void*)ring_reg_inv_kernel<64>,  (const void*)ring_reg_inv_kernel<128>,
+                       (const void*)ring_reg_inv_kernel<256>, (const void*)ring_reg_inv_kernel<512>};
   for (const void* f : fns) {
     const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    if (e != hipSuccess) return e;
-  }
-  constexpr int T = kAliasPolarTpb, TD = kAliasDotTpb;
-  constexpr int B = kAliasPolarLds, BD = kAliasDotLds;
-  const void* alias[] = {(const void*)ring_alias_polar_kernel<true, T, B>,
-                         (const void*)ring_alias_polar_kernel<false, T, B>,
-                         (const void*)ring_alias_polar_kernel<true, TD, BD>};
-  const int lds[] = {B, B, BD};
-  for (int i = 0; i < 3; ++i) {
-    const hipError_t e =
-        hipFuncSetAttribute(alias[i], hipFuncAttributeMaxDynamicSharedMemorySize, lds[i]);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
