@@ -28,7 +28,6 @@ LatArgs lat_args(const s2h_plan* p, bool forward, int batch) {
   a.rings = forward ? p->fwd_rings : p->inv_rings;
   a.nrings = forward ? p->n_fwd_rings : p->n_inv_rings;
   a.mstart = forward ? p->fwd_mstart : p->inv_mstart;
-  a.coef = forward ? p->fwd_coef : p->inv_coef;
   a.ucoef = forward ? p->fwd_ucoef : p->inv_ucoef;
   a.L = p->d.L;
   a.m_lo = p->m_lo;
@@ -37,7 +36,21 @@ LatArgs lat_args(const s2h_plan* p, bool forward, int batch) {
   a.batch = batch;
   a.flm_map_stride = flm_stride(p);
   a.groups = 1;
+  a.pos_scale = 1.0;
   return a;
+}
+
+// Pole rows of a VALU latitudinal launch; lmin_spin: the sums start at |spin|.
+LatPole lat_pole(const s2h_plan* p, bool forward, bool lmin_spin, const PlaneSet* ps) {
+  LatPole q;
+  q.south = forward ? p->fwd_row_south : p->inv_row_south;
+  q.north = forward ? p->fwd_row_north : p->inv_row_north;
+  q.spin = ps ? ps->spin0 : p->d.spin;
+  q.spin_step = ps ? ps->spin_step : 0;
+  q.lmin = p->d.L_lower;
+  q.lmin_spin = lmin_spin ? 1 : 0;
+  q.norm = forward ? p->fwd_norm : p->inv_norm;
+  return q;
 }
 
 // Optional kernel timing: HIP events recorded on the launch stream around
@@ -225,11 +238,14 @@ int lat_forward_stage(const s2h_plan* p, const cplx* ftm, void* flm, int batch, 
   const bool poles = p->fwd_row_south >= 0 || p->fwd_row_north >= 0;
   // the FP64 matrix-core projection (one workgroup per m) and the BF16 ones
   // with one ring group per m write every entry of their m columns
-  const bool mfma64 = !ps && !bf16 && !mixed && batch >= kMfmaMinBatch;
+  // so does the VALU one, pole terms and m < 0 half included
+  const bool valu = ps || (!bf16 && !mixed && batch < kMfmaMinBatch);
+  const bool mfma64 = !valu && !bf16 && !mixed;
   const bool fill =
-      mfma64 || (!ps && bf16 && !poles && lat_forward_bf16_groups(a, split) == 1);
+      valu || mfma64 || (bf16 && !poles && lat_forward_bf16_groups(a, split) == 1);
   a.fill = fill ? 1 : 0;
-  a.mirror = fill && !poles && p->d.reality && !packed ? 1 : 0;
+  a.mirror = fill && (valu || !poles) && p->d.reality && !packed ? 1 : 0;
+  if (valu) a.pole = lat_pole(p, true, true, ps);
   if (!accumulate && !fill && (st = hip_status(launch_zero(flm, 2 * fs * batch, s)))) return st;
   {
     ProfScope prof(bf16 ? S2H_KERNEL_LAT_FORWARD_BF16
@@ -238,16 +254,15 @@ int lat_forward_stage(const s2h_plan* p, const cplx* ftm, void* flm, int batch, 
     // batches of 4 or more maps share each d-value across an 8-map MFMA tile;
     // the mixed-precision projection always runs on the FP32 matrix cores
     // multi-plane launches: the VALU kernel reads each map's own tables
-    if (ps)
-      st = hip_status(launch_lat_forward(a, false, s));
+    if (valu)
+      st = hip_status(launch_lat_forward(a, ps ? false : p->fwd_paired, s));
     else if (bf16)
       st = hip_status(launch_lat_forward_bf16(a, p->fwd_paired, split, s));
-    else if (mixed || batch >= kMfmaMinBatch)
-      st = hip_status(launch_lat_forward_mfma(a, p->fwd_paired, mixed, s));
     else
-      st = hip_status(launch_lat_forward(a, p->fwd_paired, s));
+      st = hip_status(launch_lat_forward_mfma(a, p->fwd_paired, mixed, s));
     if (st) return st;
   }
+  if (valu) return S2H_OK;
 
   if (p->fwd_row_south >= 0 || p->fwd_row_north >= 0) {
     PoleArgs pa{};
@@ -258,10 +273,8 @@ int lat_forward_stage(const s2h_plan* p, const cplx* ftm, void* flm, int batch, 
     pa.ftm_ncol = p->Mc;
     pa.ftm_m_first = p->m_lo;
     pa.L = L;
-    pa.spin = ps ? ps->spin0 : p->d.spin;
-    pa.spin_step = ps ? ps->spin_step : 0;
-    pa.lmin = ps ? p->d.L_lower : a.lmin_out;
-    pa.lmin_spin = ps ? 1 : 0;
+    pa.spin = p->d.spin;
+    pa.lmin = a.lmin_out;
     pa.row_south = p->fwd_row_south;
     pa.row_north = p->fwd_row_north;
     pa.norm = p->fwd_norm;
@@ -307,15 +320,16 @@ int lat_inverse_stage(const s2h_plan* p, const void* flm, cplx* ftm, int batch, 
                    s);
     // batches of 4 or more maps: each d-value feeds 16 maps through the MFMA;
     // multi-plane launches: the VALU kernel reads each map's own tables
-    if (ps)
-      st = hip_status(launch_lat_inverse(a, false, s));
-    else if (bf16)
+    const bool valu = ps || (!bf16 && !mixed && batch < kMfmaMinBatch);
+    if (valu) {
+      a.pole = lat_pole(p, false, false, ps);
+      return hip_status(launch_lat_inverse(a, ps ? false : p->inv_paired, s));
+    }
+    if (bf16)
       st = hip_status(launch_lat_inverse_bf16(a, p->inv_paired,
                                               precision == S2H_PREC_BF16X1 ? 1 : 3, s));
-    else if (mixed || batch >= kMfmaMinBatch)
-      st = hip_status(launch_lat_inverse_mma(a, p->inv_paired, mixed, s));
     else
-      st = hip_status(launch_lat_inverse(a, p->inv_paired, s));
+      st = hip_status(launch_lat_inverse_mma(a, p->inv_paired, mixed, s));
     if (st) return st;
   }
 
@@ -328,8 +342,7 @@ int lat_inverse_stage(const s2h_plan* p, const void* flm, cplx* ftm, int batch, 
     pa.ftm_ncol = p->Mc;
     pa.ftm_m_first = p->m_lo;
     pa.L = p->d.L;
-    pa.spin = ps ? ps->spin0 : p->d.spin;
-    pa.spin_step = ps ? ps->spin_step : 0;
+    pa.spin = p->d.spin;
     pa.lmin = p->d.L_lower;
     pa.row_south = p->inv_row_south;
     pa.row_north = p->inv_row_north;
@@ -747,27 +760,9 @@ int forward_adjoint_impl(const s2h_plan* p, const PlaneSet* ps, const void* g, v
   a.ftm_m_first = p->m_lo;
   a.lmin_out = std::max(std::abs(p->d.spin), p->d.L_lower);
   if (ps) a.planes = ps->fwd;
+  // the pole rows of the synthesis are the adjoint of the forward pole terms
+  a.pole = lat_pole(p, true, true, ps);
   if ((st = hip_status(launch_lat_inverse(a, ps ? false : p->fwd_paired, s)))) return st;
-  if (p->fwd_row_south >= 0 || p->fwd_row_north >= 0) {
-    // adjoint of the forward pole terms: the pole rows of the synthesis
-    PoleArgs pa{};
-    pa.flm = const_cast<cplx*>(gin);
-    pa.flm_map_stride = fs;
-    pa.ftm = ftm;
-    pa.ftm_map_stride = ftm_stride;
-    pa.ftm_ncol = p->Mc;
-    pa.ftm_m_first = p->m_lo;
-    pa.L = L;
-    pa.spin = ps ? ps->spin0 : p->d.spin;
-    pa.spin_step = ps ? ps->spin_step : 0;
-    pa.lmin = ps ? p->d.L_lower : a.lmin_out;
-    pa.lmin_spin = ps ? 1 : 0;
-    pa.row_south = p->fwd_row_south;
-    pa.row_north = p->fwd_row_north;
-    pa.norm = p->fwd_norm;
-    pa.batch = batch;
-    if ((st = hip_status(launch_pole_inverse(pa, s)))) return st;
-  }
   int64_t in_stride = ftm_stride;
   if (resample) {
     if ((st = theta_mix_stage(p, ps, spec, ftm, batch, true, s))) return st;
@@ -800,8 +795,6 @@ int inverse_adjoint_impl(const s2h_plan* p, const PlaneSet* ps, const void* g, i
   const int64_t fs = flm_stride(p);
   cplx* ftm = static_cast<cplx*>(work);
   const int64_t ftm_stride = (int64_t)p->inv_rows * p->Mc;
-  if ((st = hip_status(launch_zero(grad_flm, 2 * fs * batch, s)))) return st;
-
   RingFwdArgs r{};
   r.f = g;
   r.f_complex = g_is_complex;
@@ -825,30 +818,11 @@ int inverse_adjoint_impl(const s2h_plan* p, const PlaneSet* ps, const void* g, i
   a.ftm_m_first = p->m_lo;
   a.lmin_out = p->d.L_lower;
   if (ps) a.planes = ps->inv;
-  if ((st = hip_status(launch_lat_forward(a, ps ? false : p->inv_paired, s)))) return st;
-  if (p->inv_row_south >= 0 || p->inv_row_north >= 0) {
-    PoleArgs pa{};
-    pa.flm = static_cast<cplx*>(grad_flm);
-    pa.flm_map_stride = fs;
-    pa.ftm = ftm;
-    pa.ftm_map_stride = ftm_stride;
-    pa.ftm_ncol = p->Mc;
-    pa.ftm_m_first = p->m_lo;
-    pa.L = L;
-    pa.spin = ps ? ps->spin0 : p->d.spin;
-    pa.spin_step = ps ? ps->spin_step : 0;
-    pa.lmin = p->d.L_lower;
-    pa.row_south = p->inv_row_south;
-    pa.row_north = p->inv_row_north;
-    pa.norm = p->inv_norm;
-    pa.batch = batch;
-    if ((st = hip_status(launch_pole_forward(pa, s)))) return st;
-  }
-  if (real) {
-    if ((st = hip_status(launch_scale_pos_m(static_cast<cplx*>(grad_flm), fs, L, batch, 2.0, s))))
-      return st;
-  }
-  return S2H_OK;
+  a.pole = lat_pole(p, false, false, ps);
+  // real maps: the inverse reads m >= 0 only and completes Hermitian-symmetrically
+  a.mirror = real ? 2 : 0;
+  a.pos_scale = real ? 2.0 : 1.0;
+  return hip_status(launch_lat_forward(a, ps ? false : p->inv_paired, s));
 }
 
 }  // namespace
@@ -896,8 +870,8 @@ extern "C" int s2h_lat_forward(const s2h_plan* p, const void* ftm, void* flm, in
   const int L = p->d.L;
   const bool wide = p->d.sampling == S2H_MWSS || p->d.sampling == S2H_HEALPIX;
   const int ncol = wide ? 2 * L : 2 * L - 1;
-  if ((st = hip_status(launch_zero(flm, 2 * flm_stride(p) * batch, s)))) return st;
   LatArgs a = lat_args(p, true, batch);
+  a.mirror = p->m_lo == 0 ? 2 : 0;
   a.rings = p->inv_rings;
   a.nrings = p->n_inv_rings;
   a.flm = static_cast<cplx*>(flm);

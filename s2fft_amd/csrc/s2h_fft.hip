@@ -162,6 +162,7 @@ hipError_t launch_wigner_fill(cplx* flmn, int L, int N, hipStream_t s) {
 hipError_t allow_large_lds() {
   hipError_t e = allow_large_lds_rings();
   if (e == hipSuccess) e = allow_large_lds_alias();
+  if (e == hipSuccess) e = allow_large_lds_lat();
   if (e != hipSuccess) return e;
   const int bytes = 2 * sizeof(double) * kFftMax;
   return hipFuncSetAttribute((const void*)chirp_setup_kernel,

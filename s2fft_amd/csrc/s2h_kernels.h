@@ -110,17 +110,25 @@ struct RingAliasArgs {
 // Wigner transform: one spin -n per map, every other table shared).
 struct LatPlane {
   const MStart* mstart;     // indexed by m - m_lo
-  const Coef* coef;         // [|m|][l]
+  const Coef* ucoef;        // [|m|][l], unit-c form
   int lmin_out;             // first l written / read
   int pad;
+};
+
+// Pole rows of the VALU latitudinal kernels (-1: none): map b has spin + spin_step
+// b, its sums run from l = lmin, or (lmin_spin) from max(lmin, |its spin|).
+struct LatPole {
+  int south = -1, north = -1;
+  int spin = 0, spin_step = 0;
+  int lmin = 0, lmin_spin = 0;
+  const double* norm = nullptr;  // per-l normalisation (times the global sign)
 };
 
 struct LatArgs {
   const LatRing* rings;
   int nrings;               // entries of rings (pairs count as one)
   const MStart* mstart;     // indexed by m - m_lo
-  const Coef* coef;         // [|m|][l]
-  const Coef* ucoef;        // [|m|][l], unit-c form {a', b', sigma, 0} (BF16 kernels)
+  const Coef* ucoef;        // [|m|][l], unit-c form {a', b', sigma, 0}
   int L;
   int m_lo;                 // first m handled (0 or -(L-1))
   int nm;                   // number of m values handled
@@ -135,12 +143,15 @@ struct LatArgs {
   int ftm_ncol;
   int ftm_m_first;
   int ftm_tiled;            // ring spectra in blocks of 8 rings (spec_row)
-  int groups;               // ring groups per m (forward); >1 accumulates atomically
+  int groups;               // ring groups per m; >1 accumulates atomically (matrix-core forwards)
   int accumulate;           // forward: add into flm instead of overwriting it
   int fill;                 // forward, one ring group per m: also write zeros below
                             // max(ell0, lmin_out), so flm needs no zeroing pass
-  int mirror;               // forward with fill, real maps: also write
-                            // flm[l, -m] = (-1)^m conj(flm[l, m]) (no conjugate fill pass)
+  int mirror;               // forward with fill, real maps: 1: also write
+                            // flm[l, -m] = (-1)^m conj(flm[l, m]) (no conjugate fill pass),
+                            // 2 (VALU kernels): zeros there
+  double pos_scale;         // VALU forward: factor of the m > 0 columns
+  LatPole pole;             // VALU kernels
   int flm_packed;           // flm in the packed m-major layout (real maps, m >= 0 only)
   const LatPlane* planes;   // non-null: map b uses planes[b] in place of mstart, coef and
                             // lmin_out (VALU kernels, unpaired rings)
@@ -183,6 +194,7 @@ hipError_t launch_ring_fft_inverse(const RingInvArgs& a, const JobSet& js, int b
                                    hipStream_t s);
 hipError_t allow_large_lds_rings();
 hipError_t allow_large_lds_alias();
+hipError_t allow_large_lds_lat();
 hipError_t launch_ring_alias(const RingAliasArgs& a, const JobSet& js, int batch, hipStream_t s);
 // pq[b] = sum_m c_m Re(conj(Y) A(Y)) over every ring of map b (part: batch x
 // ring_dot_jobs(js) doubles); alpha[b] = num[b] / pq[b] when alpha is given
@@ -237,6 +249,8 @@ hipError_t launch_wigner_fill_adjoint(cplx* g, int L, int N, hipStream_t s);
 hipError_t launch_real_to_complex(const double* in, cplx* out, int64_t n, hipStream_t s);
 hipError_t allow_large_lds();
 
+// The VALU kernels: batches of a few maps, multi-plane launches, the adjoints.  The
+// forward writes every entry of its columns (fill implied), poles included.
 hipError_t launch_lat_inverse(const LatArgs& a, bool paired, hipStream_t s);
 hipError_t launch_lat_forward(const LatArgs& a, bool paired, hipStream_t s);
 hipError_t launch_lat_forward_mfma(const LatArgs& a, bool paired, bool fp32, hipStream_t s);
@@ -337,12 +351,7 @@ struct PoleArgs {
   int row_north;            // -1 if absent
   const double* norm;       // per-l normalisation (times the global sign)
   int batch;
-  int spin_step;            // map b has spin + spin_step b (multi-plane launches)
-  int lmin_spin;            // lmin of map b is max(lmin, |its spin|)
 };
-__host__ __device__ __forceinline__ int pole_spin(const PoleArgs& a, int64_t b) {
-  return a.spin + a.spin_step * (int)b;
-}
 hipError_t launch_pole_inverse(const PoleArgs& a, hipStream_t s);
 hipError_t launch_pole_forward(const PoleArgs& a, hipStream_t s);
 hipError_t launch_zero(void* p, int64_t ndoubles, hipStream_t s);
@@ -392,8 +401,6 @@ hipError_t launch_batch_sumsq(const double* x, int64_t n, int64_t stride, int ba
 hipError_t launch_reality_fill(cplx* flm, int64_t map_stride, int L, int batch, hipStream_t s);
 hipError_t launch_reality_fold(const cplx* g, cplx* out, int64_t map_stride, int L, int batch,
                                hipStream_t s);
-hipError_t launch_scale_pos_m(cplx* flm, int64_t map_stride, int L, int batch, double factor,
-                              hipStream_t s);
 
 struct ResampleArgs {
   const cplx* in;           // phi-spectrum [b][row][col], col <-> m = m_lo + col

@@ -56,27 +56,37 @@ __device__ __forceinline__ void start_value(const MStart& st, double c2, double 
   d = ldexp(v.m, v.e - 512 * ls);
 }
 
-// m 2^e (1 + r): a product that carries its rounding errors along in r.
-struct ExtR {
-  double m;
+// (hi + lo) 2^e: a factor with its rounding error, |hi| in [1/2, 1) or zero.
+struct ExtD {
+  double hi, lo;
   int e;
-  double r;
 };
-__device__ __forceinline__ ExtR extr_mul(ExtR a, ExtR b) {
-  const double p = a.m * b.m;
+__device__ __forceinline__ ExtD extd_of(double v, double rel) {
   int e;
-  const double m = frexp(p, &e);
-  const double err = fma(a.m, b.m, -p) * __builtin_amdgcn_rcp(p);
-  return {m, a.e + b.e + e, a.r + b.r + (p != 0.0 ? err : 0.0)};
+  const double hi = frexp(v, &e);
+  return {hi, hi * rel, e};
 }
-__device__ __forceinline__ ExtR extr_pow(ExtR x, int k) {
-  ExtR r = {0.5, 1, 0.0};
+// a *= b, not normalised: hundreds of factors in [1/4, 1) fit
+__device__ __forceinline__ void extd_mul(ExtD& a, const ExtD& b) {
+  const double p = a.hi * b.hi;
+  a.lo = fma(a.hi, b.lo, fma(a.lo, b.hi, fma(a.hi, b.hi, -p)));
+  a.hi = p;
+  a.e += b.e;
+}
+// a *= x^k by squarings of x, each brought back to [1/2, 1)
+__device__ __forceinline__ void extd_mul_pow(ExtD& a, ExtD x, int k) {
   while (k) {
-    if (k & 1) r = extr_mul(r, x);
+    if (k & 1) extd_mul(a, x);
     k >>= 1;
-    if (k) x = extr_mul(x, x);
+    if (k) {
+      const double p = x.hi * x.hi;
+      const double lo = fma(2.0 * x.hi, x.lo, fma(x.hi, x.hi, -p));
+      int e;
+      x.hi = frexp(p, &e);
+      x.lo = ldexp(lo, -e);
+      x.e = 2 * x.e + e;
+    }
   }
-  return r;
 }
 
 // start_value for the FP64 kernels.  c2 and s2 rounded to FP64 and multiplied
@@ -86,22 +96,29 @@ __device__ __forceinline__ ExtR extr_pow(ExtR x, int k) {
 // of the difference of the exponents (at most 2 |n|) in place of two powers.
 __device__ __forceinline__ void start_value_fp64(const MStart& st, const LatRing& rg, double& d,
                                                  int& lscale) {
-  const Ext c = ext_of(rg.c2), s = ext_of(rg.s2);
-  const ExtR cr = {c.m, c.e, rg.c2r}, sr = {s.m, s.e, rg.s2r};
+  const ExtD c = extd_of(rg.c2, rg.c2r), s = extd_of(rg.s2, rg.s2r);
   const int k = st.ecos < st.esin ? st.ecos : st.esin;
-  ExtR v = {st.kmant, st.kexp, 0.0};
-  if (k) v = extr_mul(v, extr_pow(extr_mul(cr, sr), k));
-  if (st.ecos > k) v = extr_mul(v, extr_pow(cr, st.ecos - k));
-  if (st.esin > k) v = extr_mul(v, extr_pow(sr, st.esin - k));
-  if (v.m == 0.0) {
+  ExtD v = {st.kmant, 0.0, st.kexp};
+  if (k) {
+    ExtD cs = c;  // in [1/4, 1)
+    extd_mul(cs, s);
+    extd_mul_pow(v, cs, k);
+  }
+  if (st.ecos > k) extd_mul_pow(v, c, st.ecos - k);
+  if (st.esin > k) extd_mul_pow(v, s, st.esin - k);
+  if (v.hi == 0.0) {
     d = 0.0;
     lscale = 0;
     return;
   }
-  int ls = -((256 - v.e) >> 9);
+  int ve;
+  v.hi = frexp(v.hi, &ve);
+  v.lo = ldexp(v.lo, -ve);
+  ve += v.e;
+  int ls = -((256 - ve) >> 9);
   if (ls > 0) ls = 0;
   lscale = ls;
-  d = ldexp(fma(v.m, v.r, v.m), v.e - 512 * ls);
+  d = ldexp(v.hi + v.lo, ve - 512 * ls);
 }
 
 // Moves (d, dm1) down by 2^512 once |d| passes 2^256.  The recursion grows

@@ -8,31 +8,29 @@ namespace s2h {
 // Inverse: s2fft/transforms/spherical.py:166-177.  The south-pole row holds
 // only m = spin: sum_l (-1)^|l-spin| flm[l, spin]; the north-pole row only
 // m = -spin: sum_l flm[l, -spin] (both with the normalisation folded in).
+__device__ __forceinline__ double block_sum(double v, double* red);
+
 __global__ void __launch_bounds__(kThreads) pole_inverse_kernel(PoleArgs a) {
+  __shared__ double red[kThreads / 64];
   const int64_t b = blockIdx.y;
   const bool south = blockIdx.x == 0;
   const int row = south ? a.row_south : a.row_north;
   if (row < 0) return;
-  const int spin = pole_spin(a, b);
-  const int aspin = spin < 0 ? -spin : spin;
-  const int lmin = a.lmin_spin && aspin > a.lmin ? aspin : a.lmin;
+  const int m = south ? a.spin : -a.spin;
   cplx* r = a.ftm + b * a.ftm_map_stride + (int64_t)row * a.ftm_ncol;
-  for (int c = threadIdx.x; c < a.ftm_ncol; c += kThreads) r[c] = {0.0, 0.0};
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const int m = south ? spin : -spin;
-    const cplx* f = a.flm + b * a.flm_map_stride + (a.L - 1 + m);
-    cplx acc = {0.0, 0.0};
-    for (int l = lmin; l < a.L; ++l) {
-      double w = a.norm[l];
-      if (south && ((l - spin) & 1)) w = -w;
-      const cplx v = f[(int64_t)l * (2 * a.L - 1)];
-      acc.x += w * v.x;
-      acc.y += w * v.y;
-    }
-    const int c = m - a.ftm_m_first;
-    if (c >= 0 && c < a.ftm_ncol) r[c] = acc;
+  const int cm = m - a.ftm_m_first;
+  for (int c = threadIdx.x; c < a.ftm_ncol; c += kThreads)
+    if (c != cm) r[c] = {0.0, 0.0};
+  const cplx* f = a.flm + b * a.flm_map_stride + (a.L - 1 + m);
+  cplx acc = {0.0, 0.0};
+  for (int l = a.lmin + threadIdx.x; l < a.L; l += kThreads) {
+    const double w = a.norm[l], sw = south && ((l - a.spin) & 1) ? -w : w;
+    const cplx v = f[(int64_t)l * (2 * a.L - 1)];
+    acc = {fma(sw, v.x, acc.x), fma(sw, v.y, acc.y)};
   }
+  acc.x = block_sum(acc.x, red);
+  acc.y = block_sum(acc.y, red);
+  if (threadIdx.x == 0 && cm >= 0 && cm < a.ftm_ncol) r[cm] = acc;
 }
 
 // Forward: s2fft/transforms/spherical.py:562-571.  flm[l, spin] gets
@@ -40,10 +38,8 @@ __global__ void __launch_bounds__(kThreads) pole_inverse_kernel(PoleArgs a) {
 __global__ void __launch_bounds__(kThreads) pole_forward_kernel(PoleArgs a) {
   const int64_t b = blockIdx.y;
   const int l = blockIdx.x * kThreads + threadIdx.x;
-  const int spin = pole_spin(a, b);
-  const int aspin = spin < 0 ? -spin : spin;
-  const int lmin = a.lmin_spin && aspin > a.lmin ? aspin : a.lmin;
-  if (l < lmin || l >= a.L) return;
+  const int spin = a.spin;
+  if (l < a.lmin || l >= a.L) return;
   const cplx* base = a.ftm + b * a.ftm_map_stride;
   cplx* f = a.flm + b * a.flm_map_stride + (int64_t)l * (2 * a.L - 1);
   const double w = a.norm[l];
@@ -633,31 +629,11 @@ __global__ void __launch_bounds__(kThreads) reality_fold_kernel(const cplx* g, c
   o[L - 1 + m] = {0.5 * (a.x + s * c.x), 0.5 * (a.y - s * c.y)};
 }
 
-// flm[l, m] *= factor for m >= 1 (adjoint of the Hermitian completion).
-__global__ void __launch_bounds__(kThreads) scale_pos_m_kernel(cplx* flm, int64_t map_stride,
-                                                               int L, double factor) {
-  const int64_t b = blockIdx.z;
-  const int l = blockIdx.y;
-  const int m = blockIdx.x * kThreads + threadIdx.x + 1;
-  if (m >= L) return;
-  cplx* o = flm + b * map_stride + (int64_t)l * (2 * L - 1) + (L - 1 + m);
-  o->x *= factor;
-  o->y *= factor;
-}
-
 hipError_t launch_reality_fold(const cplx* g, cplx* out, int64_t map_stride, int L, int batch,
                                hipStream_t s) {
   if (batch == 0) return hipSuccess;
   hipLaunchKernelGGL(reality_fold_kernel, dim3((L + kThreads - 1) / kThreads, L, batch),
                      dim3(kThreads), 0, s, g, out, map_stride, L);
-  return hipGetLastError();
-}
-
-hipError_t launch_scale_pos_m(cplx* flm, int64_t map_stride, int L, int batch, double factor,
-                              hipStream_t s) {
-  if (batch == 0 || L < 2) return hipSuccess;
-  hipLaunchKernelGGL(scale_pos_m_kernel, dim3((L - 1 + kThreads - 1) / kThreads, L, batch),
-                     dim3(kThreads), 0, s, flm, map_stride, L, factor);
   return hipGetLastError();
 }
 

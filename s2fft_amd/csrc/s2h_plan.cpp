@@ -798,8 +798,8 @@ extern "C" int s2h_wigner_plan_create(s2h_wigner_plan** out, const s2h_wigner_de
     for (int k = 0; k < w->G; ++k) {
       const s2h_plan* p = w->plans[k];
       const int an = std::abs(k - (d.N - 1));
-      fp.push_back(LatPlane{p->fwd_mstart, p->fwd_coef, std::max(an, d.L_lower), 0});
-      ip.push_back(LatPlane{p->inv_mstart, p->inv_coef, d.L_lower, 0});
+      fp.push_back(LatPlane{p->fwd_mstart, p->fwd_ucoef, std::max(an, d.L_lower), 0});
+      ip.push_back(LatPlane{p->inv_mstart, p->inv_ucoef, d.L_lower, 0});
     }
     s2h_plan holder;  // upload() records allocations on a plan
     st = upload(&holder, fp, &w->fwd_planes);
