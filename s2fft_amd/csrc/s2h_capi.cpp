@@ -1453,10 +1453,7 @@ extern "C" int s2h_precompute_forward(const s2h_plan* p, const void* kernel, int
   a.flm_map_stride = flm_stride(p);
   a.scale = scale;
   a.batch = batch;
-  if ((st = hip_status(launch_pc_forward(a, s)))) return st;
-  if (p->d.reality)
-    return hip_status(launch_reality_fill(static_cast<cplx*>(flm), flm_stride(p), p->d.L, batch, s));
-  return S2H_OK;
+  return hip_status(launch_pc_forward(a, s));  // m < 0 of real maps included
 }
 
 extern "C" int s2h_precompute_inverse(const s2h_plan* p, const void* kernel, int kernel_is_complex,
