@@ -13,7 +13,37 @@ thread_local int g_last_xla_status = S2H_OK;
 
 int hip_status(hipError_t e) { return e == hipSuccess ? S2H_OK : S2H_ERR_HIP; }
 
+// FP64 latitudinal steps: the matrix-core kernels take whole tiles of maps (16 in
+// the inverse, 8 or 16 in the forward), the VALU ones each map's share.  The VALU
+// ones serve every batch below kMfmaMinBatch, and larger ones by these rules
+// (measured with HIP events; sizes are L / maps):
+// * forward, up to kValuFwdWaves waves of one ring per lane (all maps): MW 64 / 16
+//   12.5 us against 24.6, GL real 256 / 4 28 against 39, MW 128 / 16 (8160 waves) 29.5
+//   against 40; past it HEALPix real 449 / 4 (10776) 86 against 77;
+// * inverse, up to kValuInvBatch maps: HEALPix spin 2 512 / 4 154 us against 415 and
+//   / 8 317 against 424, real 449 / 5 62 against 101, 2048 / 8 4158 against 5617, MW
+//   200 / 8 40 against 37; with
+//   12 maps MW spin 2 512 284 against 247.  A larger batch leaves its last up to
+//   kValuInvBatch maps past whole tiles to them, or all up to kValuInvWaves waves
+//   (GL real 64 / 64, 4096 waves, 12 us against 17; MW 128 / 16, 8160, 25.5 against 24.6).
 constexpr int kMfmaMinBatch = 4;
+constexpr int kValuFwdWaves = 8192;
+constexpr int kValuInvWaves = 4096;
+constexpr int kValuInvBatch = 8;
+constexpr int kInvTile = 16;  // maps per workgroup of the matrix-core inverse
+
+int64_t valu_waves(const s2h_plan* p, int nrings, int batch) {
+  return (int64_t)p->nm * ((nrings + 63) / 64) * batch;
+}
+bool valu_forward(const s2h_plan* p, int batch) {
+  return batch < kMfmaMinBatch || valu_waves(p, p->n_fwd_rings, batch) <= kValuFwdWaves;
+}
+// Maps at the end of an inverse's batch that the VALU kernel takes.
+int valu_inverse_maps(const s2h_plan* p, int batch) {
+  if (batch <= kValuInvBatch || valu_waves(p, p->n_inv_rings, batch) <= kValuInvWaves) return batch;
+  const int rest = batch % kInvTile;
+  return rest <= kValuInvBatch ? rest : 0;
+}
 
 int check_device(const s2h_plan* p) {
   int dev = -1;
@@ -239,7 +269,7 @@ int lat_forward_stage(const s2h_plan* p, const cplx* ftm, void* flm, int batch, 
   // the FP64 matrix-core projection (one workgroup per m) and the BF16 ones
   // with one ring group per m write every entry of their m columns
   // so does the VALU one, pole terms and m < 0 half included
-  const bool valu = ps || (!bf16 && !mixed && batch < kMfmaMinBatch);
+  const bool valu = ps || (!bf16 && !mixed && valu_forward(p, batch));
   const bool mfma64 = !valu && !bf16 && !mixed;
   const bool fill =
       valu || mfma64 || (bf16 && !poles && lat_forward_bf16_groups(a, split) == 1);
@@ -318,12 +348,20 @@ int lat_inverse_stage(const s2h_plan* p, const void* flm, cplx* ftm, int batch, 
     ProfScope prof(bf16 ? S2H_KERNEL_LAT_INVERSE_BF16
                         : mixed ? S2H_KERNEL_LAT_INVERSE_FP32 : S2H_KERNEL_LAT_INVERSE,
                    s);
-    // batches of 4 or more maps: each d-value feeds 16 maps through the MFMA;
-    // multi-plane launches: the VALU kernel reads each map's own tables
-    const bool valu = ps || (!bf16 && !mixed && batch < kMfmaMinBatch);
-    if (valu) {
-      a.pole = lat_pole(p, false, false, ps);
-      return hip_status(launch_lat_inverse(a, ps ? false : p->inv_paired, s));
+    // the matrix-core kernel: each d-value feeds 16 maps; multi-plane launches: the
+    // VALU kernel reads each map's own tables
+    const int nv = ps ? batch
+                   : bf16 || mixed ? 0 : valu_inverse_maps(p, batch);
+    if (nv) {
+      LatArgs v = a;
+      v.batch = nv;
+      v.flm += (int64_t)(batch - nv) * a.flm_map_stride;
+      v.ftm += (int64_t)(batch - nv) * a.ftm_map_stride;
+      v.pole = lat_pole(p, false, false, ps);
+      st = hip_status(launch_lat_inverse(v, ps ? false : p->inv_paired, s));
+      batch -= nv;
+      a.batch = batch;
+      if (st || batch == 0) return st;
     }
     if (bf16)
       st = hip_status(launch_lat_inverse_bf16(a, p->inv_paired,
@@ -685,11 +723,11 @@ extern "C" int s2h_ring_dot(const s2h_plan* p, const void* Y, const double* num,
 }
 
 namespace {
-// Whether the synthesis of this call runs on the matrix-core kernels, whose
+// Whether the synthesis of this call runs on the matrix-core kernels alone, whose
 // epilogue adds up the dot over the rows without aliasing; their grid.x.
 int synth_dot_workgroups(const s2h_plan* p, int batch, int precision) {
   const bool bf16 = precision == S2H_PREC_BF16 || precision == S2H_PREC_BF16X1;
-  const bool mma = precision == S2H_PREC_MIXED || batch >= kMfmaMinBatch;
+  const bool mma = precision == S2H_PREC_MIXED || valu_inverse_maps(p, batch) == 0;
   if ((!bf16 && !mma) || p->spec_belt_wn == 0.0) return 0;
   return p->nm * ((p->n_inv_rings + 255) / 256);
 }

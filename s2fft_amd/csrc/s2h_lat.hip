@@ -554,24 +554,23 @@ int rings_per_lane(int nrings, int64_t columns, int rmax) {
   return R;
 }
 
-template <int R, int NB>
-hipError_t lat_inv_r(LatArgs a, bool paired, hipStream_t s) {
+template <int R, int NB, bool PAIRED>
+hipError_t lat_inv_r(LatArgs a, hipStream_t s) {
   // as many waves per workgroup (up to 4) as the rings fill
   const int waves = std::min(4, (a.nrings + 64 * R - 1) / (64 * R));
   a.groups = (a.nrings + 64 * R * waves - 1) / (64 * R * waves);
   const dim3 grid(a.nm * a.groups, 1, (a.batch + NB - 1) / NB), block(64 * waves);
-  if (paired)
-    hipLaunchKernelGGL((lat_inverse_kernel<R, NB, true>), grid, block, 0, s, a);
-  else
-    hipLaunchKernelGGL((lat_inverse_kernel<R, NB, false>), grid, block, 0, s, a);
+  hipLaunchKernelGGL((lat_inverse_kernel<R, NB, PAIRED>), grid, block, 0, s, a);
   return hipGetLastError();
 }
+// Sums of 4 rings of 3 or 4 maps in two parities would not fit the registers.
 template <int NB>
 hipError_t lat_inv_nb(const LatArgs& a, bool paired, hipStream_t s) {
-  switch (rings_per_lane(a.nrings, (int64_t)a.nm * ((a.batch + NB - 1) / NB), NB == 4 ? 2 : 4)) {
-    case 1: return lat_inv_r<1, NB>(a, paired, s);
-    case 2: return lat_inv_r<2, NB>(a, paired, s);
-    default: return lat_inv_r<(NB == 4 ? 2 : 4), NB>(a, paired, s);
+  const int64_t columns = (int64_t)a.nm * ((a.batch + NB - 1) / NB);
+  switch (rings_per_lane(a.nrings, columns, paired && NB > 2 ? 2 : 4)) {
+    case 1: return paired ? lat_inv_r<1, NB, true>(a, s) : lat_inv_r<1, NB, false>(a, s);
+    case 2: return paired ? lat_inv_r<2, NB, true>(a, s) : lat_inv_r<2, NB, false>(a, s);
+    default: return paired ? lat_inv_r<(NB > 2 ? 2 : 4), NB, true>(a, s) : lat_inv_r<4, NB, false>(a, s);
   }
 }
 
@@ -591,9 +590,14 @@ hipError_t lat_fwd_r(const LatArgs& a, bool paired, hipStream_t s) {
 
 hipError_t launch_lat_inverse(const LatArgs& a, bool paired, hipStream_t s) {
   if (a.nm == 0 || a.nrings == 0 || a.batch == 0) return hipSuccess;
-  if (a.planes || a.batch == 1) return lat_inv_nb<1>(a, paired, s);  // one map (plane) per block
-  if (a.batch == 2) return lat_inv_nb<2>(a, paired, s);
-  return lat_inv_nb<4>(a, paired, s);
+  // up to 4 maps per workgroup (a multi-plane launch: one), evenly
+  const int chunks = a.planes ? a.batch : (a.batch + 3) / 4;
+  switch ((a.batch + chunks - 1) / chunks) {
+    case 1: return lat_inv_nb<1>(a, paired, s);
+    case 2: return lat_inv_nb<2>(a, paired, s);
+    case 3: return lat_inv_nb<3>(a, paired, s);
+    default: return lat_inv_nb<4>(a, paired, s);
+  }
 }
 
 hipError_t launch_lat_forward(const LatArgs& a, bool paired, hipStream_t s) {

@@ -1,7 +1,7 @@
 """The latitudinal kernels of small batches against those of larger ones (needs a GPU).
 
-Batches of 1 to 3 maps take the VALU kernels, 4 and more the matrix-core ones: the
-same maps alone and inside a batch of 5 have to agree.  The sizes cover one and
+Batches of 1 to 3 maps take the VALU kernels, larger ones at the larger sizes the
+matrix-core projection: the same maps alone and inside a batch of 5 have to agree.  The sizes cover one and
 several waves of rings, one to eight rings per lane, last waves of one ring, pairs
 with and without an equator, pole rows (also for l < |spin|), a first l above zero,
 and the most rings a plan has (4096).  Both sides carry
