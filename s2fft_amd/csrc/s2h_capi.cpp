@@ -309,6 +309,7 @@ int lat_forward_stage(const s2h_plan* p, const cplx* ftm, void* flm, int batch, 
     pa.row_north = p->fwd_row_north;
     pa.norm = p->fwd_norm;
     pa.batch = batch;
+    pa.ftm_tiled = a.ftm_tiled;
     if ((st = hip_status(launch_pole_forward(pa, s)))) return st;
   }
 
@@ -394,7 +395,7 @@ int lat_inverse_stage(const s2h_plan* p, const void* flm, cplx* ftm, int batch, 
 // The theta step of the MW / MWSS forward: phi-spectra of the input rows
 // `spec` to the projection's rows `ftm` (or, adjoint, back).
 int theta_mix_stage(const s2h_plan* p, const PlaneSet* ps, cplx* spec, cplx* ftm, int batch,
-                    bool adjoint, hipStream_t s) {
+                    bool adjoint, hipStream_t s, bool tiled = false) {
   const int64_t spec_map = (int64_t)p->fwd_in_rows * p->Mc, ftm_map = (int64_t)p->fwd_rows * p->Mc;
   ThetaMixArgs t{};
   t.in = adjoint ? ftm : spec;
@@ -407,6 +408,7 @@ int theta_mix_stage(const s2h_plan* p, const PlaneSet* ps, cplx* spec, cplx* ftm
   t.spin_step = ps ? ps->spin_step : 0;
   t.adjoint = adjoint ? 1 : 0;
   t.nyquist = p->d.reality ? 0 : 1;
+  t.out_tiled = tiled ? 1 : 0;
   ProfScope prof(S2H_KERNEL_RESAMPLE, s);
   return hip_status(launch_theta_mix(p->mix.get(), t, batch, s));
 }
@@ -437,8 +439,12 @@ int forward_impl(const s2h_plan* p, const PlaneSet* ps, const void* f, int f_is_
   cplx* spec = ftm;
   if (resample) ftm = spec + (int64_t)batch * p->fwd_in_rows * p->Mc;
   if ((st = ring_analysis_stage(p, f, f_is_complex, resample ? spec : ftm, batch, s))) return st;
-  if (resample && (st = theta_mix_stage(p, ps, spec, ftm, batch, false, s))) return st;
-  return lat_forward_stage(p, ftm, flm, batch, precision, accumulate, s, false, ps);
+  if (!resample) return lat_forward_stage(p, ftm, flm, batch, precision, accumulate, s, false, ps);
+  // The FP64 projections gather single columns: in blocks of 8 rows a column is
+  // made of 128-byte runs, ring-major of one value per line.
+  const SpecView sv{(int64_t)p->fwd_rows * p->Mc, precision == S2H_PREC_FP64 ? 1 : 0};
+  if ((st = theta_mix_stage(p, ps, spec, ftm, batch, false, s, sv.tiled != 0))) return st;
+  return lat_forward_stage(p, ftm, flm, batch, precision, accumulate, s, false, ps, &sv);
 }
 
 }  // namespace

@@ -351,6 +351,7 @@ struct PoleArgs {
   int row_north;            // -1 if absent
   const double* norm;       // per-l normalisation (times the global sign)
   int batch;
+  int ftm_tiled;            // forward: ftm in blocks of 8 rows (spec_row)
 };
 hipError_t launch_pole_inverse(const PoleArgs& a, hipStream_t s);
 hipError_t launch_pole_forward(const PoleArgs& a, hipStream_t s);
@@ -433,6 +434,7 @@ struct ThetaMixArgs {
   int spin, spin_step;      // map b has spin + spin_step b
   int adjoint;
   int nyquist;              // complex signals: the theta-Nyquist term at q = -L
+  int out_tiled;            // out in blocks of 8 rows (spec_row)
 };
 hipError_t launch_theta_mix(const ThetaMix* x, const ThetaMixArgs& a, int batch, hipStream_t s);
 

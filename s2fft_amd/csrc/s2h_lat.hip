@@ -74,14 +74,6 @@ __device__ __forceinline__ StepCoef<PAIRED> step_coef(const Coef& c, double bsig
     return {c.a, -c.b * bsign};
 }
 
-// Blocks go to the 8 XCDs in turn and there to the 32 CUs in turn, the longest
-// columns first; every second row of 32 in reverse evens out what the CUs get
-// (forward at L = 1024 173 -> 165 us).
-__device__ __forceinline__ int balanced_block(int i, int n) {
-  const int j = i >> 3;
-  return ((j >> 5) & 1) && (j | 31) < (n >> 3) ? ((j ^ 31) << 3) | (i & 7) : i;
-}
-
 // One step: (d, dm1) = (e^l, e^{l-1}) -> (e^{l+1}, e^l).
 template <bool PAIRED>
 __device__ __forceinline__ void step(const StepCoef<PAIRED>& c, double x, double& d, double& dm1) {
@@ -146,7 +138,7 @@ lat_inverse_kernel(LatArgs a) {
   __shared__ StepCoef<PAIRED> cs[2][kChunk];
   __shared__ cplx fs[2][NB][kChunk];
   int g;
-  const int m = lat::m_group_of_block(balanced_block(blockIdx.x, gridDim.x), a.nm, a.groups,
+  const int m = lat::m_group_of_block(lat::balanced_block(blockIdx.x, gridDim.x), a.nm, a.groups,
                                       a.m_lo, g);
   const int am = m < 0 ? -m : m;
   const int tid = threadIdx.x, nthr = blockDim.x;
@@ -336,7 +328,7 @@ lat_forward_kernel(LatArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char fwd_raw[];
   __shared__ StepCoef<PAIRED> cs[2][kChunk];
   __shared__ double sg[2][kChunk];
-  const int m = lat::m_of_block(balanced_block(blockIdx.x, gridDim.x), a.nm, a.m_lo);
+  const int m = lat::m_of_block(lat::balanced_block(blockIdx.x, gridDim.x), a.nm, a.m_lo);
   const int am = m < 0 ? -m : m;
   const int64_t b = blockIdx.z;
   const int tid = threadIdx.x, nthr = blockDim.x, lane = tid & 63, wave = tid >> 6;
@@ -417,8 +409,8 @@ lat_forward_kernel(LatArgs a) {
   const int pspin = pole_spin_of(a.pole, b), plmin = pole_lmin_of(a.pole, b);
   const bool south = a.pole.south >= 0 && m == pspin, north = a.pole.north >= 0 && m == -pspin;
   cplx ps = {0.0, 0.0}, pn = {0.0, 0.0};
-  if (south) ps = ftm[(int64_t)a.pole.south * a.ftm_ncol];
-  if (north) pn = ftm[(int64_t)a.pole.north * a.ftm_ncol];
+  if (south) ps = ftm[spec_row(a.pole.south, a.ftm_ncol, a.ftm_tiled)];
+  if (north) pn = ftm[spec_row(a.pole.north, a.ftm_ncol, a.ftm_tiled)];
   // rows below the first l (the packed layout holds none)
   if (!a.flm_packed) {
     for (int l = tid; l < min(l0, L); l += nthr) {

@@ -131,6 +131,14 @@ __device__ __forceinline__ void rescale(double& d, double& dm1, int& lscale) {
   lscale += big ? 1 : 0;
 }
 
+// Blocks go to the 8 XCDs in turn and there to the 32 CUs in turn, the longest
+// columns first; every second row of 32 in reverse evens out what the CUs get
+// (forward at L = 1024 173 -> 165 us).
+__device__ __forceinline__ int balanced_block(int i, int n) {
+  const int j = i >> 3;
+  return ((j >> 5) & 1) && (j | 31) < (n >> 3) ? ((j ^ 31) << 3) | (i & 7) : i;
+}
+
 // blockIdx.x -> m: 4 adjacent m per XCD in a row (workgroups are dealt to the
 // 8 XCDs round-robin), heaviest (smallest |m|) first.  For m_lo < 0 the order
 // is 0, -1, 1, -2, 2, ...

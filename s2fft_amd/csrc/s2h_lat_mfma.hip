@@ -35,9 +35,6 @@ namespace s2h {
 
 namespace {
 
-constexpr int kMW = 8;         // waves per workgroup
-constexpr int kMT = kMW * 64;  // threads
-constexpr int kSets = 2;       // 64-pair sets per wave
 constexpr int kTile = 8;       // maps per tile (16 MFMA rows)
 constexpr int kPad = 17;       // LDS row stride (elements) of the d tile
 
@@ -48,25 +45,37 @@ using lat::wave_sync;
 
 }  // namespace
 
-// FP64: one workgroup per (m, 16-map tile) covers every ring pair of its m.
-// Its 8 waves take 512 pairs per pass (64 per wave); a pass walks l from the
-// m's first l to L and adds its sums into flm, so no two workgroups write one
-// element and nothing needs atomics or a zeroing pass.  The 16 maps form two
-// 8-map row tiles of the matrix-core product that share each d-value (B
-// operand), so each recursion step feeds 4 products instead of 2.  The first
-// pass stores (writing the zeros below the m's first l and, with `mirror`,
-// the m < 0 half last pass), later passes add; one thread owns each output
-// element in every pass, so each addition reads that thread's own store.
+// FP64: one workgroup per (m, tile of 8 MT maps) covers every ring pair of its m.
+// A wave takes SETS x 64 pairs per pass, one recursion per lane and set; a pass
+// walks l from the m's first l to L, 32 at a time, and adds its sums into flm, so
+// no two workgroups write one element and nothing needs atomics or a zeroing pass.
+// The first pass stores (writing the zeros below the m's first l and, with
+// `mirror`, the m < 0 half last pass), later passes add; one thread owns each
+// output element in every pass, so each addition reads that thread's own store,
+// loaded at the start of its chunk.
+// Bound by the matrix cores (64 cycles per product, one per 4 rings, 16 l and 8
+// maps), if the recursion, the sums over waves and the memory stay hidden behind
+// them: a wave alternates between the phases, so two workgroups of 4 waves share a
+// CU and fill each other's gaps.  The ring-side operands of a wave's rings sit in
+// registers for the whole pass: 128 of them hold 2 sets of 16 maps or 4 of 8, of pairs
+// (two parities) half that; past 256 pairs one workgroup of 8 waves saves the second
+// pass and the second reading of the recursions instead.  Measured: MW L = 512, spin
+// 2, 64 maps 1411 -> 1259 us, from spectra in blocks of 8 rows (a column in 128-byte
+// runs) 1035 us (0.5 ms of products); GL L = 700, spin 1, 5 maps 575 -> 413 us (all
+// 700 rings in one pass); MW L = 256, real, 32 maps 88 -> 64 us.  Pairs on 4 waves of
+// 2 sets: HEALPix L = 449, 5 maps 97 us against 74 on 8 waves, L = 512, 16 maps 519
+// against 494.
 // TILED: the spectra layout (spec_row) as a compile-time choice, so that the
 // ring-major gathers carry no layout select in their address arithmetic
-template <int MT, bool PAIRED, bool TILED>
-__global__ void __launch_bounds__(kMT) lat_forward_f64_kernel(LatArgs a) {
+template <int W, int MT, int SETS, bool PAIRED, bool TILED>
+__global__ void __launch_bounds__(64 * W, 2) lat_forward_f64_kernel(LatArgs a) {
   typedef lat::v4d acc_t;
-  static_assert(64 * kPad * sizeof(double) >= MT * 2 * 16 * 16 * sizeof(double), "result tile fits");
-  __shared__ double dte[kMW][64 * kPad];
-  __shared__ double dto[kMW][64 * kPad];
+  constexpr int P = PAIRED ? 2 : 1;  // operands: sum and difference of a pair, or the ring
+  static_assert(64 * kPad >= MT * 2 * 16 * 16, "result tile fits");
+  __shared__ double dte[W][64 * kPad];
+  __shared__ double dto[W][64 * kPad];
   __shared__ lat::ChunkCoef ccs[2][lat::kChunk];  // recursion coefficients, double-buffered
-  const int m = m_of_block(blockIdx.x, a.nm, a.m_lo);
+  const int m = m_of_block(lat::balanced_block(blockIdx.x, gridDim.x), a.nm, a.m_lo);
   const int am = m < 0 ? -m : m;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int b0 = blockIdx.z * (MT * kTile);  // first map of the tile
@@ -89,40 +98,40 @@ __global__ void __launch_bounds__(kMT) lat_forward_f64_kernel(LatArgs a) {
   const int lzero = a.flm_packed ? am : 0;
   const int nz = lfirst - lzero;
   if (!a.accumulate && nz > 0) {
-    for (int e = threadIdx.x; e < MT * kTile * 2 * nz; e += kMT) {
-      const int bi = e / (2 * nz), r = e - bi * 2 * nz;
-      const int l = lzero + (r >> 1), comp = r & 1;
+    for (int e = threadIdx.x; e < MT * kTile * nz; e += (64 * W)) {
+      const int bi = e / nz, l = lzero + e - bi * nz;
       if (b0 + bi < a.batch) {
-        double* o = reinterpret_cast<double*>(out + (int64_t)bi * a.flm_map_stride + (int64_t)l * frow);
-        o[comp] = 0.0;
-        if (mirror) o[comp - 4 * m] = 0.0;  // flm[l, -m]: 2m complex columns to the left
+        cplx* o = out + (int64_t)bi * a.flm_map_stride + (int64_t)l * frow;
+        *o = {0.0, 0.0};
+        if (mirror) o[-2 * m] = {0.0, 0.0};  // flm[l, -m]: 2m columns to the left
       }
     }
   }
-  const int npass = (a.nrings + kMW * 64 - 1) / (kMW * 64);
+  const int npass = (a.nrings + SETS * W * 64 - 1) / (SETS * W * 64);
   for (int pass = 0; pass < npass; ++pass) {
     const bool first = pass == 0, last = pass + 1 == npass;
-    // recursion state: lane owns pair p = (pass * kMW + wave) * 64 + lane
-    const int base = (pass * kMW + wave) * 64;
-    double x = 0.0, d = 0.0, dm1 = 0.0;
-    int ls = 0;
-    if (base + lane < a.nrings) {
-      const LatRing rg = a.rings[base + lane];
-      x = rg.x;
-      lat::start_value_fp64(st, rg, d, ls);
-    }
+    // recursion state: lane owns pair base(s) + lane of each set
+    const auto base = [&](int s) { return ((pass * SETS + s) * W + wave) * 64; };
+    double x[SETS], d[SETS], dm1[SETS];
+    int ls[SETS];
     // A operands: tile t, row i = lane % 16 -> (map 8t + i/2, re/im i%2), pair base + 4c + lane/16.
     // The wave's ring rows are staged in LDS (its d tile is free here), then
     // the lane's components of rings ta and tb are gathered 8 pairs at a time
     // with all 16 loads in flight: branch-free, from clamped in-bounds
     // addresses, invalid entries zeroed afterwards (a load per conditional
     // branch would wait out one memory latency each).
-    double se[MT][16], so[MT][16];
-    {
+    double sv[SETS][MT][P][16];
+#pragma unroll
+    for (int s = 0; s < SETS; ++s) {
+      x[s] = d[s] = dm1[s] = 0.0;
+      ls[s] = 0;
       int2* rrows = reinterpret_cast<int2*>(de);  // (ta, tb), -1: absent
       int2 tt = {-1, -1};
-      if (base + lane < a.nrings) {
-        tt = *reinterpret_cast<const int2*>(&a.rings[base + lane].ta);
+      if (base(s) + lane < a.nrings) {
+        const LatRing rg = a.rings[base(s) + lane];
+        x[s] = rg.x;
+        lat::start_value_fp64(st, rg, d[s], ls[s]);
+        tt = *reinterpret_cast<const int2*>(&a.rings[base(s) + lane].ta);
         if (!PAIRED || tt.y < 0 || tt.y == tt.x) tt.y = -1;
       }
       rrows[lane] = tt;
@@ -143,14 +152,18 @@ __global__ void __launch_bounds__(kMT) lat_forward_f64_kernel(LatArgs a) {
 #pragma unroll
           for (int c = 0; c < 8; ++c) {
             va[c] = mcol[2 * spec_row(rq[c].x < 0 ? 0 : rq[c].x, a.ftm_ncol, TILED)];
-            vb[c] = mcol[2 * spec_row(rq[c].y < 0 ? 0 : rq[c].y, a.ftm_ncol, TILED)];
+            if (PAIRED) vb[c] = mcol[2 * spec_row(rq[c].y < 0 ? 0 : rq[c].y, a.ftm_ncol, TILED)];
           }
 #pragma unroll
           for (int c = 0; c < 8; ++c) {
             const double ca = have_map && rq[c].x >= 0 ? va[c] : 0.0;
-            const double cb = have_map && rq[c].y >= 0 ? vb[c] : 0.0;
-            se[t][c0 + c] = ca + cb;
-            so[t][c0 + c] = PAIRED ? ca - cb : ca;
+            if constexpr (PAIRED) {
+              const double cb = have_map && rq[c].y >= 0 ? vb[c] : 0.0;
+              sv[s][t][0][c0 + c] = ca + cb;
+              sv[s][t][1][c0 + c] = ca - cb;
+            } else {
+              sv[s][t][0][c0 + c] = ca;
+            }
           }
         }
       }
@@ -165,92 +178,84 @@ __global__ void __launch_bounds__(kMT) lat_forward_f64_kernel(LatArgs a) {
       const bool more = blk + 32 < L;
       if (more && threadIdx.x < lat::kChunk) cn = lat::load_ucoef_raw(cf, blk + 32, threadIdx.x, L);
       const lat::ChunkCoef* cs = ccs[buf];
-      acc_t acc_e[MT], acc_o[MT];
+      // this thread's elements: (tile, l = blk + 2 col + parity, map)
+      const int col = threadIdx.x & 15, omap = (threadIdx.x >> 4) & 7, opar = (threadIdx.x >> 7) & 1;
+      const int ot = threadIdx.x >> 8;  // first tile (eight waves: two at a time)
+      const int ol = blk + 2 * col + opar;
+      constexpr int TS = W / 4, NO = (MT + TS - 1) / TS;
+      cplx old[NO];
 #pragma unroll
-      for (int t = 0; t < MT; ++t) acc_e[t] = acc_o[t] = acc_t{0.0, 0.0, 0.0, 0.0};
-      const bool live = ls == 0;
-      // 32 steps: even offsets to one tile, odd to the other (zero past the
-      // band-limit: zero coefficients from l = L - 1 on); each 4-step group's
-      // coefficients are read from LDS while the previous group steps
-      double ca[4], cb[4], na[4], nb[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        ca[e] = cs[e].a;
-        cb[e] = cs[e].nb;
+      for (int t = 0; t < NO; ++t) {
+        const int bi = (t * TS + ot) * kTile + omap;
+        old[t] = {0.0, 0.0};
+        if ((!first || a.accumulate) && ol < L && t * TS + ot < MT && b0 + bi < a.batch)
+          old[t] = out[(int64_t)bi * a.flm_map_stride + (int64_t)ol * frow];
       }
+      acc_t acc[2][MT];
 #pragma unroll
-      for (int g = 0; g < 8; ++g) {
-        if (g < 7) {
+      for (int t = 0; t < MT; ++t) acc[0][t] = acc[1][t] = acc_t{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            na[e] = cs[4 * (g + 1) + e].a;
-            nb[e] = cs[4 * (g + 1) + e].nb;
-          }
-        }
+      for (int s = 0; s < SETS; ++s) {
+        if (base(s) >= a.nrings) break;  // the wave's remaining sets are empty
+        const bool live = ls[s] == 0;
+        // 32 steps: even offsets to one tile, odd to the other (zero past the
+        // band-limit: zero coefficients from l = L - 1 on)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int i = 4 * g + e;
-          const double v = live ? d : 0.0;
+        for (int i = 0; i < 32; ++i) {
+          const double v = live ? d[s] : 0.0;
           if (i & 1)
             dodd[lane * kPad + (i >> 1)] = v;
           else
             de[lane * kPad + (i >> 1)] = v;
-          const double dn = fma(fma(ca[e], x, cb[e]), d, -dm1);
-          dm1 = d;
-          d = dn;
+          const double dn = fma(fma(cs[i].a, x[s], cs[i].nb), d[s], -dm1[s]);
+          dm1[s] = d[s];
+          d[s] = dn;
         }
+        lat::rescale(d[s], dm1[s], ls[s]);
+        wave_sync();
+        // each d tile element (B operand) feeds the MT map tiles; even and odd
+        // products alternate, 2 MT accumulation chains in flight
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          ca[e] = na[e];
-          cb[e] = nb[e];
+        for (int c = 0; c < 16; ++c) {
+          const double be = de[(4 * c + kq) * kPad + row];
+          const double bo = dodd[(4 * c + kq) * kPad + row];
+#pragma unroll
+          for (int t = 0; t < MT; ++t) {
+            acc[0][t] = Mma<double>::run(sv[s][t][0][c], be, acc[0][t]);
+            acc[1][t] = Mma<double>::run(sv[s][t][P - 1][c], bo, acc[1][t]);
+          }
         }
+        wave_sync();
       }
-      wave_sync();
-      // each d tile element (B operand) feeds the MT map tiles; even and odd
-      // products alternate, 2 MT accumulation chains in flight
-#pragma unroll
-      for (int c = 0; c < 16; ++c) {
-        const double be = de[(4 * c + kq) * kPad + row];
-        const double bo = dodd[(4 * c + kq) * kPad + row];
-#pragma unroll
-        for (int t = 0; t < MT; ++t) {
-          acc_e[t] = Mma<double>::run(se[t][c], be, acc_e[t]);
-          acc_o[t] = Mma<double>::run(so[t][c], bo, acc_o[t]);
-        }
-      }
-      wave_sync();
-      lat::rescale(d, dm1, ls);
       // the wave's sums: [tile][parity][row][col] over the (now free) even tile
 #pragma unroll
       for (int t = 0; t < MT; ++t) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int i = Mma<double>::row_of(r, kq);
-          ctw[t * 512 + i * 16 + row] = acc_e[t][r];
-          ctw[t * 512 + 256 + i * 16 + row] = acc_o[t][r];
+          ctw[t * 512 + i * 16 + row] = acc[0][t][r];
+          ctw[t * 512 + 256 + i * 16 + row] = acc[1][t][r];
         }
       }
       if (more && threadIdx.x < lat::kChunk) ccs[buf ^ 1][threadIdx.x] = lat::finish_coef(cn, bsign);
       __syncthreads();
-      // sum the waves in a fixed order; element (tile, parity, row, col) ->
-      // l = blk + 2 col + parity, map b0 + 8 tile + row/2, component row%2.
-      // Thread e owns element e in every pass and chunk.
-      for (int e = threadIdx.x; e < MT * 512; e += kMT) {
-        const int t = e >> 9, par = (e >> 8) & 1, rr = (e >> 4) & 15, col = e & 15;
-        const int l = blk + 2 * col + par;
-        const int bi = t * kTile + (rr >> 1);
-        if (l < L && b0 + bi < a.batch) {
-          double v = dte[0][e];
+      // sum the waves in a fixed order; thread e owns its element of each map
+      // tile in every pass and chunk
 #pragma unroll
-          for (int w = 1; w < kMW; ++w) v += dte[w][e];
-          v *= cs[2 * col + par].c;  // sigma_l: e_l -> d_l
-          double* o = reinterpret_cast<double*>(out + (int64_t)bi * a.flm_map_stride +
-                                                (int64_t)l * frow) + (rr & 1);
-          if (l < a.lmin_out) v = 0.0;
-          if (!first || a.accumulate) v += *o;
+      for (int t = 0; t < NO; ++t) {
+        const int tile = t * TS + ot, bi = tile * kTile + omap;
+        if (ol < L && tile < MT && b0 + bi < a.batch) {
+          const int e = tile * 512 + opar * 256 + omap * 32 + col;
+          cplx v = {dte[0][e], dte[0][e + 16]};
+#pragma unroll
+          for (int w = 1; w < W; ++w) v = {v.x + dte[w][e], v.y + dte[w][e + 16]};
+          const double sigma = cs[2 * col + opar].c;  // e_l -> d_l
+          v = ol < a.lmin_out ? cplx{0.0, 0.0} : cplx{sigma * v.x, sigma * v.y};
+          v = cadd(v, old[t]);
+          cplx* o = out + (int64_t)bi * a.flm_map_stride + (int64_t)ol * frow;
           *o = v;
-          // flm[l, -m] = (-1)^m conj(flm[l, m]), 2m complex columns to the left
-          if (last && mirror) o[-4 * m] = (rr & 1) ? -msgn * v : msgn * v;
+          // flm[l, -m] = (-1)^m conj(flm[l, m]), 2m columns to the left
+          if (last && mirror) o[-2 * m] = {msgn * v.x, -msgn * v.y};
         }
       }
       __syncthreads();
@@ -414,25 +419,29 @@ static hipError_t lat_fwd_f32(const LatArgs& a0, bool paired, hipStream_t s) {
   return hipGetLastError();
 }
 
-template <int MT>
-static hipError_t lat_fwd_f64(const LatArgs& a, bool paired, hipStream_t s) {
+template <int W, int MT, int SETS, bool PAIRED>
+static hipError_t lat_fwd_f64(const LatArgs& a, hipStream_t s) {
   dim3 grid(a.nm, 1, (a.batch + MT * kTile - 1) / (MT * kTile));
-  if (paired && a.ftm_tiled)
-    hipLaunchKernelGGL((lat_forward_f64_kernel<MT, true, true>), grid, dim3(kMT), 0, s, a);
-  else if (paired)
-    hipLaunchKernelGGL((lat_forward_f64_kernel<MT, true, false>), grid, dim3(kMT), 0, s, a);
-  else if (a.ftm_tiled)
-    hipLaunchKernelGGL((lat_forward_f64_kernel<MT, false, true>), grid, dim3(kMT), 0, s, a);
+  if (a.ftm_tiled)
+    hipLaunchKernelGGL((lat_forward_f64_kernel<W, MT, SETS, PAIRED, true>), grid, dim3(64 * W), 0, s, a);
   else
-    hipLaunchKernelGGL((lat_forward_f64_kernel<MT, false, false>), grid, dim3(kMT), 0, s, a);
+    hipLaunchKernelGGL((lat_forward_f64_kernel<W, MT, SETS, PAIRED, false>), grid, dim3(64 * W), 0, s, a);
   return hipGetLastError();
 }
 
 hipError_t launch_lat_forward_mfma(const LatArgs& a, bool paired, bool fp32, hipStream_t s) {
   if (a.nm == 0 || a.nrings == 0 || a.batch == 0) return hipSuccess;
   if (fp32) return lat_fwd_f32(a, paired, s);
-  // FP64: 16-map tiles from 9 maps on, 8-map tiles below
-  return a.batch > kTile ? lat_fwd_f64<2>(a, paired, s) : lat_fwd_f64<1>(a, paired, s);
+  // FP64: 16-map tiles from 9 maps on
+  const bool wide = a.batch > kTile;
+  const int sets = (a.nrings + 255) / 256;  // of 64 rings per wave, four waves
+  if (paired) {
+    if (sets > 1) return wide ? lat_fwd_f64<8, 2, 1, true>(a, s) : lat_fwd_f64<8, 1, 1, true>(a, s);
+    return wide ? lat_fwd_f64<4, 2, 1, true>(a, s) : lat_fwd_f64<4, 1, 1, true>(a, s);
+  }
+  if (wide) return sets > 1 ? lat_fwd_f64<4, 2, 2, false>(a, s) : lat_fwd_f64<4, 2, 1, false>(a, s);
+  if (sets > 2) return lat_fwd_f64<4, 1, 4, false>(a, s);
+  return sets > 1 ? lat_fwd_f64<4, 1, 2, false>(a, s) : lat_fwd_f64<4, 1, 1, false>(a, s);
 }
 
 // One V_MFMA_F64_16X16X4F64 on caller-provided operands, for checking the

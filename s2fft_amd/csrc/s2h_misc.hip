@@ -46,7 +46,8 @@ __global__ void __launch_bounds__(kThreads) pole_forward_kernel(PoleArgs a) {
   if (a.row_south >= 0) {
     const int c = spin - a.ftm_m_first;
     if (c >= 0 && c < a.ftm_ncol) {
-      const cplx v = base[(int64_t)a.row_south * a.ftm_ncol + c];
+      const cplx v = base[spec_row(a.row_south, a.ftm_ncol, a.ftm_tiled) +
+                          c * spec_cstride(a.ftm_tiled)];
       const double s = ((l - spin) & 1) ? -w : w;
       cplx* o = f + (a.L - 1 + spin);
       o->x += s * v.x;
@@ -56,7 +57,8 @@ __global__ void __launch_bounds__(kThreads) pole_forward_kernel(PoleArgs a) {
   if (a.row_north >= 0) {
     const int c = -spin - a.ftm_m_first;
     if (c >= 0 && c < a.ftm_ncol) {
-      const cplx v = base[(int64_t)a.row_north * a.ftm_ncol + c];
+      const cplx v = base[spec_row(a.row_north, a.ftm_ncol, a.ftm_tiled) +
+                          c * spec_cstride(a.ftm_tiled)];
       cplx* o = f + (a.L - 1 - spin);
       o->x += w * v.x;
       o->y += w * v.y;

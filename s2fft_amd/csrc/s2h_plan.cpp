@@ -571,7 +571,7 @@ static int plan_build(s2h_plan* p) {
     // the theta operators' output: MWSS at L, rows 0..L, poles at 0 and L; the
     // operators absorb the rounding of the rows' cosines (delta)
     p->fwd_kind = d.sampling == S2H_MW ? 1 : 2;
-    p->fwd_rows = L + 1;
+    p->fwd_rows = (L + 1 + kSpecBlock - 1) / kSpecBlock * kSpecBlock;  // whole blocks
     std::vector<double> xs, delta(L + 1, 0.0);
     for (int t = 0; t <= L; ++t) xs.push_back(mwss_cos(t, L));
     for (int t = 1; t < L; ++t)

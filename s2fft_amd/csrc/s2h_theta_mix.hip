@@ -377,6 +377,7 @@ struct MixKernelArgs {
   int L, K, R;              // input rows, output rows
   int KT, KTpad, RT;        // K-steps in use, K-steps / row tiles of the packed operator
   int in_poles, out_poles;  // rows in mix_row order
+  int out_tiled;            // out in blocks of 8 rows (spec_row)
   int row_blocks, col_blocks;
 };
 
@@ -493,11 +494,201 @@ __global__ void __launch_bounds__(256) theta_mix_kernel(MixKernelArgs a) {
         if (col < a.ncol) {
           double v = acc[mt][nt][r];
           if (term) v = fma(pr, vv[nt], v);
-          ob[2 * ((int64_t)row * a.ncol + col)] = v;
+          ob[2 * (spec_row(row, a.ncol, a.out_tiled) + col * spec_cstride(a.out_tiled))] = v;
         }
       }
     }
   }
+}
+
+// The same product for launches that fill the card: operator and spectra pass
+// through LDS, so that the four waves of a workgroup (two column parities, two
+// column halves) share what they load and the matrix cores, not the L1's 64 bytes
+// per cycle, set the pace.  One workgroup: 64 rows of both parities x 64 columns;
+// a wave 4 row tiles x 2 column tiles; 16 input rows per LDS chunk, double-buffered
+// through registers (64 KB: two workgroups per CU).  The spectra are staged by
+// parity, (re, im) of 32 columns per input row, rows 640 bytes apart so that the two
+// rows of a half wave use all banks.  At MW L = 512, 64 maps the matrix cores are busy
+// for 68 % of its 1550 us (loads one chunk ahead instead of two: 2140 us).
+constexpr int kMixRows = 64, kMixCols = 64, kMixK = 16;
+constexpr int kMixPad = 80;  // doubles per staged row of one parity
+
+template <bool VFULL>
+__global__ void __launch_bounds__(256, 2) theta_mix_lds_kernel(MixKernelArgs a) {
+  constexpr int MT = 4, NT = 2, KS = kMixK / 4;
+  __shared__ __attribute__((aligned(16))) double as[2][2][MT][KS][64];  // [buffer][parity][tile][step]
+  __shared__ __attribute__((aligned(16))) double bs[2][2][kMixK][kMixPad];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int j = lane & 15, kq = lane >> 4, comp = j & 1;
+  const int seq = blockIdx.x >> 3;
+  const int rb = seq % a.row_blocks;
+  const int cb = (seq / a.row_blocks) * 8 + (blockIdx.x & 7);
+  if (cb >= a.col_blocks) return;
+  const int b = blockIdx.y;
+  const int par = wave & 1, half = wave >> 1;
+  const int spin = a.spin + a.spin_step * b;
+  const int c0 = cb * kMixCols, r0 = rb * kMixRows;
+  if (a.out_poles && r0 >= a.L - 1) {
+    // pole rows only: the pole terms read the columns m = +-spin
+    const int cs = spin - a.m_lo, cn = -spin - a.m_lo;
+    if (!(cs >= c0 && cs < c0 + kMixCols) && !(cn >= c0 && cn < c0 + kMixCols)) return;
+  }
+  const int off = (a.m_lo + spin) & 1;  // parity of column c0 (c0 is even)
+  const cplx* in = a.in + (int64_t)b * a.in_map_stride;
+
+  // staging: 4 columns' values and 8 operator values per thread and chunk.  Column
+  // c0 + c (c = tid % 64) goes to parity (c + off) % 2, place c / 2; the input rows
+  // tid / 64 + 4 i.
+  const int sc = tid & 63, sr = tid >> 6;
+  const int scol = c0 + sc < a.ncol ? c0 + sc : a.ncol - 1;  // in bounds; not stored
+  struct Staged {
+    cplx b[4];
+    double2 a[4];
+  };
+  // addresses: a uniform base per load plus the thread's own offset.  Input rows up to
+  // `plain` follow their index (with poles: one further); the rest go through mix_at
+  const int plain = a.in_poles ? a.L - 1 : a.K;
+  const unsigned boff = 16u * (unsigned)(sr * a.ncol + scol);
+  unsigned aoff[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    // tile of element tid + 256 i of a parity's [tile][step][64] pairs; tiles past the
+    // operator's: the last again, not stored
+    const int mt = 2 * i + (tid >> 7), rt = rb * MT + mt < a.RT ? rb * MT + mt : a.RT - 1;
+    aoff[i] = 8u * (unsigned)(rt * a.KTpad * 64 + 2 * (tid & 127));
+  }
+  const auto load = [&](int kc, Staged& v) {
+    if ((kc + 1) * kMixK <= plain) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const cplx* base = in + (int64_t)(kc * kMixK + 4 * i + (a.in_poles ? 1 : 0)) * a.ncol;
+        v.b[i] = *reinterpret_cast<const cplx*>(reinterpret_cast<const char*>(base) + boff);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int k = kc * kMixK + sr + 4 * i;
+        v.b[i] = in[(int64_t)mix_at(k < a.K ? k : a.K - 1, a.L, a.in_poles) * a.ncol + scol];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const double* base = a.mat + ((int64_t)(i >> 1) * a.RT * a.KTpad + kc * KS) * 64;
+      v.a[i] = *reinterpret_cast<const double2*>(reinterpret_cast<const char*>(base) + aoff[i & 1]);
+    }
+  };
+  double* bst = &bs[0][(sc + off) & 1][sr][2 * (sc >> 1)];
+  double2* ast = reinterpret_cast<double2*>(&as[0][0][0][0][0]) + tid;
+  const auto stage = [&](int kc, const Staged& v) {
+    const int buf = kc & 1;
+    const bool whole = (kc + 1) * kMixK <= a.K;  // else zero past K, as the operator is
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const bool in_k = whole || kc * kMixK + sr + 4 * i < a.K;
+      *reinterpret_cast<cplx*>(bst + buf * (2 * kMixK * kMixPad) + 4 * i * kMixPad) =
+          cplx{in_k ? v.b[i].x : 0.0, in_k ? v.b[i].y : 0.0};
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) ast[buf * (2 * MT * KS * 32) + 256 * i] = v.a[i];
+  };
+
+  lat::v4d acc[MT][NT], accv[NT];
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) {
+    accv[nt] = lat::v4d{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) acc[mt][nt] = lat::v4d{0.0, 0.0, 0.0, 0.0};
+  }
+  const bool full = VFULL && a.vmode[par] == 2;
+  const double* qv = a.q + par * a.K;
+  const int chunks = (a.K + kMixK - 1) / kMixK;
+  const auto products = [&](int kc) {
+    const int buf = kc & 1;
+#pragma unroll
+    for (int u = 0; u < KS; ++u) {
+      double ca[MT], cbv[NT];
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) ca[mt] = as[buf][par][mt][u][lane];
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) cbv[nt] = bs[buf][par][4 * u + kq][(half * NT + nt) * 16 + j];
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+          acc[mt][nt] = lat::Mma<double>::run(ca[mt], cbv[nt], acc[mt][nt]);
+      if (full) {
+        const int k = kc * kMixK + 4 * u + kq;
+        const double cq = k < a.K ? qv[mix_at(k, a.L, a.in_poles)] : 0.0;
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) accv[nt] = lat::Mma<double>::run(cq, cbv[nt], accv[nt]);
+      }
+    }
+  };
+  // loads run two chunks ahead of the products, LDS one (past the end: the last
+  // chunk again, unused)
+  Staged va, vb;
+  load(0, va);
+  load(min(1, chunks - 1), vb);
+  stage(0, va);
+  __syncthreads();
+  for (int kc = 0; kc < chunks; kc += 2) {
+    load(min(kc + 2, chunks - 1), va);
+    products(kc);
+    stage(kc + 1, vb);
+    __syncthreads();
+    if (kc + 1 >= chunks) break;
+    load(min(kc + 3, chunks - 1), vb);
+    products(kc + 1);
+    stage(kc + 2, va);
+    __syncthreads();
+  }
+
+  // rank-one term: every row of accv holds v; sparse q reads its two rows
+  const bool term = a.p && a.vmode[par] != 0;
+  int col[NT];
+  double vv[NT];
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) {
+    // place 8 (2 half + nt) + j / 2 of the parity
+    col[nt] = c0 + 2 * ((half * NT + nt) * 8 + (j >> 1)) + ((par + off) & 1);
+    vv[nt] = accv[nt][0];
+    if (term && !full) {
+      const double* bp = reinterpret_cast<const double*>(in + (col[nt] < a.ncol ? col[nt] : 0)) + comp;
+      vv[nt] = qv[0] * bp[0] + qv[a.K - 1] * bp[2 * (int64_t)(a.K - 1) * a.ncol];
+    }
+    // i v: the real part takes -Im v, the imaginary part Re v
+    vv[nt] = a.sgn * (comp ? 1.0 : -1.0) * __shfl_xor(vv[nt], 1);
+  }
+  double* ob = reinterpret_cast<double*>(a.out + (int64_t)b * a.out_map_stride) + comp;
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = r0 + 16 * mt + lat::Mma<double>::row_of(r, kq);
+      if (i >= a.R) continue;
+      const int row = mix_at(i, a.L, a.out_poles);
+      const double pr = term ? a.p[par * a.R + row] : 0.0;
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) {
+        if (col[nt] < a.ncol) {
+          double v = acc[mt][nt][r];
+          if (term) v = fma(pr, vv[nt], v);
+          ob[2 * (spec_row(row, a.ncol, a.out_tiled) + col[nt] * spec_cstride(a.out_tiled))] = v;
+        }
+      }
+    }
+  }
+}
+
+hipError_t mix_launch_lds(MixKernelArgs k, int batch, hipStream_t s) {
+  k.row_blocks = (k.R + kMixRows - 1) / kMixRows;
+  k.col_blocks = (k.ncol + kMixCols - 1) / kMixCols;
+  const unsigned gx = (unsigned)(8 * k.row_blocks * ((k.col_blocks + 7) / 8));
+  if (k.p && (k.vmode[0] == 2 || k.vmode[1] == 2))
+    hipLaunchKernelGGL(theta_mix_lds_kernel<true>, dim3(gx, batch), dim3(256), 0, s, k);
+  else
+    hipLaunchKernelGGL(theta_mix_lds_kernel<false>, dim3(gx, batch), dim3(256), 0, s, k);
+  return hipGetLastError();
 }
 
 template <int MT, int NT, int D>
@@ -528,6 +719,7 @@ hipError_t launch_theta_mix(const ThetaMix* x, const ThetaMixArgs& a, int batch,
   k.KT = (k.K + 3) / 4;
   k.in_poles = a.adjoint;
   k.out_poles = !a.adjoint;
+  k.out_tiled = a.out_tiled;
   k.in = a.in;
   k.in_map_stride = a.in_map_stride;
   k.out = a.out;
@@ -544,15 +736,17 @@ hipError_t launch_theta_mix(const ThetaMix* x, const ThetaMixArgs& a, int batch,
     k.vmode[0] = x->mw ? 0 : 2;
     k.vmode[1] = a.adjoint ? 2 : 1;
   }
-  // 2 x 2 tiles from 1536 waves on (2 parities x 32 rows x 32 columns x maps),
-  // below that single tiles: at L = 193, 3 maps 23 us with 1950 single-tile
-  // waves.  The loads bound it, not the products: 4 x 4 tiles (two waves per
-  // SIMD) took 2.16 ms at L = 512, 64 maps where 2 x 2 take 1.65, 2 x 4 1.60
-  // and 4 x 2 1.72.
+  // Through LDS from 4096 waves of 4 x 2 tiles on (MW L = 512, 64 maps 1550 us against
+  // 1690 with 2 x 2 tiles from registers, MWSS L = 512, spin 2, 16 maps 564 against 698,
+  // MW 512 / 8, 4608 waves, 246 against 257; with fewer it starves: MW 512 / 3 124
+  // against 112, MW 256 / 4 45 against 23); 2 x 2 tiles from 1536 waves on (2 parities
+  // x 32 rows x 32 columns x maps), below that single tiles: at L = 193, 3 maps 23 us
+  // with 1950 single-tile waves.
   const auto waves = [&](int mt, int nt) {
     return (int64_t)batch * 2 * ((k.R + 16 * mt - 1) / (16 * mt)) *
            ((k.ncol + 16 * nt - 1) / (16 * nt));
   };
+  if (waves(4, 2) >= 4096) return mix_launch_lds(k, batch, s);
   if (waves(2, 2) >= 1536) return mix_launch<2, 2, 4>(k, batch, s);
   return mix_launch<1, 1, 8>(k, batch, s);
 }
