@@ -90,11 +90,11 @@ def inverse(flm, L, spin=0, kernel=None, sampling="mw", reality=False, method="h
     reality = _common(method, spin, reality)
     t, restore = sph._as_device_tensor(flm, complex_only=True)
     tb, batched = sph._split_batch(t, s2_samples.flm_shape(L), "flm")
-    with torch.cuda.device(tb.device):
+    with sph._on_device(tb.device):
         if kernel is None:
             kernel = construct.spin_spherical_kernel(L, spin, reality, sampling, nside, False)
         f = inverse_transform_hip(tb, kernel, L, sampling, reality, spin, nside)
-    return restore(f if batched else f[0])
+    return restore(f if batched else f.squeeze(0))
 
 
 def forward(f, L, spin=0, kernel=None, sampling="mw", reality=False, method="hip", nside=None,
@@ -105,7 +105,7 @@ def forward(f, L, spin=0, kernel=None, sampling="mw", reality=False, method="hip
     reality = _common(method, spin, reality)
     t, restore = sph._as_device_tensor(f)
     tb, batched = sph._split_batch(t, s2_samples.f_shape(L, sampling, nside), "f")
-    with torch.cuda.device(tb.device):
+    with sph._on_device(tb.device):
         if kernel is None:
             kernel = construct.spin_spherical_kernel(L, spin, reality, sampling, nside, True)
         flm = forward_transform_hip(tb, kernel, L, sampling, reality, spin, nside)
@@ -117,4 +117,4 @@ def forward(f, L, spin=0, kernel=None, sampling="mw", reality=False, method="hip
                     rec = rec.real
                 flm = flm + forward_transform_hip(tb - rec, kernel, L, sampling, reality, spin,
                                                   nside)
-    return restore(flm if batched else flm[0])
+    return restore(flm if batched else flm.squeeze(0))

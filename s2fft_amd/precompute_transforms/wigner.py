@@ -43,7 +43,7 @@ def inverse(flmn, L, N, kernel=None, sampling="mw", reality=False, method="hip",
     _check(method)
     s = sampling.lower()
     t, restore = sph._as_device_tensor(flmn, complex_only=True)
-    with torch.cuda.device(t.device):
+    with sph._on_device(t.device):
         K = _kernel(kernel, L, N, s, nside, reality, False, t.device)
         fshape = so3_samples.f_shape(L, N, s, nside)
         npix = int(np.prod(fshape[1:]))
@@ -71,7 +71,7 @@ def forward(f, L, N, kernel=None, sampling="mw", reality=False, method="hip", ns
     _check(method)
     s = sampling.lower()
     t, restore = sph._as_device_tensor(f)
-    with torch.cuda.device(t.device):
+    with sph._on_device(t.device):
         K = _kernel(kernel, L, N, s, nside, reality, True, t.device)
         G = 2 * N - 1
         npix = t[0].numel()

@@ -10,6 +10,7 @@ tensors (the result stays on the tensor's device); a leading batch axis is
 accepted and transformed in one launch per kernel.
 """
 
+import contextlib
 import ctypes
 import threading
 
@@ -71,13 +72,26 @@ def _as_device_tensor(x, complex_only=False):
 
 
 def _stream(device):
-    return torch.cuda.current_stream(device).cuda_stream
+    """The current stream's handle, without a Stream object (2 us a call)."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None
+                                              else index)
+
+
+_HERE = contextlib.nullcontext()
+
+
+def _on_device(device):
+    """torch.cuda.device(device), entered only where it is not the current one."""
+    index = device.index
+    return _HERE if index is None or index == torch.cuda.current_device() \
+        else torch.cuda.device(index)
 
 
 def _split_batch(t, core_shape, what):
     core = tuple(core_shape)
     if tuple(t.shape) == core:
-        return t.reshape((1,) + core), False
+        return t.unsqueeze(0), False
     if t.dim() == len(core) + 1 and tuple(t.shape[1:]) == core:
         return t, True
     raise ValueError(f"{what} has shape {tuple(t.shape)}, expected {core} or (batch,) + {core}")
@@ -527,9 +541,9 @@ def inverse(flm, L, spin=0, nside=None, sampling="mw", method="hip", reality=Fal
     _check_common(method, spin, sampling, nside)
     t, restore = _as_device_tensor(flm, complex_only=True)
     tb, batched = _split_batch(t, samples.flm_shape(L), "flm")
-    with torch.cuda.device(tb.device):
+    with _on_device(tb.device):
         f = inverse_diff(tb, L, spin, nside, sampling, reality, L_lower)
-    return restore(f if batched else f[0])
+    return restore(f if batched else f.squeeze(0))
 
 
 def forward(f, L, spin=0, nside=None, sampling="mw", method="hip", reality=False,
@@ -544,6 +558,6 @@ def forward(f, L, spin=0, nside=None, sampling="mw", method="hip", reality=False
         iter = 0
     t, restore = _as_device_tensor(f)
     tb, batched = _split_batch(t, samples.f_shape(L, sampling, nside), "f")
-    with torch.cuda.device(tb.device):
+    with _on_device(tb.device):
         flm = forward_iterative_hip(tb, L, spin, nside, sampling, reality, L_lower, iter)
-    return restore(flm if batched else flm[0])
+    return restore(flm if batched else flm.squeeze(0))

@@ -201,7 +201,7 @@ def inverse(flmn, L, N, nside=None, sampling="mw", method="hip", reality=False,
     """SO(3) inverse (s2fft/transforms/wigner.py:13-107)."""
     _check(method, N)
     t, restore = sph._as_device_tensor(flmn, complex_only=True)
-    with torch.cuda.device(t.device):
+    with sph._on_device(t.device):
         f = inverse_diff(t, L, N, nside, sampling, reality, L_lower)
     return restore(f)
 
@@ -211,6 +211,6 @@ def forward(f, L, N, nside=None, sampling="mw", method="hip", reality=False,
     """SO(3) forward (s2fft/transforms/wigner.py:346-439)."""
     _check(method, N)
     t, restore = sph._as_device_tensor(f)
-    with torch.cuda.device(t.device):
+    with sph._on_device(t.device):
         flmn = forward_diff(t, L, N, nside, sampling, reality, L_lower)
     return restore(flmn)
