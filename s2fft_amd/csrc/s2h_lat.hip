@@ -139,7 +139,7 @@ lat_inverse_kernel(LatArgs a) {
   __shared__ cplx fs[2][NB][kChunk];
   int g;
   const int m = lat::m_group_of_block(lat::balanced_block(blockIdx.x, gridDim.x), a.nm, a.groups,
-                                      a.m_lo, g);
+                                      a.m_lo, g, 4);
   const int am = m < 0 ? -m : m;
   const int tid = threadIdx.x, nthr = blockDim.x;
   const int b0 = blockIdx.z * NB;
@@ -328,7 +328,7 @@ lat_forward_kernel(LatArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char fwd_raw[];
   __shared__ StepCoef<PAIRED> cs[2][kChunk];
   __shared__ double sg[2][kChunk];
-  const int m = lat::m_of_block(lat::balanced_block(blockIdx.x, gridDim.x), a.nm, a.m_lo);
+  const int m = lat::m_of_block(lat::balanced_block(blockIdx.x, gridDim.x), a.nm, a.m_lo, 4);
   const int am = m < 0 ? -m : m;
   const int64_t b = blockIdx.z;
   const int tid = threadIdx.x, nthr = blockDim.x, lane = tid & 63, wave = tid >> 6;

@@ -139,15 +139,22 @@ __device__ __forceinline__ int balanced_block(int i, int n) {
   return ((j >> 5) & 1) && (j | 31) < (n >> 3) ? ((j ^ 31) << 3) | (i & 7) : i;
 }
 
-// blockIdx.x -> m: 4 adjacent m per XCD in a row (workgroups are dealt to the
-// 8 XCDs round-robin), heaviest (smallest |m|) first.  For m_lo < 0 the order
-// is 0, -1, 1, -2, 2, ...
-__device__ __forceinline__ int m_of_block(int i, int nm, int m_lo) {
-  const int nfull = nm & ~31;  // the remap is a bijection on [0, nfull)
+// blockIdx.x -> m: c adjacent m per XCD in a row (workgroups are dealt to the
+// 8 XCDs round-robin), heaviest (smallest |m|) first, every second row over the
+// XCDs in reverse.  For m_lo < 0 the order is 0, -1, 1, -2, 2, ...: two runs of c / 2
+// columns, and the matrix-core kernels, bound by their 16-byte accesses to the
+// spectra, take c = 16 so that an XCD's L2 sees whole lines (MW L = 512, spin 2, 64
+// maps: BF16 inverse, which wrote 1.05 GB for 0.54 GB of spectra, 825 us with c = 4,
+// 735 with 16; HEALPix L = 512, spin 2, 16 maps, forward 660 and 620); 4 spread the
+// work more evenly (VALU forward, GL L = 400, spin 1, 3 maps 97 us and 100).
+__device__ __forceinline__ int m_of_block(int i, int nm, int m_lo, int cfull = 16) {
+  const int c = m_lo == 0 ? 4 : cfull;
+  const int nfull = nm & ~(8 * c - 1);  // the remap is a bijection on [0, nfull)
   int idx = i;
   if (i < nfull) {
-    const int xcd = i & 7, k = i >> 3;
-    idx = ((k >> 2) << 5) + (xcd << 2) + (k & 3);
+    const int k = i >> 3, r = k / c;
+    const int xcd = r & 1 ? 7 - (i & 7) : i & 7;
+    idx = r * 8 * c + xcd * c + k % c;
   }
   if (m_lo == 0) return idx;
   return (idx & 1) ? -((idx + 1) >> 1) : (idx >> 1);
@@ -159,7 +166,8 @@ __device__ __forceinline__ int m_of_block(int i, int nm, int m_lo) {
 // of one m are consecutive blocks of one XCD.  They run together and read the
 // m's harmonic and recursion coefficients through that XCD's L2, not HBM.  The m-values
 // follow m_of_block.  A bijection of [0, nm G) onto [0, nm) x [0, G).
-__device__ __forceinline__ int m_group_of_block(int i, int nm, int G, int m_lo, int& g) {
+__device__ __forceinline__ int m_group_of_block(int i, int nm, int G, int m_lo, int& g,
+                                                int cfull = 16) {
   const int nm8 = nm & ~7;
   int ip;
   if (i < nm8 * G) {
@@ -173,7 +181,7 @@ __device__ __forceinline__ int m_group_of_block(int i, int nm, int G, int m_lo, 
     g = r - k * G;
     ip = nm8 + k;
   }
-  return m_of_block(ip, nm, m_lo);
+  return m_of_block(ip, nm, m_lo, cfull);
 }
 
 // Recursion coefficients of one 32-step chunk, staged in LDS so that every
