@@ -225,6 +225,10 @@ int ring_analysis_stage(const s2h_plan* p, const void* f, int f_is_complex, cplx
   // carries both)
   r.apply_weight = resample || raw ? 0 : 1;
   r.apply_phase = !raw && p->d.sampling == S2H_HEALPIX;
+  if (out_map_stride > 0) {  // ring spectra of the C ABI: zero padding rows
+    r.pad_row0 = p->fwd_rows;
+    r.pad_rows = p->spec_rows - p->fwd_rows;
+  }
   r.zero_neg_2L = 0;
   r.L = p->d.L;
   r.chirp_pool = p->chirp;
@@ -242,6 +246,19 @@ struct SpecView {
   int64_t map_stride;
   int tiled;
 };
+
+// map stride of the C ABI's ring spectra (rows padded to whole row blocks)
+int64_t spec_stride(const s2h_plan* p) { return (int64_t)p->spec_rows * p->Mc; }
+SpecView spec_view(const s2h_plan* p, int flags) {
+  return SpecView{spec_stride(p), (flags & S2H_SPECTRA_TILED) ? 1 : 0};
+}
+// zeros into the padding rows of C-ABI spectra the call wrote.  The ring FFTs, the VALU
+// synthesis and the ring-major residual write them along (HEALPix nside 192, 5 maps,
+// forward with 3 iterations: seven launches fewer, 540 -> 509 us)
+int zero_spec_pad(const s2h_plan* p, void* spec, int tiled, int batch, hipStream_t s) {
+  return hip_status(launch_spec_pad_zero(static_cast<cplx*>(spec), spec_stride(p), p->Mc,
+                                         p->fwd_rows, p->spec_rows, tiled, batch, s));
+}
 
 int lat_forward_stage(const s2h_plan* p, const cplx* ftm, void* flm, int batch, int precision,
                       bool accumulate, hipStream_t s, bool packed = false,
@@ -359,6 +376,8 @@ int lat_inverse_stage(const s2h_plan* p, const void* flm, cplx* ftm, int batch, 
       v.flm += (int64_t)(batch - nv) * a.flm_map_stride;
       v.ftm += (int64_t)(batch - nv) * a.ftm_map_stride;
       v.pole = lat_pole(p, false, false, ps);
+      v.pad_row0 = p->fwd_rows;
+      v.pad_rows = sv ? p->spec_rows - p->fwd_rows : 0;
       st = hip_status(launch_lat_inverse(v, ps ? false : p->inv_paired, s));
       batch -= nv;
       a.batch = batch;
@@ -371,6 +390,7 @@ int lat_inverse_stage(const s2h_plan* p, const void* flm, cplx* ftm, int batch, 
       st = hip_status(launch_lat_inverse_mma(a, p->inv_paired, mixed, s));
     if (st) return st;
   }
+  if (sv) return zero_spec_pad(p, ftm, sv->tiled, batch, s);  // no pole rows there
 
   if (p->inv_row_south >= 0 || p->inv_row_north >= 0) {
     PoleArgs pa{};
@@ -523,19 +543,6 @@ extern "C" int s2h_inverse_ex(const s2h_plan* p, const void* flm, void* f, void*
 // The transforms split at the ring spectra, for refinement in spectral space:
 // F(f - I(x)) = Lat_fwd(G - A(Lat_inv(x))) with G the ring spectra of f and A
 // the ring FFT of the ring iFFT, applied without either FFT.
-namespace {
-// map stride of the C ABI's ring spectra (rows padded to whole row blocks)
-int64_t spec_stride(const s2h_plan* p) { return (int64_t)p->spec_rows * p->Mc; }
-SpecView spec_view(const s2h_plan* p, int flags) {
-  return SpecView{spec_stride(p), (flags & S2H_SPECTRA_TILED) ? 1 : 0};
-}
-// zeros into the padding rows of C-ABI spectra the call wrote
-int zero_spec_pad(const s2h_plan* p, void* spec, int tiled, int batch, hipStream_t s) {
-  return hip_status(launch_spec_pad_zero(static_cast<cplx*>(spec), spec_stride(p), p->Mc,
-                                         p->fwd_rows, p->spec_rows, tiled, batch, s));
-}
-}  // namespace
-
 extern "C" size_t s2h_ring_spectra_bytes(const s2h_plan* p, int batch) {
   if (!p || batch < 0 || !spectral_ok(p)) return 0;
   return (size_t)batch * (size_t)spec_stride(p) * sizeof(cplx);
@@ -548,10 +555,8 @@ extern "C" int s2h_ring_analysis(const s2h_plan* p, const void* f, int f_is_comp
   if (batch == 0) return S2H_OK;
   int st = check_device(p);
   if (st) return st;
-  if ((st = ring_analysis_stage(p, f, f_is_complex, static_cast<cplx*>(G), batch,
-                                static_cast<hipStream_t>(stream), false, spec_stride(p))))
-    return st;
-  return zero_spec_pad(p, G, 0, batch, static_cast<hipStream_t>(stream));
+  return ring_analysis_stage(p, f, f_is_complex, static_cast<cplx*>(G), batch,
+                             static_cast<hipStream_t>(stream), false, spec_stride(p));
 }
 
 extern "C" int s2h_forward_rings(const s2h_plan* p, const void* G, void* flm, int batch,
@@ -584,10 +589,8 @@ extern "C" int s2h_inverse_rings(const s2h_plan* p, const void* flm, void* Y, in
   int st = check_device(p);
   if (st) return st;
   const SpecView sv = spec_view(p, flags);
-  if ((st = lat_inverse_stage(p, flm, static_cast<cplx*>(Y), batch, precision,
-                              static_cast<hipStream_t>(stream), packed, nullptr, &sv)))
-    return st;
-  return zero_spec_pad(p, Y, sv.tiled, batch, static_cast<hipStream_t>(stream));
+  return lat_inverse_stage(p, flm, static_cast<cplx*>(Y), batch, precision,
+                           static_cast<hipStream_t>(stream), packed, nullptr, &sv);
 }
 
 extern "C" int s2h_flm_pack(int L, const void* flm, void* flm_p, int batch, s2h_stream stream) {
@@ -672,12 +675,16 @@ extern "C" int s2h_ring_residual_ex(const s2h_plan* p, const void* G, const void
   } else {
     RingAliasArgs a = alias_args(p, G, Y, R);
     a.alpha = alpha;
+    if (R != G) {
+      a.pad_row0 = p->fwd_rows;
+      a.pad_rows = p->spec_rows - p->fwd_rows;
+    }
     st = sumsq ? hip_status(launch_ring_alias_sumsq(a, p->fwd_set, batch,
                                                     static_cast<double*>(work), sumsq, s))
                : hip_status(launch_ring_alias(a, p->fwd_set, batch, s));
   }
-  if (st || R == G) return st;
-  return zero_spec_pad(p, R, tiled ? 1 : 0, batch, s);
+  if (st || R == G || !tiled) return st;
+  return zero_spec_pad(p, R, 1, batch, s);
 }
 
 extern "C" int s2h_ring_residual_scaled(const s2h_plan* p, const void* G, const void* Y,
@@ -769,7 +776,6 @@ extern "C" int s2h_inverse_rings_dot(const s2h_plan* p, const void* flm, void* Y
   if ((st = lat_inverse_stage(p, flm, static_cast<cplx*>(Y), batch, precision, s, packed, nullptr,
                               &sv, head > 0 ? part : nullptr, stride)))
     return st;
-  if ((st = zero_spec_pad(p, Y, 1, batch, s))) return st;
   ProfScope ps(S2H_KERNEL_RING_RESIDUAL, s);
   const RingAliasTiledArgs a = alias_tiled_args(p, Y, Y, nullptr, true);
   if (head == 0)  // vector-ALU synthesis: the whole dot over the spectra

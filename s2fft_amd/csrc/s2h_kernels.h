@@ -25,6 +25,7 @@ struct RingFwdArgs {
   int in_single;            // complex64 input (complex, unpaired maps only)
   int out_single;           // complex64 output
   int norm_mode;            // extra per-ring scale: 0 none, 1: 1/nphi, 2: 1/sqrt(nphi)
+  int pad_row0, pad_rows;   // ring-major spectra: also zeros into these rows of out
 };
 
 struct RingInvArgs {
@@ -104,6 +105,8 @@ struct RingAliasArgs {
   int L;
   const double* alpha;      // per-map scale of A(Y) in R = G - alpha A(Y) (null: 1)
   double* part;             // [map][ring job] partial sums: the dot (dot mode) or |R|^2
+  int jobs_end;             // set by the launcher: ring jobs, then the padding rows
+  int pad_row0, pad_rows;   // writes zeros into these rows of r (not in dot mode)
 };
 
 // Recursion tables of one map of a multi-plane launch (the n-planes of a
@@ -152,6 +155,7 @@ struct LatArgs {
                             // 2 (VALU kernels): zeros there
   double pos_scale;         // VALU forward: factor of the m > 0 columns
   LatPole pole;             // VALU kernels
+  int pad_row0, pad_rows;   // VALU inverse: also zeros into these rows of ftm
   int flm_packed;           // flm in the packed m-major layout (real maps, m >= 0 only)
   const LatPlane* planes;   // non-null: map b uses planes[b] in place of mstart, coef and
                             // lmin_out (VALU kernels, unpaired rings)

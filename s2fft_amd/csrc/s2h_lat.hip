@@ -280,7 +280,11 @@ lat_inverse_kernel(LatArgs a) {
       }
     }
   }
-  if (g != 0 || (a.pole.south < 0 && a.pole.north < 0)) return;
+  if (g != 0) return;
+  for (int e = tid; e < a.pad_rows * nb; e += nthr)
+    out[(int64_t)(e / a.pad_rows) * a.ftm_map_stride +
+        spec_row(a.pad_row0 + e % a.pad_rows, a.ftm_ncol, a.ftm_tiled)] = {0.0, 0.0};
+  if (a.pole.south < 0 && a.pole.north < 0) return;
   // the pole rows' column m (spherical.py:166-177): the south row holds only m =
   // spin, sum_l (-1)^|l-spin| flm[l, spin], the north row only m = -spin, sum_l
   // flm[l, -spin] (both with the normalisation); the first wave sums over l

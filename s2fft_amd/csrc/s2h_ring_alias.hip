@@ -74,6 +74,11 @@ struct FastDiv {
 template <int TPB, bool DOT>
 __global__ void __launch_bounds__(TPB) ring_alias_kernel(RingAliasArgs a) {
   __shared__ double part[2 * TPB];
+  if (!DOT && (int)blockIdx.x == a.jobs_end) {  // the padding rows, one run
+    cplx* pad = a.r + (int64_t)blockIdx.y * a.map_stride + (int64_t)a.pad_row0 * a.ncol;
+    for (int i = threadIdx.x; i < a.pad_rows * a.ncol; i += TPB) pad[i] = {0.0, 0.0};
+    return;
+  }
   const RingJob job = a.jobs[blockIdx.x];
   const int n = job.nphi;
   const int64_t off = (int64_t)blockIdx.y * a.map_stride + (int64_t)job.row * a.ncol;
@@ -223,7 +228,7 @@ __global__ void __launch_bounds__(TPB) ring_alias_kernel(RingAliasArgs a) {
     if (t == 0) {
       double tot = 0.0;
       for (int w = 0; w < TPB / 64; ++w) tot += part[w];
-      a.part[(int64_t)blockIdx.y * gridDim.x + blockIdx.x] = tot;
+      a.part[(int64_t)blockIdx.y * a.jobs_end + blockIdx.x] = tot;
     }
   }
 }
@@ -569,8 +574,9 @@ hipError_t launch_ring_alias(const RingAliasArgs& a, const JobSet& js, int batch
   if (batch == 0 || njobs == 0) return hipSuccess;
   RingAliasArgs b = a;
   b.jobs = js.jobs;
-  hipLaunchKernelGGL((ring_alias_kernel<kTpbAlias, false>), dim3(njobs, batch), dim3(kTpbAlias), 0,
-                     s, b);
+  b.jobs_end = njobs;
+  hipLaunchKernelGGL((ring_alias_kernel<kTpbAlias, false>), dim3(njobs + (b.pad_rows > 0), batch),
+                     dim3(kTpbAlias), 0, s, b);
   return hipGetLastError();
 }
 
@@ -581,8 +587,9 @@ hipError_t launch_ring_alias_sumsq(const RingAliasArgs& a, const JobSet& js, int
   RingAliasArgs b = a;
   b.jobs = js.jobs;
   b.part = part;
-  hipLaunchKernelGGL((ring_alias_kernel<kTpbAlias, false>), dim3(njobs, batch), dim3(kTpbAlias), 0,
-                     s, b);
+  b.jobs_end = njobs;
+  hipLaunchKernelGGL((ring_alias_kernel<kTpbAlias, false>), dim3(njobs + (b.pad_rows > 0), batch),
+                     dim3(kTpbAlias), 0, s, b);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(ring_dot_final_kernel, dim3(batch), dim3(256), 0, s, part, njobs, nullptr,
@@ -696,6 +703,7 @@ hipError_t launch_ring_dot(const RingAliasArgs& a, const JobSet& js, int batch, 
   b.jobs = js.jobs;
   b.part = part;
   b.alpha = nullptr;
+  b.jobs_end = njobs;
   hipLaunchKernelGGL((ring_alias_kernel<kTpbAlias, true>), dim3(njobs, batch), dim3(kTpbAlias), 0,
                      s, b);
   hipError_t e = hipGetLastError();

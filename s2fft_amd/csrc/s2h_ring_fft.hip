@@ -982,6 +982,13 @@ __global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(2)))
 ring_reg_fwd_kernel(RingFwdArgs a, RingSegs g, int paired) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
   ring_body<WG, 0>(a, seg_of_block(g), paired, lds_raw);
+  if (a.pad_rows && blockIdx.x == gridDim.x - 1) {
+    const int maps = paired ? 2 : 1;
+    for (int b = maps * blockIdx.y; b < min(a.batch, maps * ((int)blockIdx.y + 1)); ++b) {
+      cplx* pad = a.out + (int64_t)b * a.out_map_stride + (int64_t)a.pad_row0 * a.ncol;
+      for (int i = threadIdx.x; i < a.pad_rows * a.ncol; i += WG) pad[i] = {0.0, 0.0};
+    }
+  }
 }
 template <int WG>
 __global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(2)))
