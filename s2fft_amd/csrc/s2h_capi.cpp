@@ -280,6 +280,7 @@ int lat_forward_stage(const s2h_plan* p, const cplx* ftm, void* flm, int batch, 
   a.ftm_m_first = p->m_lo;
   a.ftm_tiled = sv ? sv->tiled : 0;
   a.lmin_out = std::max(std::abs(p->d.spin), p->d.L_lower);
+  if (bf16 || mixed) a.ucoef = p->fwd_rcoef;
   a.accumulate = accumulate ? 1 : 0;
   if (ps) a.planes = ps->fwd;
   const bool poles = p->fwd_row_south >= 0 || p->fwd_row_north >= 0;
@@ -354,6 +355,7 @@ int lat_inverse_stage(const s2h_plan* p, const void* flm, cplx* ftm, int batch, 
   a.ftm_ncol = p->Mc;
   a.ftm_m_first = p->m_lo;
   a.ftm_tiled = sv ? sv->tiled : 0;
+  if (bf16 || mixed) a.ucoef = p->inv_rcoef;
   if (ps) a.planes = ps->inv;
   if (dot_part) {
     a.dot_wn = p->spec_belt_wn;
@@ -1405,7 +1407,7 @@ extern "C" int s2h_compute_all_slices(const s2h_plan* p, const double* beta, int
   if (st) return st;
   DTableArgs a{};
   a.mstart = p->inv_mstart;
-  a.coef = p->inv_coef;
+  a.coef = p->inv_ucoef;
   a.theta = beta;
   a.T = ntheta;
   a.L = p->d.L;
@@ -1434,7 +1436,7 @@ extern "C" int s2h_precompute_kernel(const s2h_plan* p, int forward, double scal
   const bool hp = p->d.sampling == S2H_HEALPIX;
   DTableArgs a{};
   a.mstart = forward ? p->fwd_mstart : p->inv_mstart;
-  a.coef = forward ? p->fwd_coef : p->inv_coef;
+  a.coef = forward ? p->fwd_ucoef : p->inv_ucoef;
   a.theta = forward ? p->fwd_theta : p->inv_theta;
   a.T = forward ? p->pc_rows : p->inv_rows;
   a.L = p->d.L;

@@ -53,7 +53,8 @@ struct MStart {
   int32_t pad2;
 };
 
-// d^{l+1} = (a x - b) d^l - c d^{l-1} for the normalised d (per |m|, l).
+// One step in unit-c form, e_{l+1} = (a x - b) e_l - e_{l-1}; c: sigma_l, d_l =
+// sigma_l e_l for the normalised d (per |m|, l).
 struct Coef {
   double a, b, c, pad;
 };

@@ -186,37 +186,21 @@ __device__ __forceinline__ int m_group_of_block(int i, int nm, int G, int m_lo, 
 
 // Recursion coefficients of one 32-step chunk, staged in LDS so that every
 // step reads them with a broadcast LDS load instead of a dependent global or
-// scalar load.  (a, -b * bsign, c) for l = blk + i; zero from l = L - 1 on,
-// which makes the steps past the band-limit produce zeros.
+// scalar load: (a', -b' * bsign, sigma) for l = blk + i; a' and b' are zero from
+// l = L - 1 on, which makes the steps past the band-limit produce zeros.
 struct ChunkCoef {
   double a, nb, c, pad;
 };
 constexpr int kChunk = 32;
 
-// Chunk `blk`'s coefficient for lane i (< 32) as stored (zero from l = L - 1
-// on).  A prefetch keeps it in this form until it is written to LDS
-// (finish_coef there): arithmetic on the loaded value right after the load
-// would make the wave wait for the memory latency at once.
-__device__ __forceinline__ Coef load_coef_raw(const Coef* __restrict__ cf, int blk, int i, int L) {
-  const int l = blk + i;
-  Coef v = {0.0, 0.0, 0.0, 0.0};
-  if (l + 1 < L) v = cf[l];
-  return v;
-}
-
 __device__ __forceinline__ ChunkCoef finish_coef(const Coef& c, double bsign) {
   return {c.a, -c.b * bsign, c.c, 0.0};
 }
 
-// Loads chunk `blk`'s coefficient for lane i (< 32) into registers.
-__device__ __forceinline__ ChunkCoef load_coef(const Coef* __restrict__ cf, int blk, int i, int L,
-                                               double bsign) {
-  return finish_coef(load_coef_raw(cf, blk, i, L), bsign);
-}
-
-// Unit-c coefficients {a', b', sigma, 0} (the plan's make_unit_coefs) of
-// chunk `blk` for lane i, read as stored up to l = L - 1 (a' and b' are
-// already zero there; sigma_{L-1} is needed), zero past it.
+// Chunk `blk`'s coefficient for lane i (< 32) as stored, zero past l = L - 1.  A
+// prefetch keeps it in this form until it is written to LDS (finish_coef
+// there): arithmetic on the loaded value right after the load would make the
+// wave wait for the memory latency at once.
 __device__ __forceinline__ Coef load_ucoef_raw(const Coef* __restrict__ cf, int blk, int i, int L) {
   const int l = blk + i;
   Coef v = {0.0, 0.0, 0.0, 0.0};
@@ -224,11 +208,7 @@ __device__ __forceinline__ Coef load_ucoef_raw(const Coef* __restrict__ cf, int 
   return v;
 }
 
-// One recursion step with staged coefficients: returns d_{l+1}.
-__device__ __forceinline__ double rec_step(const ChunkCoef& c, double x, double d, double dm1) {
-  return fma(fma(c.a, x, c.nb), d, -c.c * dm1);
-}
-// The same step in unit-c form (unit coefficients staged): e_{l+1}.
+// One recursion step with staged coefficients: e_{l+1}.
 __device__ __forceinline__ double rec_step_unit(const ChunkCoef& c, double x, double e, double em1) {
   return fma(fma(c.a, x, c.nb), e, -em1);
 }

@@ -222,63 +222,58 @@ MStart make_mstart(int m, int n, int kind, bool inverse, double sign) {
   return st;
 }
 
-// Normalised three-term coefficients for |m| (b for m = +|m|).
-void make_coefs(int L, int n, int kind, bool inverse, std::vector<Coef>& out) {
-  out.assign((size_t)L * L, Coef{0, 0, 0, 0});
+// Recursion coefficients for |m| (b for m = +|m|), in two unit-c forms.  The normalised
+// three-term recursion d_{l+1} = (A x - B) d_l - C d_{l-1} becomes, with d_l = sigma_l
+// e_l, sigma_l0 = sigma_{l0+1} = 1 and sigma_{l+1} = C_l sigma_{l-1},
+//   e_{l+1} = (a' x - b') e_l - e_{l-1},
+// a multiplication less per step.  C_l > 0 for l > l0, so sigma never vanishes; it
+// varies slowly with l (the C_l are near 1 away from l = |m|, |n|).  unit: a', b' and
+// sigma rounded once each from the exact values (the FP64 kernels: a rounded
+// coefficient acts on every ring alike, and rounding A, B and C first left the spin 2
+// recursions of L = 350 with 1.0e-13 relative error, against 0.8e-13 in the three-term
+// form and 0.2e-13 so).  rounded: formed from A, B and C rounded to FP64 (the reduced-
+// precision kernels, whose results hang on every bit of d).
+void make_coefs(int L, int n, int kind, bool inverse, std::vector<Coef>& unit,
+                std::vector<Coef>& rounded) {
+  unit.assign((size_t)L * L, Coef{0, 0, 0, 0});
+  rounded.assign((size_t)L * L, Coef{0, 0, 0, 0});
   std::vector<long double> N(L + 1);
   for (int l = 0; l <= L; ++l) N[l] = ell_norm(kind, l, inverse);
   const long double nn = n;
+  struct Sigma {
+    long double prev = 1.0L, cur = 1.0L;  // sigma_{l-1}, sigma_l
+    Coef step(bool first, bool last, long double A, long double B, long double C) {
+      const long double next = first ? 1.0L : C * prev;
+      Coef u{0, 0, (double)cur, 0};
+      if (!last) {
+        u.a = (double)(A * cur / next);
+        u.b = (double)(B * cur / next);
+      }
+      prev = cur;
+      cur = next;
+      return u;
+    }
+  };
   for (int am = 0; am < L; ++am) {
     const long double mm = am;
     const int l0 = std::max(am, std::abs(n));
+    Sigma su, sr;
     for (int l = l0; l < L; ++l) {
-      Coef c{0, 0, 0, 0};
+      long double A, B = 0.0L, C = 0.0L;
       if (l == 0) {
-        c.a = (double)(N[1] / N[0]);
+        A = N[1] / N[0];
       } else {
         const long double L1 = l + 1.0L, Ll = l;
         const long double D =
             Ll * std::sqrt((L1 * L1 - mm * mm) * (L1 * L1 - nn * nn));
-        const long double A = (2.0L * Ll + 1.0L) * Ll * L1 / D;
-        const long double B = (2.0L * Ll + 1.0L) * mm * nn / D;
-        const long double C =
-            L1 * std::sqrt(std::max(0.0L, (Ll * Ll - mm * mm) * (Ll * Ll - nn * nn))) / D;
-        c.a = (double)(A * N[l + 1] / N[l]);
-        c.b = (double)(B * N[l + 1] / N[l]);
-        c.c = (double)(C * N[l + 1] / N[l - 1]);
+        A = (2.0L * Ll + 1.0L) * Ll * L1 / D * N[l + 1] / N[l];
+        B = (2.0L * Ll + 1.0L) * mm * nn / D * N[l + 1] / N[l];
+        C = L1 * std::sqrt(std::max(0.0L, (Ll * Ll - mm * mm) * (Ll * Ll - nn * nn))) / D *
+            N[l + 1] / N[l - 1];
       }
-      out[(size_t)am * L + l] = c;
-    }
-  }
-}
-
-// The same recursion with unit c: d_l = sigma_l e_l, where sigma_l0 =
-// sigma_{l0+1} = 1 and sigma_{l+1} = c_l sigma_{l-1}, turns
-//   d_{l+1} = (a_l x - b_l) d_l - c_l d_{l-1}
-// into e_{l+1} = (a'_l x - b'_l) e_l - e_{l-1} with (a', b') = (a, b) sigma_l /
-// sigma_{l+1}: one FP64 multiply less per step.  Entry l holds
-// {a'_l, b'_l, sigma_l, 0}; a' and b' are zero from l = L - 1 on (the steps
-// past the band-limit give zeros), sigma is kept up to l = L - 1.  c_l > 0
-// for l > l0, so sigma never vanishes; it varies slowly with l (the c_l are
-// near 1 away from l = |m|, |n|).
-void make_unit_coefs(int L, int n, const std::vector<Coef>& c, std::vector<Coef>& out) {
-  out.assign((size_t)L * L, Coef{0, 0, 0, 0});
-  for (int am = 0; am < L; ++am) {
-    const int l0 = std::max(am, std::abs(n));
-    if (l0 >= L) continue;
-    const Coef* cm = c.data() + (size_t)am * L;
-    Coef* um = out.data() + (size_t)am * L;
-    long double s_prev = 1.0L, s_cur = 1.0L;  // sigma_{l-1}, sigma_l at l = l0
-    for (int l = l0; l < L; ++l) {
-      const long double s_next = l == l0 ? 1.0L : (long double)cm[l].c * s_prev;
-      Coef u{0, 0, (double)s_cur, 0};
-      if (l + 1 < L) {
-        u.a = (double)((long double)cm[l].a * s_cur / s_next);
-        u.b = (double)((long double)cm[l].b * s_cur / s_next);
-      }
-      um[l] = u;
-      s_prev = s_cur;
-      s_cur = s_next;
+      const size_t i = (size_t)am * L + l;
+      unit[i] = su.step(l == l0, l + 1 == L, A, B, C);
+      rounded[i] = sr.step(l == l0, l + 1 == L, (double)A, (double)B, (double)C);
     }
   }
 }
@@ -605,10 +600,7 @@ static int plan_build(s2h_plan* p) {
     msf.push_back(make_mstart(m, n, d.norm, false, p->sign));
     msi.push_back(make_mstart(m, n, d.norm, true, p->sign));
   }
-  std::vector<Coef> cf, ci;
-  make_coefs(L, n, d.norm, false, cf);
   const bool same = d.norm != S2H_NORM_WIGNER;
-  if (!same) make_coefs(L, n, d.norm, true, ci);
   std::vector<double> nf(L), ni(L);
   for (int l = 0; l < L; ++l) {
     nf[l] = (double)(ell_norm(d.norm, l, false) * p->sign);
@@ -662,21 +654,17 @@ static int plan_build(s2h_plan* p) {
   }
   if ((st = upload(p, msf, &p->fwd_mstart))) return st;
   if ((st = upload(p, msi, &p->inv_mstart))) return st;
-  if ((st = upload(p, cf, &p->fwd_coef))) return st;
-  if (same) {
-    p->inv_coef = p->fwd_coef;
-  } else if ((st = upload(p, ci, &p->inv_coef))) {
-    return st;
-  }
   {
-    std::vector<Coef> u;
-    make_unit_coefs(L, n, cf, u);
-    if ((st = upload(p, u, &p->fwd_ucoef))) return st;
-    if (same) {
-      p->inv_ucoef = p->fwd_ucoef;
-    } else {
-      make_unit_coefs(L, n, ci, u);
-      if ((st = upload(p, u, &p->inv_ucoef))) return st;
+    std::vector<Coef> unit, rounded;
+    make_coefs(L, n, d.norm, false, unit, rounded);
+    if ((st = upload(p, unit, &p->fwd_ucoef))) return st;
+    if ((st = upload(p, rounded, &p->fwd_rcoef))) return st;
+    p->inv_ucoef = p->fwd_ucoef;
+    p->inv_rcoef = p->fwd_rcoef;
+    if (!same) {
+      make_coefs(L, n, d.norm, true, unit, rounded);
+      if ((st = upload(p, unit, &p->inv_ucoef))) return st;
+      if ((st = upload(p, rounded, &p->inv_rcoef))) return st;
     }
   }
   if ((st = upload(p, nf, &p->fwd_norm))) return st;

@@ -26,8 +26,8 @@ struct s2h_plan {
   bool fwd_paired = false;
   int fwd_row_south = -1, fwd_row_north = -1;
   s2h::MStart* fwd_mstart = nullptr;
-  s2h::Coef* fwd_coef = nullptr;
-  s2h::Coef* fwd_ucoef = nullptr;  // unit-c form (make_unit_coefs)
+  s2h::Coef* fwd_ucoef = nullptr;  // make_coefs: FP64 kernels
+  s2h::Coef* fwd_rcoef = nullptr;  // reduced-precision kernels
   double* fwd_norm = nullptr;
   int rs_info[8] = {0};           // stored-kernel resampling: DFT lengths / conv lengths
   int64_t rs_chirp[4] = {0};
@@ -40,8 +40,8 @@ struct s2h_plan {
   bool inv_paired = false;
   int inv_row_south = -1, inv_row_north = -1;
   s2h::MStart* inv_mstart = nullptr;
-  s2h::Coef* inv_coef = nullptr;
   s2h::Coef* inv_ucoef = nullptr;
+  s2h::Coef* inv_rcoef = nullptr;
   double* inv_norm = nullptr;
   bool inv_out_complex = true;
 

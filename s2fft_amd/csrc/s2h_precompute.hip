@@ -70,9 +70,9 @@ __global__ void __launch_bounds__(kThreads) dtable_kernel(DTableArgs a) {
   int lscale;
   lat::start_value(st, c2, s2, d, lscale);
   for (int l = l0; l < a.L; ++l) {
-    put(l, lscale == 0 ? d * fac * (a.lw ? a.lw[l] : 1.0) : 0.0);
-    const lat::ChunkCoef c = lat::load_coef(cf, l, 0, a.L, bsign);
-    const double dn = lat::rec_step(c, x, d, dm1);
+    const lat::ChunkCoef c = lat::finish_coef(cf[l], bsign);  // d: e_l, d_l = sigma_l e_l
+    put(l, lscale == 0 ? c.c * d * fac * (a.lw ? a.lw[l] : 1.0) : 0.0);
+    const double dn = lat::rec_step_unit(c, x, d, dm1);
     dm1 = d;
     d = dn;
     if (((l - l0) % kRescale) == kRescale - 1) lat::rescale(d, dm1, lscale);
