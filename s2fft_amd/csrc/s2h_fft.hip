@@ -48,57 +48,56 @@ __global__ void __launch_bounds__(kThreads) chirp_setup_kernel(const ChirpEntry*
 // restricted to n >= 0: Re sum_{n >= 0} x_n e^{+2 pi i n g / G}), 5 the
 // adjoint of mode 3: from real f, the N rows n >= 0 of the forward sum, the
 // rows n >= 1 doubled.
-__global__ void __launch_bounds__(kThreads) gamma_dft_kernel(int N, int64_t npix, int mode,
-                                                             double scale, const void* in_,
-                                                             void* out_) {
+// A sample's inputs sit in registers (N a template parameter), the G roots of
+// unity in LDS; blockIdx.y takes every gridDim.y-th output.  Bound by its
+// launch at the sizes of a Wigner transform: MW L = 64, N = 4 22 -> 3.4 us (before,
+// a root evaluated for every term and the inputs in scratch memory).
+template <int N>
+__global__ void __launch_bounds__(kThreads) gamma_dft_kernel(int64_t npix, int mode, double scale,
+                                                             const void* in_, void* out_) {
+  constexpr int G = 2 * N - 1;
+  __shared__ cplx w[G];  // e^{2 pi i j / G}
+  if (threadIdx.x < G) w[threadIdx.x] = expi_pi(2 * (int64_t)threadIdx.x, G);
+  __syncthreads();
   const int64_t p = (int64_t)blockIdx.x * kThreads + threadIdx.x;
   if (p >= npix) return;
-  const int G = 2 * N - 1;
-  cplx x[15];
-  if (mode == 0 || mode == 1) {
-    const cplx* in = static_cast<const cplx*>(in_);
-    for (int g = 0; g < G; ++g) x[g] = in[(int64_t)g * npix + p];
-  } else if (mode == 2 || mode == 5) {
-    const double* in = static_cast<const double*>(in_);
-    for (int g = 0; g < G; ++g) x[g] = {in[(int64_t)g * npix + p], 0.0};
-  } else {
-    const cplx* in = static_cast<const cplx*>(in_);
-    for (int k = 0; k < N; ++k) x[k] = in[(int64_t)k * npix + p];
+  cplx x[G];
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    x[g] = {0.0, 0.0};
+    if (mode == 2 || mode == 5)
+      x[g].x = static_cast<const double*>(in_)[(int64_t)g * npix + p];
+    else if (mode < 2 || g < N)  // modes 3, 4: the N rows n >= 0
+      x[g] = static_cast<const cplx*>(in_)[(int64_t)g * npix + p];
   }
-  if (mode == 0 || mode == 2) {
-    cplx* out = static_cast<cplx*>(out_);
-    for (int k = 0; k < G; ++k) {
-      const int n = k - (N - 1);
-      cplx acc = {0.0, 0.0};
-      for (int g = 0; g < G; ++g) acc = cadd(acc, cmul(x[g], expi_pi(-2 * (int64_t)n * g, G)));
-      out[(int64_t)k * npix + p] = {acc.x * scale, acc.y * scale};
-    }
-  } else if (mode == 5) {
-    cplx* out = static_cast<cplx*>(out_);
-    for (int n = 0; n < N; ++n) {
-      cplx acc = {0.0, 0.0};
-      for (int g = 0; g < G; ++g) acc = cadd(acc, cmul(x[g], expi_pi(-2 * (int64_t)n * g, G)));
-      const double w = (n ? 2.0 : 1.0) * scale;
-      out[(int64_t)n * npix + p] = {acc.x * w, acc.y * w};
-    }
-  } else if (mode == 1) {
-    cplx* out = static_cast<cplx*>(out_);
-    for (int g = 0; g < G; ++g) {
-      cplx acc = {0.0, 0.0};
-      for (int k = 0; k < G; ++k) {
-        const int n = k - (N - 1);
-        acc = cadd(acc, cmul(x[k], expi_pi(2 * (int64_t)n * g, G)));
-      }
-      out[(int64_t)g * npix + p] = {acc.x * scale, acc.y * scale};
-    }
-  } else {
-    double* out = static_cast<double*>(out_);
-    const double wn = mode == 3 ? 2.0 : 1.0;
-    for (int g = 0; g < G; ++g) {
+  const auto wrap = [](int j) { return j >= G ? j - G : j; };
+  const int nout = mode == 5 ? N : G;
+  for (int k = blockIdx.y; k < nout; k += gridDim.y) {
+    cplx* out = static_cast<cplx*>(out_) + (int64_t)k * npix + p;
+    if (mode == 3 || mode == 4) {  // sample g = k from x[n]
+      const double wn = mode == 3 ? 2.0 : 1.0;
       double acc = x[0].x;
-      for (int n = 1; n < N; ++n) acc += wn * cmul(x[n], expi_pi(2 * (int64_t)n * g, G)).x;
-      out[(int64_t)g * npix + p] = acc * scale;
+      int j = 0;
+#pragma unroll
+      for (int n = 1; n < N; ++n) {
+        j = wrap(j + k);
+        acc += wn * cmul(x[n], w[j]).x;
+      }
+      static_cast<double*>(out_)[(int64_t)k * npix + p] = acc * scale;
+      continue;
     }
+    // row n from the samples: root -n g; sample k from the rows: root (i - (N - 1)) k
+    const int n = mode == 5 ? k : k - (N - 1);
+    const int step = mode == 1 ? k : n > 0 ? G - n : -n;
+    int j = mode == 1 ? (N * k) % G : 0;  // -(N - 1) = N modulo G
+    cplx acc = {0.0, 0.0};
+#pragma unroll
+    for (int i = 0; i < G; ++i) {
+      acc = cadd(acc, cmul(x[i], w[j]));
+      j = wrap(j + step);
+    }
+    const double f = mode == 5 && n ? 2.0 * scale : scale;
+    *out = {acc.x * f, acc.y * f};
   }
 }
 
@@ -147,8 +146,18 @@ hipError_t launch_gamma_dft(int N, int64_t npix, int mode, double scale, const v
                             void* out, hipStream_t s) {
   if (npix == 0) return hipSuccess;
   const int64_t blocks = (npix + kThreads - 1) / kThreads;
-  hipLaunchKernelGGL(gamma_dft_kernel, dim3((unsigned)blocks), dim3(kThreads), 0, s, N, npix,
-                     mode, scale, in, out);
+  // few samples: one output per thread
+  const dim3 grid((unsigned)blocks, blocks < 512 ? 2 * N - 1 : 1), block(kThreads);
+  switch (N) {
+#define S2H_GAMMA(n)                                                                              \
+  case n:                                                                                         \
+    hipLaunchKernelGGL(gamma_dft_kernel<n>, grid, block, 0, s, npix, mode, scale, in, out);       \
+    break;
+    S2H_GAMMA(1) S2H_GAMMA(2) S2H_GAMMA(3) S2H_GAMMA(4)
+    S2H_GAMMA(5) S2H_GAMMA(6) S2H_GAMMA(7) S2H_GAMMA(8)
+#undef S2H_GAMMA
+    default: return hipErrorInvalidValue;
+  }
   return hipGetLastError();
 }
 
