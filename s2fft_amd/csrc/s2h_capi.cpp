@@ -173,7 +173,9 @@ extern "C" int s2h_version(void) { return 1; }
 
 extern "C" size_t s2h_workspace_bytes(const s2h_plan* p, int batch) {
   if (!p || batch < 0) return 0;
-  size_t rows = (size_t)std::max(p->pc_rows, p->inv_rows);
+  // the stored-kernel forward's rows, the projection's (whole blocks of 8, which is
+  // more for L = 2 and 3) or the synthesis'
+  size_t rows = (size_t)std::max(std::max(p->pc_rows, p->fwd_rows), p->inv_rows);
   if (p->fwd_kind != 0) rows += (size_t)p->fwd_in_rows;
   // + one flm-sized buffer for the adjoint of the conjugate fill
   const size_t flm = (size_t)p->d.L * (2 * p->d.L - 1);
