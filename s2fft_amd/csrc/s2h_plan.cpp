@@ -231,7 +231,8 @@ MStart make_mstart(int m, int n, int kind, bool inverse, double sign) {
 // sigma rounded once each from the exact values (the FP64 kernels: a rounded
 // coefficient acts on every ring alike, and rounding A, B and C first left the spin 2
 // recursions of L = 350 with 1.0e-13 relative error, against 0.8e-13 in the three-term
-// form and 0.2e-13 so).  rounded: formed from A, B and C rounded to FP64 (the reduced-
+// form and 0.2e-13 so; spin 0, L = 300: 2.1e-13 three-term, 0.6e-13 from rounded and
+// 0.7e-13 so).  rounded: formed from A, B and C rounded to FP64 (the reduced-
 // precision kernels, whose results hang on every bit of d).
 void make_coefs(int L, int n, int kind, bool inverse, std::vector<Coef>& unit,
                 std::vector<Coef>& rounded) {
@@ -657,14 +658,18 @@ static int plan_build(s2h_plan* p) {
   {
     std::vector<Coef> unit, rounded;
     make_coefs(L, n, d.norm, false, unit, rounded);
-    if ((st = upload(p, unit, &p->fwd_ucoef))) return st;
+    // spin 0 (b = 0): one set serves every kernel; the recursion is as accurate with the
+    // rounded one, and refinements run FP64 and reduced-precision steps of one operator
     if ((st = upload(p, rounded, &p->fwd_rcoef))) return st;
+    p->fwd_ucoef = p->fwd_rcoef;
+    if (n != 0 && (st = upload(p, unit, &p->fwd_ucoef))) return st;
     p->inv_ucoef = p->fwd_ucoef;
     p->inv_rcoef = p->fwd_rcoef;
     if (!same) {
       make_coefs(L, n, d.norm, true, unit, rounded);
-      if ((st = upload(p, unit, &p->inv_ucoef))) return st;
       if ((st = upload(p, rounded, &p->inv_rcoef))) return st;
+      p->inv_ucoef = p->inv_rcoef;
+      if (n != 0 && (st = upload(p, unit, &p->inv_ucoef))) return st;
     }
   }
   if ((st = upload(p, nf, &p->fwd_norm))) return st;

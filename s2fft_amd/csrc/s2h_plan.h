@@ -26,7 +26,7 @@ struct s2h_plan {
   bool fwd_paired = false;
   int fwd_row_south = -1, fwd_row_north = -1;
   s2h::MStart* fwd_mstart = nullptr;
-  s2h::Coef* fwd_ucoef = nullptr;  // make_coefs: FP64 kernels
+  s2h::Coef* fwd_ucoef = nullptr;  // make_coefs: FP64 kernels (spin 0: rcoef)
   s2h::Coef* fwd_rcoef = nullptr;  // reduced-precision kernels
   double* fwd_norm = nullptr;
   int rs_info[8] = {0};           // stored-kernel resampling: DFT lengths / conv lengths
