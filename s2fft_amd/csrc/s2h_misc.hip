@@ -612,8 +612,7 @@ namespace s2h {
 // Adjoint of the conjugate fill (reality): for m >= 1
 // out[l, m] = (g[l, m] + (-1)^m conj(g[l, -m])) / 2, out[l, 0] = Re g[l, 0].
 // The 1/2 pairs with the Hermitian completion of the inverse ring kernel, which
-// takes real m = 0 values (it transforms maps in pairs x_0 + i x_1: an imaginary
-// part here would end up in the partner's map).
+// takes the real part at m = 0.
 __global__ void __launch_bounds__(kThreads) reality_fold_kernel(const cplx* g, cplx* out,
                                                                 int64_t map_stride, int L) {
   const int64_t b = blockIdx.z;

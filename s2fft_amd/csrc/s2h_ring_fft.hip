@@ -550,7 +550,9 @@ struct FoldIn {
     ph = ring_phase(a.apply_phase, job);
   }
   // u[e] = c(m), or c_x(m) + i c_y(m), for m = at(e), zero where m is outside
-  // [lo, hi]; m < 0 of Hermitian spectra from conj c(-m)
+  // [lo, hi]; m < 0 of Hermitian spectra from conj c(-m), m = 0 without its
+  // imaginary part: a map alone drops it with the imaginary part of the ring, in a
+  // pair it would be the partner's
   template <int E, typename At>
   __device__ __forceinline__ void gather(cplx* u, At at) const {
     const auto place = [&](int e) {
@@ -567,10 +569,15 @@ struct FoldIn {
 #pragma unroll
       for (int e = 0; e < E; ++e) u[e] = x[place(e)];
     }
+    const auto real0 = [&](int e, cplx& c) { c.y = herm && at(e) == 0 ? 0.0 : c.y; };
+#pragma unroll
+    for (int e = 0; e < E; ++e) real0(e, u[e]);
     if (y) {
       cplx r[E];
 #pragma unroll
       for (int e = 0; e < E; ++e) r[e] = y[place(e)];
+#pragma unroll
+      for (int e = 0; e < E; ++e) real0(e, r[e]);
 #pragma unroll
       for (int e = 0; e < E; ++e) {
         const double sg = herm && at(e) < 0 ? -1.0 : 1.0;

@@ -1,0 +1,61 @@
+"""Batches of real maps against each map alone, for coefficients as an optimisation
+hands them over: the imaginary part at m = 0 not zero (needs a GPU).
+
+Real rings are transformed in pairs x + i y.  A map alone has no imaginary part at m =
+0 (it takes the real part of the sum), so inside a batch it has to have none either.
+FP64 rounding of two maps of one scale: 1e-13 of a map's own maximum is some hundred
+eps; the imaginary parts are of order one.
+"""
+
+import pytest
+import torch
+
+import s2fft_amd
+from s2fft_amd import precompute_transforms as pc
+from s2fft_amd.transforms import spherical as sph
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-13
+
+
+def _flm(B, L, seed):
+    gen = torch.Generator().manual_seed(seed)
+    flm = torch.randn((B, L, 2 * L - 1), generator=gen, dtype=torch.complex128)
+    m = torch.arange(-(L - 1), L)[None, :]
+    return (flm * (m.abs() <= torch.arange(L)[:, None])).cuda()
+
+
+def _own_error(got, want):
+    return float((got - want).abs().max() / want.abs().max())
+
+
+@pytest.mark.parametrize("sampling,L,nside", [("healpix", 16, 8), ("healpix", 61, 30),
+                                              ("gl", 20, None), ("mw", 33, None),
+                                              ("mwss", 32, None), ("dh", 17, None)])
+@pytest.mark.parametrize("batch", [2, 3, 9])
+def test_m0_stays_with_its_map(sampling, L, nside, batch):
+    flm = _flm(batch, L, L)
+    kw = dict(nside=nside, sampling=sampling, reality=True)
+    for real_output in (False, True):
+        got = sph.inverse_hip(flm, L, real_output=real_output, **kw)
+        for b in range(batch):
+            one = sph.inverse_hip(flm[b:b + 1], L, real_output=real_output, **kw)[0]
+            assert _own_error(got[b], one) < TOL
+    # and the gradient says the same
+    x = flm.clone().requires_grad_()
+    g = torch.randn(s2fft_amd.inverse(flm, L, **kw).shape, dtype=torch.float64,
+                    generator=torch.Generator("cuda").manual_seed(1), device="cuda")
+    (grad,) = torch.autograd.grad(s2fft_amd.inverse(x, L, **kw).real, x, g)
+    for b in range(batch):
+        x = flm[b].clone().requires_grad_()
+        (one,) = torch.autograd.grad(s2fft_amd.inverse(x, L, **kw).real, x, g[b])
+        assert _own_error(grad[b], one) < TOL
+
+
+@pytest.mark.parametrize("sampling,L,nside", [("healpix", 16, 8), ("gl", 20, None)])
+def test_m0_stays_with_its_map_stored_kernel(sampling, L, nside):
+    flm = _flm(3, L, L)
+    kw = dict(nside=nside, sampling=sampling, reality=True)
+    got = pc.spherical.inverse(flm, L, **kw)
+    for b in range(3):
+        assert _own_error(got[b], pc.spherical.inverse(flm[b], L, **kw)) < TOL
