@@ -552,8 +552,8 @@ struct FoldIn {
   // u[e] = c(m), or c_x(m) + i c_y(m), for m = at(e), zero where m is outside
   // [lo, hi]; m < 0 of Hermitian spectra from conj c(-m), m = 0 without its
   // imaginary part: a map alone drops it with the imaginary part of the ring, in a
-  // pair it would be the partner's
-  template <int E, typename At>
+  // pair it would be the partner's (at(e) = 0 for an e < N0 at most)
+  template <int E, int N0, typename At>
   __device__ __forceinline__ void gather(cplx* u, At at) const {
     const auto place = [&](int e) {
       const int m = at(e);
@@ -571,13 +571,13 @@ struct FoldIn {
     }
     const auto real0 = [&](int e, cplx& c) { c.y = herm && at(e) == 0 ? 0.0 : c.y; };
 #pragma unroll
-    for (int e = 0; e < E; ++e) real0(e, u[e]);
+    for (int e = 0; e < N0; ++e) real0(e, u[e]);
     if (y) {
       cplx r[E];
 #pragma unroll
       for (int e = 0; e < E; ++e) r[e] = y[place(e)];
 #pragma unroll
-      for (int e = 0; e < E; ++e) real0(e, r[e]);
+      for (int e = 0; e < N0; ++e) real0(e, r[e]);
 #pragma unroll
       for (int e = 0; e < E; ++e) {
         const double sg = herm && at(e) < 0 ? -1.0 : 1.0;
@@ -602,7 +602,7 @@ struct FoldIn {
     if (hi - lo < n) {  // one m per residue
 #pragma unroll
       for (int e0 = 0; e0 < E; e0 += 8)
-        gather<8>(v + e0, [&](int e) {
+        gather<8, 1>(v + e0, [&](int e) {
           const int q = t + T * (e0 + e);
           return q >= n ? hi + 1 : q <= hi ? q : q - n;
         });
@@ -621,7 +621,7 @@ struct FoldIn {
 #pragma unroll
       for (int e0 = 0; e0 < E; e0 += 8) {
         cplx u[8];
-        gather<8>(u, [&](int e) {
+        gather<8, 1>(u, [&](int e) {
           const int q = t + T * (e0 + e);
           return q < n ? q + j * n : hi + 1;
         });
@@ -641,7 +641,7 @@ struct FoldIn {
     const int j1 = floor_div(hi, n);
     for (int jb = floor_div(lo, n) + g; jb <= j1; jb += 8 * G) {
       cplx u[8];
-      gather<8>(u, [&](int i) { return q + (jb + i * G) * n; });
+      gather<8, 8>(u, [&](int i) { return q + (jb + i * G) * n; });
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const double sg = ph && ((jb + i * G) & 1) ? -1.0 : 1.0;
