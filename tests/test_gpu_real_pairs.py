@@ -2,7 +2,8 @@
 hands them over: the imaginary part at m = 0 not zero (needs a GPU).
 
 Real rings are transformed in pairs x + i y.  A map alone has no imaginary part at m =
-0 (it takes the real part of the sum), so inside a batch it has to have none either.
+0 (it takes the real part of the sum), so inside a batch it has to have none either.  Maps returned as complex128 are
+transformed alone: a partner that is larger by 1e8 or holds a NaN leaves no trace.
 FP64 rounding of two maps of one scale: 1e-13 of a map's own maximum is some hundred
 eps; the imaginary parts are of order one.
 """
@@ -59,3 +60,23 @@ def test_m0_stays_with_its_map_stored_kernel(sampling, L, nside):
     got = pc.spherical.inverse(flm, L, **kw)
     for b in range(3):
         assert _own_error(got[b], pc.spherical.inverse(flm[b], L, **kw)) < TOL
+
+
+@pytest.mark.parametrize("L,nside", [(16, 8), (61, 30), (200, 100), (256, 128)])
+def test_complex_maps_are_alone(L, nside):
+    flm = _flm(3, L, L)
+    flm[1] *= 1e8
+    nan = flm.clone()
+    nan[1, 3, L] = float("nan")
+    kernel = pc.construct.spin_spherical_kernel(L, 0, True, "healpix", nside, False) \
+        if L < 100 else None
+    calls = [lambda x: sph.inverse_hip(x, L, 0, nside, "healpix", True)]
+    if kernel is not None:
+        calls.append(lambda x: pc.spherical.inverse(x, L, 0, kernel, "healpix", True, nside=nside))
+    for call in calls:
+        one = [call(flm[b:b + 1])[0] for b in range(3)]
+        got, with_nan = call(flm), call(nan)
+        for b in range(3):
+            assert _own_error(got[b], one[b]) < TOL
+        for b in (0, 2):
+            assert _own_error(with_nan[b], one[b]) < TOL
