@@ -262,6 +262,11 @@ int zero_spec_pad(const s2h_plan* p, void* spec, int tiled, int batch, hipStream
                                          p->fwd_rows, p->spec_rows, tiled, batch, s));
 }
 
+// MW / MWSS forwards in BF16 project the 2L + 1 rows of MWSS at 2L.
+bool wide_rows(const s2h_plan* p, int precision) {
+  return p->fwd_kind != 0 && (precision == S2H_PREC_BF16 || precision == S2H_PREC_BF16X1);
+}
+
 int lat_forward_stage(const s2h_plan* p, const cplx* ftm, void* flm, int batch, int precision,
                       bool accumulate, hipStream_t s, bool packed = false,
                       const PlaneSet* ps = nullptr, const SpecView* sv = nullptr) {
@@ -283,6 +288,11 @@ int lat_forward_stage(const s2h_plan* p, const cplx* ftm, void* flm, int batch, 
   a.ftm_tiled = sv ? sv->tiled : 0;
   a.lmin_out = std::max(std::abs(p->d.spin), p->d.L_lower);
   if (bf16 || mixed) a.ucoef = p->fwd_rcoef;
+  const bool wide = wide_rows(p, precision);
+  if (wide) {
+    a.rings = p->wide_rings;
+    a.nrings = p->n_wide_rings;
+  }
   a.accumulate = accumulate ? 1 : 0;
   if (ps) a.planes = ps->fwd;
   const bool poles = p->fwd_row_south >= 0 || p->fwd_row_north >= 0;
@@ -319,13 +329,13 @@ int lat_forward_stage(const s2h_plan* p, const cplx* ftm, void* flm, int batch, 
     pa.flm = static_cast<cplx*>(flm);
     pa.flm_map_stride = fs;
     pa.ftm = const_cast<cplx*>(ftm);
-    pa.ftm_map_stride = ftm_stride;
+    pa.ftm_map_stride = a.ftm_map_stride;
     pa.ftm_ncol = p->Mc;
     pa.ftm_m_first = p->m_lo;
     pa.L = L;
     pa.spin = p->d.spin;
     pa.lmin = a.lmin_out;
-    pa.row_south = p->fwd_row_south;
+    pa.row_south = wide ? p->pc_rows - 1 : p->fwd_row_south;
     pa.row_north = p->fwd_row_north;
     pa.norm = p->fwd_norm;
     pa.batch = batch;
@@ -419,8 +429,9 @@ int lat_inverse_stage(const s2h_plan* p, const void* flm, cplx* ftm, int batch, 
 // The theta step of the MW / MWSS forward: phi-spectra of the input rows
 // `spec` to the projection's rows `ftm` (or, adjoint, back).
 int theta_mix_stage(const s2h_plan* p, const PlaneSet* ps, cplx* spec, cplx* ftm, int batch,
-                    bool adjoint, hipStream_t s, bool tiled = false) {
-  const int64_t spec_map = (int64_t)p->fwd_in_rows * p->Mc, ftm_map = (int64_t)p->fwd_rows * p->Mc;
+                    bool adjoint, hipStream_t s, bool tiled = false, bool wide = false) {
+  const int64_t spec_map = (int64_t)p->fwd_in_rows * p->Mc,
+                ftm_map = (int64_t)(wide ? p->pc_rows : p->fwd_rows) * p->Mc;
   ThetaMixArgs t{};
   t.in = adjoint ? ftm : spec;
   t.in_map_stride = adjoint ? ftm_map : spec_map;
@@ -431,6 +442,7 @@ int theta_mix_stage(const s2h_plan* p, const PlaneSet* ps, cplx* spec, cplx* ftm
   t.spin = ps ? ps->spin0 : p->d.spin;
   t.spin_step = ps ? ps->spin_step : 0;
   t.adjoint = adjoint ? 1 : 0;
+  t.wide = wide ? 1 : 0;
   t.nyquist = p->d.reality ? 0 : 1;
   t.out_tiled = tiled ? 1 : 0;
   ProfScope prof(S2H_KERNEL_RESAMPLE, s);
@@ -466,8 +478,10 @@ int forward_impl(const s2h_plan* p, const PlaneSet* ps, const void* f, int f_is_
   if (!resample) return lat_forward_stage(p, ftm, flm, batch, precision, accumulate, s, false, ps);
   // The FP64 projections gather single columns: in blocks of 8 rows a column is
   // made of 128-byte runs, ring-major of one value per line.
-  const SpecView sv{(int64_t)p->fwd_rows * p->Mc, precision == S2H_PREC_FP64 ? 1 : 0};
-  if ((st = theta_mix_stage(p, ps, spec, ftm, batch, false, s, sv.tiled != 0))) return st;
+  const bool wide = wide_rows(p, precision);
+  const SpecView sv{(int64_t)(wide ? p->pc_rows : p->fwd_rows) * p->Mc,
+                    precision == S2H_PREC_FP64 ? 1 : 0};
+  if ((st = theta_mix_stage(p, ps, spec, ftm, batch, false, s, sv.tiled != 0, wide))) return st;
   return lat_forward_stage(p, ftm, flm, batch, precision, accumulate, s, false, ps, &sv);
 }
 

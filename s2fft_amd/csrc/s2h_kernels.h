@@ -426,7 +426,7 @@ struct ResampleArgs {
 hipError_t launch_resample(const ResampleArgs& a, int batch, hipStream_t s);
 hipError_t allow_large_lds_resample();
 
-// MW / MWSS forward: input rows -> the L + 1 weighted rows the projection
+// MW / MWSS forward: input rows -> the L + 1 (wide: 2L + 1) weighted rows the projection
 // takes (or, adjoint, back), columns of both parities (s2h_theta_mix.hip).
 struct ThetaMix;
 struct ThetaMixArgs {
@@ -437,6 +437,7 @@ struct ThetaMixArgs {
   int ncol, m_lo;           // columns of both arrays
   int spin, spin_step;      // map b has spin + spin_step b
   int adjoint;
+  int wide;                 // forward: the 2L + 1 rows of MWSS at 2L
   int nyquist;              // complex signals: the theta-Nyquist term at q = -L
   int out_tiled;            // out in blocks of 8 rows (spec_row)
 };

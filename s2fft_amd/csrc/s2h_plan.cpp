@@ -594,6 +594,11 @@ static int plan_build(s2h_plan* p) {
     }
   }
   p->pc_rows = p->fwd_kind == 0 ? p->fwd_rows : 2 * L + 1;
+  std::vector<double> thf_rows = thi;  // of the pc_rows
+  if (p->fwd_kind != 0) {
+    thf_rows.clear();
+    for (int t = 0; t <= 2 * L; ++t) thf_rows.push_back(2.0 * t * M_PI / (4.0 * L));
+  }
 
   // ---------------- recursion tables
   std::vector<MStart> msf, msi;
@@ -613,6 +618,11 @@ static int plan_build(s2h_plan* p) {
   p->n_inv_rings = (int)inv_r.size();
   if ((st = upload(p, fwd_r, &p->fwd_rings))) return st;
   p->n_fwd_rings = (int)fwd_r.size();
+  if (p->fwd_kind != 0) {
+    const std::vector<LatRing> wide = lat_rings(thf_rows, 1, 2 * L - 1, pair_ok);
+    if ((st = upload(p, wide, &p->wide_rings))) return st;
+    p->n_wide_rings = (int)wide.size();
+  }
   if ((st = make_set(p, inv_j, &p->inv_set))) return st;
   if ((st = make_set(p, fwd_j, &p->fwd_set))) return st;
   {
@@ -675,12 +685,6 @@ static int plan_build(s2h_plan* p) {
   if ((st = upload(p, nf, &p->fwd_norm))) return st;
   if ((st = upload(p, ni, &p->inv_norm))) return st;
   {
-    std::vector<double> thf_rows;
-    if (p->fwd_kind == 0) {
-      thf_rows = thi;
-    } else {
-      for (int t = 0; t <= 2 * L; ++t) thf_rows.push_back(2.0 * t * M_PI / (4.0 * L));
-    }
     if ((st = upload(p, thf_rows, &p->fwd_theta))) return st;
     if ((st = upload(p, thi, &p->inv_theta))) return st;
     if ((st = upload(p, wf, &p->fwd_row_w))) return st;

@@ -20,6 +20,9 @@ struct s2h_plan {
   int fwd_in_rows = 0;  // rows of the phi-spectrum before the theta step (kinds 1, 2)
   std::shared_ptr<s2h::ThetaMix> mix;  // kinds 1, 2
   int pc_rows = 0;   // rows a stored forward kernel contracts: 2L + 1 (kinds 1, 2) or fwd_rows
+  // BF16 projections of kinds 1, 2: the rings of MWSS at 2L, pole rows 0 and 2L
+  s2h::LatRing* wide_rings = nullptr;
+  int n_wide_rings = 0;
   s2h::JobSet fwd_set;
   s2h::LatRing* fwd_rings = nullptr;
   int n_fwd_rings = 0;

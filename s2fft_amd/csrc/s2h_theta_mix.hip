@@ -34,6 +34,11 @@
 // errors: without this the forward's error at L = 512 was 5.8e-14 instead of
 // the 5.4e-14 of the 2L + 1 rings.)
 // The adjoint uses the transposed matrices.
+// The BF16 projections take the 2L + 1 rows w U instead (`wide`): their error is the
+// rounding of rows and d, which twice the rows average out by sqrt 2.  From L + 1 rows
+// the single BF16 projection had an error of 2.2e-3 instead of 1.5e-3, the split one
+// 4.1e-6 instead of 2.9e-6 (L = 24 to 1024).  Split BF16 forward, MW L = 512, 8 maps:
+// 677 us from 2L + 1 rows (493 from L + 1; the column FFT chain 7.9 ms).
 //
 // What bounds it: 8 L^2 flops per complex element of the column on
 // V_MFMA_F64_16X16X4F64.  The operators are shared by every map, spin and
@@ -177,6 +182,18 @@ __global__ void __launch_bounds__(kThreads) mix_add_kernel(int64_t n, const doub
     y[i] += x[i];
 }
 
+// U -> w U (times phi), and its rank-one vector w (-sin(L theta_t))
+__global__ void __launch_bounds__(kThreads) mix_weight_kernel(int L, int K, const double* w,
+                                                              double phi, double* u, double* su) {
+  const int64_t T = 2 * L + 1, n = 2 * T * K;
+  const int64_t i0 = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+  for (int64_t i = i0; i < n; i += (int64_t)gridDim.x * kThreads) u[i] *= phi * w[i / K % T];
+  for (int64_t i = i0; i < 2 * T; i += (int64_t)gridDim.x * kThreads) {
+    const int t = (int)(i % T);
+    su[i] = t & 1 ? ((t & 3) == 1 ? -phi : phi) * w[t] : 0.0;
+  }
+}
+
 // n (K entries) and s (L + 1 entries) of the rank-one Nyquist term per parity
 __global__ void __launch_bounds__(kThreads) mix_nyquist_kernel(int L, int K, int mw,
                                                                const double* pm, double* nv,
@@ -224,7 +241,7 @@ __global__ void __launch_bounds__(kGT * kGT) mix_product_kernel(int R, int T, in
 }
 
 // The interior rows come first, the pole rows last: position i -> MWSS row
-// (0 .. L).  An output tile of pole rows alone is wanted for two columns only.
+// (0 .. L, wide: 0 .. 2L).  An output tile of pole rows alone is wanted for two columns only.
 __host__ __device__ __forceinline__ int mix_row(int i, int L) {
   return i < L - 1 ? i + 1 : i == L - 1 ? L : 0;
 }
@@ -257,13 +274,15 @@ struct ThetaMix {
   int device = 0, L = 0, K = 0, mw = 0;
   double* fwd = nullptr;  // packed [parity][RT][KT][64]
   double* adj = nullptr;
+  double* wide = nullptr; // w U on the 2L + 1 rows of MWSS at 2L
   double* nv = nullptr;   // [parity][K]
   double* sv = nullptr;   // [parity][L + 1], MWSS row order
+  double* su = nullptr;   // [parity][2L + 1], for wide
   ~ThetaMix() {
     int cur = 0;
     (void)hipGetDevice(&cur);
     (void)hipSetDevice(device);
-    for (double* q : {fwd, adj, nv, sv})
+    for (double* q : {fwd, adj, wide, nv, sv, su})
       if (q) (void)hipFree(q);
     (void)hipSetDevice(cur);
   }
@@ -272,6 +291,7 @@ struct ThetaMix {
 namespace {
 int fwd_rt(int L) { return pad_to((L + 1 + 15) / 16, kRowTiles); }
 int fwd_kt(int K) { return pad_to((K + 3) / 4, kStepPad); }
+int wide_rt(int L) { return fwd_rt(2 * L); }
 int adj_rt(int K) { return pad_to((K + 15) / 16, kRowTiles); }
 int adj_kt(int L) { return pad_to((L + 1 + 3) / 4, kStepPad); }
 
@@ -301,10 +321,13 @@ int mix_build(ThetaMix* x, const std::vector<double>& weights, const std::vector
   double* sm = tmp.get(5, (int64_t)2 * (L + 1) * (L + 1));
   double* dc = tmp.get(6, 2 * T * (L + 1));
   const int64_t nf = (int64_t)2 * fwd_rt(L) * fwd_kt(K) * 64,
+                nw = (int64_t)2 * wide_rt(L) * fwd_kt(K) * 64,
                 na = (int64_t)2 * adj_rt(K) * adj_kt(L) * 64;
   if (!u || !pm || !c || !w || !dl || !sm || !dc ||
       hipMalloc(&x->fwd, sizeof(double) * nf) != hipSuccess ||
       hipMalloc(&x->adj, sizeof(double) * na) != hipSuccess ||
+      hipMalloc(&x->wide, sizeof(double) * nw) != hipSuccess ||
+      hipMalloc(&x->su, sizeof(double) * 2 * T) != hipSuccess ||
       hipMalloc(&x->nv, sizeof(double) * 2 * K) != hipSuccess ||
       hipMalloc(&x->sv, sizeof(double) * 2 * (L + 1)) != hipSuccess)
     return S2H_ERR_NOMEM;
@@ -333,6 +356,10 @@ int mix_build(ThetaMix* x, const std::vector<double>& weights, const std::vector
                      fwd_kt(K), 0, x->fwd);
   hipLaunchKernelGGL(mix_pack_kernel, blocks(na / 2), dim3(kThreads), 0, 0, L, K, c, adj_rt(K),
                      adj_kt(L), 1, x->adj);
+  hipLaunchKernelGGL(mix_weight_kernel, dim3(blocks(2 * T * K).x), dim3(kThreads), 0, 0, L, K, w,
+                     phi, u, x->su);
+  hipLaunchKernelGGL(mix_pack_kernel, blocks(nw / 2), dim3(kThreads), 0, 0, 2 * L, K, u,
+                     wide_rt(L), fwd_kt(K), 0, x->wide);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess) e = hipStreamSynchronize(0);
   return e == hipSuccess ? S2H_OK : S2H_ERR_HIP;
@@ -340,7 +367,10 @@ int mix_build(ThetaMix* x, const std::vector<double>& weights, const std::vector
 }  // namespace
 
 // The operators of (device, sampling, L), shared by every live plan that uses
-// them (they do not depend on the spin) and freed with the last one.
+// them (they do not depend on the spin) and freed with the last one.  They are built
+// with the plan, since the calls neither allocate nor wait: 64 L^2 bytes (the
+// projection's, its transpose for gradients, and twice that for BF16), 268 MB at L =
+// 2048, and 128 L^2 bytes of temporaries meanwhile.
 int theta_mix_get(int device, bool mw, int L, const std::vector<double>& weights,
                   const std::vector<double>& delta, std::shared_ptr<ThetaMix>* out) {
   std::lock_guard<std::mutex> lock(g_mix_mu);
@@ -374,7 +404,8 @@ struct MixKernelArgs {
   cplx* out;
   int64_t out_map_stride;
   int ncol, m_lo, spin, spin_step;
-  int L, K, R;              // input rows, output rows
+  int last;                 // of the MWSS rows on one side: rows 0 .. last
+  int K, R;                 // input rows, output rows
   int KT, KTpad, RT;        // K-steps in use, K-steps / row tiles of the packed operator
   int in_poles, out_poles;  // rows in mix_row order
   int out_tiled;            // out in blocks of 8 rows (spec_row)
@@ -402,7 +433,7 @@ __global__ void __launch_bounds__(256) theta_mix_kernel(MixKernelArgs a) {
   const int c0 = (2 * cb + (wave >> 1)) * (16 * NT);
   if (c0 >= a.ncol) return;
   const int r0 = rb * 16 * MT;
-  if (a.out_poles && r0 >= a.L - 1) {
+  if (a.out_poles && r0 >= a.last - 1) {
     // pole rows only: the pole terms read the columns m = +-spin
     const int cs = spin - a.m_lo, cn = -spin - a.m_lo;
     if (!(cs >= c0 && cs < c0 + 16 * NT) && !(cn >= c0 && cn < c0 + 16 * NT)) return;
@@ -432,7 +463,7 @@ __global__ void __launch_bounds__(256) theta_mix_kernel(MixKernelArgs a) {
   // (the rows past K repeat row K - 1's address)
   auto load = [&](int kt, double (&va)[MT], double (&vb)[NT], double& vq) {
     const int k = 4 * kt + kq;
-    const int row = mix_at(k < a.K ? k : a.K - 1, a.L, a.in_poles);
+    const int row = mix_at(k < a.K ? k : a.K - 1, a.last, a.in_poles);
     const int64_t ro = 2 * (int64_t)row * a.ncol;
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) va[mt] = ap[((int64_t)mt * a.KTpad + kt) * 64];
@@ -486,7 +517,7 @@ __global__ void __launch_bounds__(256) theta_mix_kernel(MixKernelArgs a) {
     for (int r = 0; r < 4; ++r) {
       const int i = r0 + 16 * mt + lat::Mma<double>::row_of(r, kq);
       if (i >= a.R) continue;
-      const int row = mix_at(i, a.L, a.out_poles);
+      const int row = mix_at(i, a.last, a.out_poles);
       const double pr = term ? a.p[par * a.R + row] : 0.0;
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) {
@@ -528,7 +559,7 @@ __global__ void __launch_bounds__(256, 2) theta_mix_lds_kernel(MixKernelArgs a) 
   const int par = wave & 1, half = wave >> 1;
   const int spin = a.spin + a.spin_step * b;
   const int c0 = cb * kMixCols, r0 = rb * kMixRows;
-  if (a.out_poles && r0 >= a.L - 1) {
+  if (a.out_poles && r0 >= a.last - 1) {
     // pole rows only: the pole terms read the columns m = +-spin
     const int cs = spin - a.m_lo, cn = -spin - a.m_lo;
     if (!(cs >= c0 && cs < c0 + kMixCols) && !(cn >= c0 && cn < c0 + kMixCols)) return;
@@ -547,7 +578,7 @@ __global__ void __launch_bounds__(256, 2) theta_mix_lds_kernel(MixKernelArgs a) 
   };
   // addresses: a uniform base per load plus the thread's own offset.  Input rows up to
   // `plain` follow their index (with poles: one further); the rest go through mix_at
-  const int plain = a.in_poles ? a.L - 1 : a.K;
+  const int plain = a.in_poles ? a.last - 1 : a.K;
   const unsigned boff = 16u * (unsigned)(sr * a.ncol + scol);
   unsigned aoff[2];
 #pragma unroll
@@ -568,7 +599,7 @@ __global__ void __launch_bounds__(256, 2) theta_mix_lds_kernel(MixKernelArgs a) 
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int k = kc * kMixK + sr + 4 * i;
-        v.b[i] = in[(int64_t)mix_at(k < a.K ? k : a.K - 1, a.L, a.in_poles) * a.ncol + scol];
+        v.b[i] = in[(int64_t)mix_at(k < a.K ? k : a.K - 1, a.last, a.in_poles) * a.ncol + scol];
       }
     }
 #pragma unroll
@@ -618,7 +649,7 @@ __global__ void __launch_bounds__(256, 2) theta_mix_lds_kernel(MixKernelArgs a) 
           acc[mt][nt] = lat::Mma<double>::run(ca[mt], cbv[nt], acc[mt][nt]);
       if (full) {
         const int k = kc * kMixK + 4 * u + kq;
-        const double cq = k < a.K ? qv[mix_at(k, a.L, a.in_poles)] : 0.0;
+        const double cq = k < a.K ? qv[mix_at(k, a.last, a.in_poles)] : 0.0;
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) accv[nt] = lat::Mma<double>::run(cq, cbv[nt], accv[nt]);
       }
@@ -666,7 +697,7 @@ __global__ void __launch_bounds__(256, 2) theta_mix_lds_kernel(MixKernelArgs a) 
     for (int r = 0; r < 4; ++r) {
       const int i = r0 + 16 * mt + lat::Mma<double>::row_of(r, kq);
       if (i >= a.R) continue;
-      const int row = mix_at(i, a.L, a.out_poles);
+      const int row = mix_at(i, a.last, a.out_poles);
       const double pr = term ? a.p[par * a.R + row] : 0.0;
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) {
@@ -710,11 +741,11 @@ hipError_t launch_theta_mix(const ThetaMix* x, const ThetaMixArgs& a, int batch,
   if (batch == 0 || a.ncol == 0) return hipSuccess;
   MixKernelArgs k{};
   const int L = x->L;
-  k.L = L;
+  k.last = a.wide ? 2 * L : L;
   k.K = a.adjoint ? L + 1 : x->K;
-  k.R = a.adjoint ? x->K : L + 1;
-  k.mat = a.adjoint ? x->adj : x->fwd;
-  k.RT = a.adjoint ? adj_rt(x->K) : fwd_rt(L);
+  k.R = a.adjoint ? x->K : k.last + 1;
+  k.mat = a.adjoint ? x->adj : a.wide ? x->wide : x->fwd;
+  k.RT = a.adjoint ? adj_rt(x->K) : fwd_rt(k.last);
   k.KTpad = a.adjoint ? adj_kt(L) : fwd_kt(x->K);
   k.KT = (k.K + 3) / 4;
   k.in_poles = a.adjoint;
@@ -730,7 +761,7 @@ hipError_t launch_theta_mix(const ThetaMix* x, const ThetaMixArgs& a, int batch,
   k.spin_step = a.spin_step;
   k.q = a.adjoint ? x->sv : x->nv;
   if (a.nyquist) {
-    k.p = a.adjoint ? x->nv : x->sv;
+    k.p = a.adjoint ? x->nv : a.wide ? x->su : x->sv;
     k.sgn = a.adjoint ? -1.0 : 1.0;
     // the term's n: none for even MW columns, one or two samples for odd ones
     k.vmode[0] = x->mw ? 0 : 2;

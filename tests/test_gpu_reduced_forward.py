@@ -1,0 +1,35 @@
+"""The error of MW / MWSS forwards in reduced precision (needs a GPU).
+
+A coefficient is a sum over rings of rounded d times rounded rows.  The roundings are
+independent, so that 2N rows leave 1 / sqrt 2 of the error of N rows (the terms are half
+as large).  Relative RMS over random coefficients, measured with the 2L + 1 rows of MWSS
+at 2L: single BF16 1.53e-3, split BF16 2.9e-6 at every L; with L + 1 rows 2.16e-3 and
+4.1e-6.  The bounds lie between the two.
+"""
+
+import pytest
+import torch
+
+from s2fft_amd.transforms import spherical as sph
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("sampling", ["mw", "mwss"])
+@pytest.mark.parametrize("L,batch,spin,reality", [
+    (24, 8, 0, False), (64, 8, 2, False), (101, 8, 0, True),
+    (256, 4, 2, False), (385, 4, 0, False), (385, 4, 0, True),
+    (512, 8, -1, False), (1024, 1, 0, False),
+])
+def test_rms_error(sampling, L, batch, spin, reality):
+    gen = torch.Generator().manual_seed(L)
+    flm = torch.randn((batch, L, 2 * L - 1), generator=gen, dtype=torch.complex128)
+    m, l = torch.arange(-(L - 1), L)[None, :], torch.arange(L)[:, None]
+    flm = flm * ((m.abs() <= l) & (l >= abs(spin)))
+    if reality:
+        flm = 0.5 * (flm + (1.0 - 2.0 * (m % 2)) * flm.flip(-1).conj())
+    flm = flm.cuda()
+    f = sph.inverse_hip(flm, L, spin, None, sampling, reality)
+    for precision, bound in (("bf16x1", 1.8e-3), ("bf16", 3.4e-6)):
+        got = sph.forward_hip(f, L, spin, None, sampling, reality, precision=precision)
+        assert float((got - flm).norm() / flm.norm()) < bound, precision
