@@ -102,7 +102,7 @@ int s2h_inverse(const s2h_plan *plan, const void *flm, void *f, void *work, int 
  * FFTs and every sum across waves stay FP64:
  * S2H_PREC_MIXED: the d-values and the ring (or flm) data are rounded to FP32
  *   and multiplied on the FP32 matrix cores with FP32 accumulation over one
- *   wave's 128 rings (forward) or one 32-l chunk (inverse); relative error
+ *   64 of a wave's rings (forward) or one 32-l chunk (inverse); relative error
  *   ~1e-7 of max |flm| for band-limited maps at L = 2048.
  * S2H_PREC_BF16: each operand split into two BF16 (hi + lo, 16 significant
  *   bits), products hi*hi + hi*lo + lo*hi on the BF16 matrix cores with FP32

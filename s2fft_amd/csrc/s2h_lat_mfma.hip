@@ -267,10 +267,15 @@ namespace {
 constexpr int kFW = 4;              // waves per workgroup, FP32 kernel
 constexpr int kFT = kFW * 64;       // threads
 constexpr int kFSets = 4;           // 64-pair sets per wave
+// FP32 sums per parity and element, met in FP64: a chain adds up 64 of the wave's 256
+// rings.  With two (128 rings) the L + 1 rows of MW / MWSS left up to 1.86e-7 (L =
+// 1024; the 2L + 1 rows of the column FFT chain 1.77e-7), with four 1.34e-7, HEALPix L
+// = 2048 1.80e-7 -> 1.27e-7, at 1 % of the time (7.74 -> 7.81 ms for 16 maps).
+constexpr int kFChains = 4;
 }  // namespace
 
 template <bool PAIRED, bool TILED>
-__global__ void __launch_bounds__(kFT) lat_forward_f32_kernel(LatArgs a) {
+__global__ void __launch_bounds__(kFT, 2) lat_forward_f32_kernel(LatArgs a) {
   typedef typename Mma<float>::acc acc_t;
   // per wave, two buffers of the d tiles [parity][pair][l_local]: set s goes
   // to buffer s % 2.  After the chunk's products buffer 0 holds the wave's
@@ -340,7 +345,9 @@ __global__ void __launch_bounds__(kFT) lat_forward_f32_kernel(LatArgs a) {
     const bool more = blk + 32 < L;
     if (more && threadIdx.x < lat::kChunk) cn = lat::load_ucoef_raw(cf, blk + 32, threadIdx.x, L);
     const lat::ChunkCoef* cs = ccs[buf];
-    acc_t acc_e[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}}, acc_o[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+    acc_t acc[2][kFChains];  // even and odd l
+#pragma unroll
+    for (int q = 0; q < kFChains; ++q) acc[0][q] = acc[1][q] = acc_t{0, 0, 0, 0};
     // recursion step i (0..31) of set s into buffer s % 2 (even offsets to
     // one tile, odd to the other)
     auto step = [&](int s, int i) {
@@ -363,8 +370,8 @@ __global__ void __launch_bounds__(kFT) lat_forward_f32_kernel(LatArgs a) {
       for (int c = 0; c < 16; ++c) {
         const float be = te[(4 * c + kq) * kPad + row];
         const float bo = to[(4 * c + kq) * kPad + row];
-        acc_e[c & 1] = Mma<float>::run(se[s][c], be, acc_e[c & 1]);
-        acc_o[c & 1] = Mma<float>::run(so[s][c], bo, acc_o[c & 1]);
+        acc[0][c % kFChains] = Mma<float>::run(se[s][c], be, acc[0][c % kFChains]);
+        acc[1][c % kFChains] = Mma<float>::run(so[s][c], bo, acc[1][c % kFChains]);
         if (s + 1 < kFSets) {
           step(s + 1, 2 * c);
           step(s + 1, 2 * c + 1);
@@ -376,8 +383,13 @@ __global__ void __launch_bounds__(kFT) lat_forward_f32_kernel(LatArgs a) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int i = Mma<float>::row_of(r, kq);
-      ctw[i * 16 + row] = (double)acc_e[0][r] + (double)acc_e[1][r];
-      ctw[256 + i * 16 + row] = (double)acc_o[0][r] + (double)acc_o[1][r];
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        double v = 0.0;
+#pragma unroll
+        for (int k = 0; k < kFChains; ++k) v += (double)acc[q][k][r];
+        ctw[256 * q + i * 16 + row] = v;
+      }
     }
     if (more && threadIdx.x < lat::kChunk) ccs[buf ^ 1][threadIdx.x] = lat::finish_coef(cn, bsign);
     __syncthreads();

@@ -159,7 +159,7 @@ def forward_hip(f, L, spin=0, nside=None, sampling="mw", reality=False, L_lower=
     """Batched forward on device tensors: f (B, ...) -> flm (B, L, 2L-1) complex128.
 
     ``precision``: "fp64" (default), "mixed" (FP64 recursion and ring FFTs,
-    FP32 matrix-core projection with FP32 accumulation over 128 rings),
+    FP32 matrix-core projection with FP32 accumulation over 64 rings),
     "bf16" (split-BF16 matrix-core projection, FP32 accumulation) or "bf16x1"
     (single-product BF16 projection, ~4e-3 relative: a refinement's
     correction transform).  ``accumulate_into``: an flm tensor (contiguous
