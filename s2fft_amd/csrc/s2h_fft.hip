@@ -16,8 +16,16 @@ __global__ void __launch_bounds__(kThreads) chirp_setup_kernel(const ChirpEntry*
   const int n = en.n, M = en.M;
   double* re = smem;
   double* im = smem + M;
-  if (blockIdx.x == 0)
-    for (int j = threadIdx.x; j < kBlueTwiddles; j += kThreads) pool[j] = expi_pi(-j, kMaxConvLen / 2);
+  if (blockIdx.x == 0) {
+    for (int j = threadIdx.x; j < kRingTwiddles; j += kThreads) {
+      const TwiddleOf w = ring_twiddle(j);
+      pool[j] = expi_pi(-2 * w.num, w.N);
+    }
+  }
+  if (en.ring == 2) {
+    for (int k = threadIdx.x; k < n; k += kThreads) pool[en.off + k] = expi_pi(-k, n);
+    return;
+  }
   for (int j = threadIdx.x; j < M; j += kThreads) {
     cplx v = {0.0, 0.0};
     if (j < n)
@@ -28,7 +36,7 @@ __global__ void __launch_bounds__(kThreads) chirp_setup_kernel(const ChirpEntry*
     im[j] = v.y;
   }
   __syncthreads();
-  fft_mixed<kFftMax>(re, im, M, -1);
+  fft_mixed<kFftMax, true>(re, im, M, -1);
   cplx* dst = pool + en.off;
   const double s = 1.0 / M;
   for (int j = threadIdx.x; j < M; j += kThreads)

@@ -101,8 +101,9 @@ struct SmallDft {
 // ------------------------------------------------------------ Stockham pass
 // One radix-R pass over n points; Ns = product of the radices already done.
 // Butterfly j reads in[j + r n/R], twists by exp(sign 2 pi i r (j mod Ns)/(Ns R)),
-// and writes out[(j div Ns) Ns R + (j mod Ns) + k Ns].
-template <int R, int MAXN>
+// and writes out[(j div Ns) Ns R + (j mod Ns) + k Ns].  EXACT: every twiddle evaluated,
+// not multiplied up (tables, whose error is in every transform that reads them).
+template <int R, int MAXN, bool EXACT>
 __device__ void stockham_pass(double* re, double* im, int n, int Ns, int sign) {
   constexpr int MAXB = (MAXN / R + kThreads - 1) / kThreads;
   const int nb = n / R;
@@ -131,7 +132,7 @@ __device__ void stockham_pass(double* re, double* im, int n, int Ns, int sign) {
 #pragma unroll
         for (int r = 1; r < R; ++r) {
           v[c][r] = cmul(v[c][r], wr);
-          if (r + 1 < R) wr = cmul(wr, w1);
+          if (r + 1 < R) wr = EXACT ? expi_pi((int64_t)2 * sign * jl * (r + 1), Ns * R) : cmul(wr, w1);
         }
       }
       SmallDft<R>::run(v[c], sign, w);
@@ -157,33 +158,33 @@ __device__ void stockham_pass(double* re, double* im, int n, int Ns, int sign) {
 
 // Mixed-radix FFT in place, all prime factors of n must be <= 13.
 // sign = -1: X[k] = sum_p x[p] e^{-2 pi i k p/n};  sign = +1: unnormalised inverse.
-template <int MAXN>
+template <int MAXN, bool EXACT = false>
 __device__ void fft_mixed(double* re, double* im, int n, int sign) {
   int rem = n, Ns = 1;
   while (rem > 1) {
     if (rem % 8 == 0) {
-      stockham_pass<8, MAXN>(re, im, n, Ns, sign);
+      stockham_pass<8, MAXN, EXACT>(re, im, n, Ns, sign);
       Ns *= 8; rem /= 8;
     } else if (rem % 4 == 0) {
-      stockham_pass<4, MAXN>(re, im, n, Ns, sign);
+      stockham_pass<4, MAXN, EXACT>(re, im, n, Ns, sign);
       Ns *= 4; rem /= 4;
     } else if (rem % 2 == 0) {
-      stockham_pass<2, MAXN>(re, im, n, Ns, sign);
+      stockham_pass<2, MAXN, EXACT>(re, im, n, Ns, sign);
       Ns *= 2; rem /= 2;
     } else if (rem % 3 == 0) {
-      stockham_pass<3, MAXN>(re, im, n, Ns, sign);
+      stockham_pass<3, MAXN, EXACT>(re, im, n, Ns, sign);
       Ns *= 3; rem /= 3;
     } else if (rem % 5 == 0) {
-      stockham_pass<5, MAXN>(re, im, n, Ns, sign);
+      stockham_pass<5, MAXN, EXACT>(re, im, n, Ns, sign);
       Ns *= 5; rem /= 5;
     } else if (rem % 7 == 0) {
-      stockham_pass<7, MAXN>(re, im, n, Ns, sign);
+      stockham_pass<7, MAXN, EXACT>(re, im, n, Ns, sign);
       Ns *= 7; rem /= 7;
     } else if (rem % 11 == 0) {
-      stockham_pass<11, MAXN>(re, im, n, Ns, sign);
+      stockham_pass<11, MAXN, EXACT>(re, im, n, Ns, sign);
       Ns *= 11; rem /= 11;
     } else if (rem % 13 == 0) {
-      stockham_pass<13, MAXN>(re, im, n, Ns, sign);
+      stockham_pass<13, MAXN, EXACT>(re, im, n, Ns, sign);
       Ns *= 13; rem /= 13;
     } else {
       return;  // unreachable for supported lengths (checked on the host)

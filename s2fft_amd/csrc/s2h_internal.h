@@ -23,22 +23,24 @@ struct RingJob {
   int32_t row;          // row of the ftm array this ring maps to
   double phi0_over_pi;  // azimuth of the first pixel / pi
   double weight;        // quadrature weight applied by the forward FFT
-  int32_t conv_len;     // 0: the power-of-two length; else Bluestein length M
-  int32_t pad;
+  int32_t conv_len;     // 0: the grid's power-of-two length; else Bluestein length M
+  int32_t sub;          // another power of two, on the threads of a ring of conv_len
   int64_t chirp_off;    // offset (complex elements) of the length's tables in the chirp pool
 };
 
 // Ring jobs of one transform on the device: n_pow2 rings of one power-of-two
-// length, then n_blue Bluestein rings (by decreasing convolution length).
+// length, then the rest by decreasing convolution length, of each the Bluestein
+// rings and then the shorter powers of two.
 constexpr int kBlueLogMin = 6;   // convolutions of 64 ...
 constexpr int kBlueClasses = 8;  // ... to 8192 = kMaxConvLen points
 
 struct JobSet {
   RingJob* jobs = nullptr;
-  int n_pow2 = 0, n_blue = 0;
+  int n_pow2 = 0, n_rest = 0;
   int blue[kBlueClasses] = {};  // Bluestein rings by convolution length 64 << class
+  int sub[kBlueClasses] = {};   // shorter powers of two likewise
   int log_pow2 = 0;     // log2 of the power-of-two length
-  int min_blue = 0;     // shortest Bluestein ring
+  int min_rest = 0;     // shortest ring of the rest
   int max_nphi = 0;     // longest ring
 };
 

@@ -222,12 +222,23 @@ hipError_t launch_ring_alias_sumsq(const RingAliasArgs& a, const JobSet& js, int
                                    double* part, double* sumsq, hipStream_t s);
 hipError_t launch_ring_dot(const RingAliasArgs& a, const JobSet& js, int batch, double* part,
                            const double* num, double* pq, double* alpha, hipStream_t s);
-// Chirp pool.  It starts with kBlueTwiddles twiddles e^{-2 pi i j / 8192}; then
-// per length n with convolution M either (ring 0: the stored-kernel resampling)
-// FFT_M(b) / M, b_j = e^{i pi j^2 / n}, or (ring 1: the Bluestein ring kernels)
-// FFT_M(b) / M at the places blue_place(k, M), the n chirps e^{-i pi k^2 / n} and
-// the n phases e^{-i pi k / n}.
-constexpr int kBlueTwiddles = 512;
+// Chirp pool.  It starts with the twiddles of the ring kernels' radix-16 passes: for N
+// = 32, 64 .. 8192 and T = N / 16, from 4 (T - 2) on, e^{-2 pi i t c / N} for c = 1, 2, 4
+// and 8, t < T (ring_twiddle: the j-th entry).  Then per length n with convolution M
+// either (ring 0: the stored-kernel resampling) FFT_M(b) / M, b_j = e^{i pi j^2 / n}, or
+// (ring 1: the Bluestein ring kernels) FFT_M(b) / M at the places blue_place(k, M), the
+// n chirps e^{-i pi k^2 / n} and the n phases e^{-i pi k / n}, or (ring 2: powers of
+// two) the phases alone.
+constexpr int kRingTwiddles = 4 * (kMaxConvLen / 8 - 2);
+struct TwiddleOf {
+  int num, N;  // e^{-2 pi i num / N}
+};
+__host__ __device__ inline TwiddleOf ring_twiddle(int j) {
+  int T = 2;
+  while (4 * (2 * T - 2) <= j) T *= 2;
+  const int k = j - 4 * (T - 2);
+  return {(k % T) << (k / T), 16 * T};
+}
 struct ChirpEntry {
   int n, M, ring, pad;
   int64_t off;

@@ -288,7 +288,7 @@ int next_pow2(int v) {
 
 struct ChirpBuilder {
   std::map<std::tuple<int, int, int>, int64_t> table;  // (n, M, ring) -> offset
-  int64_t total = kBlueTwiddles;
+  int64_t total = kRingTwiddles;
   int max_conv = 0;
   // Returns the convolution length of an n-point column DFT (0 = mixed radix)
   // and sets the offset of its tables.
@@ -300,12 +300,14 @@ struct ChirpBuilder {
   int add_ring(int n, int64_t* off, int min_m) {
     return insert(n, next_pow2(std::max(std::max(2 * n - 1, 1 << kBlueLogMin), min_m)), 1, off);
   }
+  // The phases of an n-point ring that is transformed as a power of two.
+  void add_sub(int n, int64_t* off) { insert(n, 0, 2, off); }
   int insert(int n, int M, int ring, int64_t* off) {
     const auto key = std::make_tuple(n, M, ring);
     auto it = table.find(key);
     if (it == table.end()) {
       it = table.emplace(key, total).first;
-      total += M + (ring ? 2 * n : 0);
+      total += M + (ring == 1 ? 2 * n : ring == 2 ? n : 0);
       max_conv = std::max(max_conv, M);
     }
     *off = it->second;
@@ -345,8 +347,8 @@ struct ChirpBuilder {
   }
 };
 
-// A grid's one power-of-two length pow2 (0: none) runs as such from 64 points
-// on, every other ring by Bluestein.
+// A grid's one power-of-two length pow2 (0: none) runs in registers from 64 points
+// on, other powers of two in LDS, every other ring by Bluestein.
 RingJob make_job(int64_t off, int nphi, int row, double phi0, double w, ChirpBuilder& cb, int pow2,
                  int min_m = 0) {
   RingJob j{};
@@ -356,7 +358,14 @@ RingJob make_job(int64_t off, int nphi, int row, double phi0, double w, ChirpBui
   j.phi0_over_pi = phi0;
   j.weight = w;
   const bool direct = nphi == pow2 && (nphi & (nphi - 1)) == 0 && nphi >= 64;
-  if (!direct) j.conv_len = cb.add_ring(nphi, &j.chirp_off, min_m);
+  if (direct) return j;
+  if ((nphi & (nphi - 1)) == 0) {
+    j.sub = 1;
+    j.conv_len = next_pow2(std::max(std::max(2 * nphi, 1 << kBlueLogMin), min_m));
+    cb.add_sub(nphi, &j.chirp_off);
+  } else {
+    j.conv_len = cb.add_ring(nphi, &j.chirp_off, min_m);
+  }
   return j;
 }
 
@@ -365,8 +374,8 @@ RingJob make_job(int64_t off, int nphi, int row, double phi0, double w, ChirpBui
 // each, and the short rings share one launch.
 int ragged_min_conv(int ncol) { return std::min(next_pow2(ncol), kMaxConvLen); }
 
-// Orders the jobs (the power of two, then Bluestein by decreasing convolution
-// length, longest rings first) and uploads them.
+// Orders the jobs (the power of two, then by decreasing convolution length, Bluestein
+// before the shorter powers of two, longest rings first) and uploads them.
 int blue_class(int M) {
   int c = 0;
   while ((1 << (kBlueLogMin + c)) < M) ++c;
@@ -376,7 +385,8 @@ int blue_class(int M) {
 int make_set(s2h_plan* p, std::vector<RingJob> jobs, JobSet* out) {
   std::stable_sort(jobs.begin(), jobs.end(), [](const RingJob& x, const RingJob& y) {
     if ((x.conv_len == 0) != (y.conv_len == 0)) return x.conv_len == 0;
-    return x.conv_len != y.conv_len ? x.conv_len > y.conv_len : x.nphi > y.nphi;
+    if (x.conv_len != y.conv_len) return x.conv_len > y.conv_len;
+    return x.sub != y.sub ? x.sub < y.sub : x.nphi > y.nphi;
   });
   JobSet js;
   for (auto& j : jobs) {
@@ -385,9 +395,9 @@ int make_set(s2h_plan* p, std::vector<RingJob> jobs, JobSet* out) {
       ++js.n_pow2;
       while ((1 << js.log_pow2) < j.nphi) ++js.log_pow2;
     } else {
-      ++js.n_blue;
-      ++js.blue[blue_class(j.conv_len)];
-      js.min_blue = js.n_blue == 1 ? j.nphi : std::min(js.min_blue, j.nphi);
+      ++js.n_rest;
+      ++(j.sub ? js.sub : js.blue)[blue_class(j.conv_len)];
+      js.min_rest = js.n_rest == 1 ? j.nphi : std::min(js.min_rest, j.nphi);
     }
   }
   const int st = upload<RingJob>(p, jobs, &js.jobs);

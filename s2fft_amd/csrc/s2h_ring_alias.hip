@@ -570,7 +570,7 @@ constexpr int kTpbAlias = 256;
 }  // namespace
 
 hipError_t launch_ring_alias(const RingAliasArgs& a, const JobSet& js, int batch, hipStream_t s) {
-  const int njobs = js.n_pow2 + js.n_blue;
+  const int njobs = js.n_pow2 + js.n_rest;
   if (batch == 0 || njobs == 0) return hipSuccess;
   RingAliasArgs b = a;
   b.jobs = js.jobs;
@@ -597,7 +597,7 @@ hipError_t launch_ring_alias_sumsq(const RingAliasArgs& a, const JobSet& js, int
   return hipGetLastError();
 }
 
-int ring_dot_jobs(const JobSet& js) { return js.n_pow2 + js.n_blue; }
+int ring_dot_jobs(const JobSet& js) { return js.n_pow2 + js.n_rest; }
 int ring_dot_tiled_parts(int nblocks) { return nblocks * kAliasSlots; }
 namespace {
 // both tiled alias kernels over their blocks (part: null, or the per-block slots)

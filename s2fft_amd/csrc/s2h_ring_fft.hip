@@ -8,10 +8,15 @@
 //   F_t[q] = sum_{m = q mod nphi} exp(+i m phi0_t) c(m), f_t[p] = sum_q F_t[q] e^{2 pi i q p/nphi}
 //   the folding and the phase are fused into the load.
 //
-// Two kinds of rings: the grid's one power-of-two length as such, every other
-// length by Bluestein's chirp-z (Bluestein 1970).  Lengths with small prime
-// factors too: with a mixed-radix LDS kernel for those the grid of nside 192,
-// five maps, took 109 us and 62 without it.
+// Three kinds of rings: the grid's one power-of-two length as such (from 64 points on),
+// other powers of two in passes through LDS, every other length by Bluestein's chirp-z
+// (Bluestein 1970).  Lengths with small prime factors too: with a mixed-radix LDS
+// kernel for those the grid of nside 192, five maps, took 109 us and 62 without it.
+// RMS error of a ring against extended precision, the former LDS kernels (radix 8, odd
+// primes to 13, convolutions) beside it: powers of two 1.9e-16 at 256 points (2.6e-16)
+// and 2.4e-16 at 4096 (4.5e-16); other lengths 3.5e-16 below 64 points (4.5e-16 and
+// more), 4.4e-16 below 1100 (smooth lengths 13.8e-16, others 7.3e-16) and 4.9e-16 above
+// (18.8e-16, 8.8e-16).  Powers of two as convolutions would have 2 to 4 times theirs.
 // Two real maps share one complex transform (z = x + i y, split by the
 // conjugate symmetry of the spectra), halving the transforms for real data.
 //
@@ -31,7 +36,9 @@
 // stored in the order of the registers.  Four barriers per convolution; the
 // zero upper half of the input and the unwanted upper half of the output are
 // left out of the first and last pass.
-// Chirps, FFT(chirp) and twiddles come from the plan's table.
+// Chirps, FFT(chirp) and twiddles come from the plan's table, every one rounded from its
+// own evaluation: FFT(chirp) from a transform with multiplied-up twiddles, and twiddles
+// multiplied up here, left 1.6 times the error.
 //
 // What bounds it: the large grids their HBM traffic (64 maps of L = 512 MW, 1.07
 // GB: 0.38 ms forward and 0.40 inverse, 2.8 TB/s; the former LDS kernels with
@@ -156,10 +163,23 @@ __device__ __forceinline__ void dft16(cplx* v) {
   for (int k = 0; k < (HALF_OUT ? 8 : 16); ++k) v[k] = x[k];
 }
 
-// v[k] *= w^k (INV: conj w^k), the powers by products of depth 4
+// w, w^2, w^4 and w^8 of w = e^{-2 pi i t / 2^LOG}, t < T = 2^LOG / 16, from the
+// plan's table (ring_twiddles), each rounded once.
+struct Tw16 {
+  cplx w, w2, w4, w8;
+};
+__device__ __forceinline__ Tw16 load_tw16(const cplx* __restrict__ tab, int T, int t) {
+  const cplx* p = tab + 4 * (T - 2) + t;
+  return {p[0], p[T], p[2 * T], p[3 * T]};
+}
+
+// v[k] *= w^k (INV: conj w^k), the other powers by products of depth 2 at most.
+// Squared up from w alone they carry up to 15 times its rounding error: rings of 256
+// points had 3.6e-16 of RMS error instead of 1.9e-16, of 4096 5.2e-16 instead of 2.4e-16
+// (MW L = 512, 64 maps, inverse rings 434 -> 443 us; nside 512, one map, unchanged).
 template <bool INV>
-__device__ __forceinline__ void twiddle16(cplx* v, cplx w) {
-  const cplx w2 = cmul(w, w), w4 = cmul(w2, w2), w8 = cmul(w4, w4);
+__device__ __forceinline__ void twiddle16(cplx* v, const Tw16& q) {
+  const cplx w = q.w, w2 = q.w2, w4 = q.w4, w8 = q.w8;
   v[1] = tmul<INV>(v[1], w);
   v[2] = tmul<INV>(v[2], w2);
   v[4] = tmul<INV>(v[4], w4);
@@ -202,10 +222,6 @@ struct Shape {
 // powers, LDS places) is computed again and not held in registers meanwhile.
 __device__ __forceinline__ int renew(int x) {
   asm volatile("" : "+v"(x));
-  return x;
-}
-__device__ __forceinline__ cplx renew(cplx x) {
-  asm volatile("" : "+v"(x.x), "+v"(x.y));
   return x;
 }
 
@@ -253,7 +269,7 @@ __device__ __forceinline__ void blue_conv(cplx* v, cplx* lds, int t0, const cplx
   typedef Shape<LOGM> P;
   constexpr int T = P::T, S = P::S;
   int t = t0;
-  const cplx w1 = tw[t << (13 - LOGM)];  // e^{-2 pi i t / M}
+  const Tw16 w1 = load_tw16(tw, T, t);  // of e^{-2 pi i t / M}
   dft16<false, true, false>(v);
   twiddle16<false>(v, w1);
 #pragma unroll
@@ -271,7 +287,6 @@ __device__ __forceinline__ void blue_conv(cplx* v, cplx* lds, int t0, const cplx
     for (int i = 0; i < 16; ++i) lds[P::at((t + T * (i / S)) * S + i % S)] = v[i];
   } else {
     int nn = t % S, base = (t / S) * T + nn;
-    const cplx w2 = S > 1 ? tw[nn << (17 - LOGM)] : cplx{1.0, 0.0};  // e^{-2 pi i nn / T}
 #pragma unroll
     for (int i = 0; i < 16; ++i) v[i] = lds[P::at(base + i * S)];
     dft16<false, false, false>(v);
@@ -279,7 +294,7 @@ __device__ __forceinline__ void blue_conv(cplx* v, cplx* lds, int t0, const cplx
 #pragma unroll
       for (int i = 0; i < 16; ++i) v[i] = cmul(v[i], bhat[i * T + t]);
     } else {
-      twiddle16<false>(v, w2);
+      twiddle16<false>(v, load_tw16(tw, S, nn));  // of e^{-2 pi i nn / T}
 #pragma unroll
       for (int i = 0; i < 16; ++i) lds[P::at(base + i * S)] = v[i];
       __syncthreads();
@@ -316,23 +331,25 @@ __device__ __forceinline__ void blue_conv(cplx* v, cplx* lds, int t0, const cplx
 #pragma unroll
         for (int i = 0; i < 16; ++i) lds[P::at((t >> 1) * 32 + (t & 1) + 2 * i)] = v[i];
       }
-      __syncthreads();
       nn = t % S;
       base = (t / S) * T + nn;
+      const Tw16 w2 = load_tw16(tw, S, nn);
+      __syncthreads();
 #pragma unroll
       for (int i = 0; i < 16; ++i) v[i] = lds[P::at(base + i * S)];
-      twiddle16<true>(v, renew(w2));
+      twiddle16<true>(v, w2);
     }
     dft16<true, false, false>(v);
     base = renew(base);
 #pragma unroll
     for (int i = 0; i < 16; ++i) lds[P::at(base + i * S)] = v[i];
   }
-  __syncthreads();
   t = renew(t);
+  const Tw16 w3 = load_tw16(tw, T, t);
+  __syncthreads();
 #pragma unroll
   for (int k = 0; k < 16; ++k) v[k] = lds[P::at(k * T + t)];
-  twiddle16<true>(v, renew(w1));
+  twiddle16<true>(v, w3);
   dft16<true, false, true>(v);
 }
 
@@ -356,8 +373,9 @@ template <int LOGN, bool INV>
 __device__ __forceinline__ void pow2_fft(cplx* v, cplx* lds, int t, const cplx* __restrict__ tw) {
   typedef Pow2Shape<LOGN> P;
   constexpr int T = P::T, S = P::S;
+  const Tw16 w1 = load_tw16(tw, T, t);
   dft16<INV, false, false>(v);
-  twiddle16<INV>(v, tw[t << (13 - LOGN)]);
+  twiddle16<INV>(v, w1);
 #pragma unroll
   for (int k = 0; k < 16; ++k) lds[P::at(k * T + t)] = v[k];
   __syncthreads();
@@ -367,7 +385,7 @@ __device__ __forceinline__ void pow2_fft(cplx* v, cplx* lds, int t, const cplx* 
     for (int i = 0; i < 16; ++i) v[i] = lds[P::at(base + i * S)];
     dft16<INV, false, false>(v);
     if constexpr (S > 1) {
-      twiddle16<INV>(v, tw[nn << (17 - LOGN)]);
+      twiddle16<INV>(v, load_tw16(tw, S, nn));
 #pragma unroll
       for (int i = 0; i < 16; ++i) lds[P::at(base + i * S)] = v[i];
       __syncthreads();
@@ -405,8 +423,8 @@ __device__ __forceinline__ bool ring_phase(int apply, const RingJob& job) {
 
 // v[e] = pixel t + T e of the ring (z = x + i y for a pair of real maps), zero
 // from n on.
-template <int T, int E>
-__device__ __forceinline__ void load_pixels(cplx* v, const RingFwdArgs& a, const RingJob& job,
+template <int E>
+__device__ __forceinline__ void load_pixels(const int T, cplx* v, const RingFwdArgs& a, const RingJob& job,
                                             int t, int64_t b0, int paired, bool two) {
   const int n = job.nphi;
   const int64_t off = b0 * a.map_stride + job.pix_offset;
@@ -444,8 +462,8 @@ __device__ __forceinline__ void load_pixels(cplx* v, const RingFwdArgs& a, const
 
 // Stores a ring whose residues have at most one column each, from registers:
 // residue p = t + T e (phased) is column m = p or p - n.
-template <int T, int E>
-__device__ __forceinline__ void store_direct(const cplx* v, const RingFwdArgs& a,
+template <int E>
+__device__ __forceinline__ void store_direct(const int T, const cplx* v, const RingFwdArgs& a,
                                              const RingJob& job, int t, int64_t b0, bool ph) {
   const int n = job.nphi;
   cplx* d0 = a.out + b0 * a.out_map_stride + (int64_t)job.row * a.ncol;
@@ -462,8 +480,7 @@ __device__ __forceinline__ void store_direct(const cplx* v, const RingFwdArgs& a
 
 // Stores a ring's columns from its residues in LDS: [0, n), real pairs the
 // second map's at [n, 2n).  Column m = k + j n is (-1)^j times residue k (ph).
-template <int T>
-__device__ __forceinline__ void store_columns(const cplx* lds, const RingFwdArgs& a,
+__device__ __forceinline__ void store_columns(const int T, const cplx* lds, const RingFwdArgs& a,
                                               const RingJob& job, int t, int64_t b0, bool two,
                                               bool ph) {
   const int n = job.nphi;
@@ -498,8 +515,8 @@ __device__ __forceinline__ void store_columns(const cplx* lds, const RingFwdArgs
 // Natural-order residues v[e] (t + T e) into LDS for store_columns, times
 // phase(p); real pairs split into X = (z + conj z')/2, Y = (z - conj z')/(2i),
 // z' the residue n - p.  Called by every thread; ends on a barrier.
-template <int T, int E, typename Phase>
-__device__ __forceinline__ void residues_to_lds(cplx* v, cplx* lds, int n, int t, int paired,
+template <int E, typename Phase>
+__device__ __forceinline__ void residues_to_lds(const int T, cplx* v, cplx* lds, int n, int t, int paired,
                                                 Phase phase) {
   __syncthreads();
 #pragma unroll
@@ -597,8 +614,8 @@ struct FoldIn {
   __device__ static int floor_div(int p, int q) { return p >= 0 ? p / q : -((q - 1 - p) / q); }
 
   // v[e] = F[t + T e], for rings longer than T
-  template <int T, int E>
-  __device__ __forceinline__ void owned(cplx* v, int t) const {
+  template <int E>
+  __device__ __forceinline__ void owned(const int T, cplx* v, int t) const {
     if (hi - lo < n) {  // one m per residue
 #pragma unroll
       for (int e0 = 0; e0 < E; e0 += 8)
@@ -633,8 +650,7 @@ struct FoldIn {
   }
   // a thread's share of residue t % n, for rings of at most T points: the
   // G = T / n threads of a residue take j = j0 + g, j0 + g + G, ...
-  template <int T>
-  __device__ __forceinline__ cplx shared(int t) const {
+  __device__ __forceinline__ cplx shared(const int T, int t) const {
     cplx part = {0.0, 0.0};
     const int G = T / n, q = t % n, g = t / n;
     if (g >= G) return part;
@@ -650,11 +666,28 @@ struct FoldIn {
     }
     return part;
   }
+  // v[e] = F[t + T e], e < 8.  Called by every thread, with one barrier inside;
+  // another before lds is written again.
+  __device__ __forceinline__ void residues(const int T, cplx* v, cplx* lds, int t) const {
+    cplx part = {0.0, 0.0};
+    if (n > T) {
+      owned<8>(T, v, t);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = {0.0, 0.0};
+      part = shared(T, t);
+    }
+    lds[t] = part;
+    __syncthreads();
+    if (n <= T && t < n) {
+      for (int g = 0; g < T / n; ++g) v[0] = cadd(v[0], lds[g * n + t]);
+    }
+  }
 };
 
 // Stores pixel t + T e from v[e]; with sub_from the result is subtracted from it.
-template <int T, int E>
-__device__ __forceinline__ void store_pixels(cplx* v, const RingInvArgs& a, const RingJob& job,
+template <int E>
+__device__ __forceinline__ void store_pixels(const int T, cplx* v, const RingInvArgs& a, const RingJob& job,
                                              int t, int64_t b0, int paired, bool two, bool herm) {
   const int n = job.nphi;
   const int64_t off = b0 * a.map_stride + job.pix_offset;
@@ -707,13 +740,14 @@ __device__ __forceinline__ void store_pixels(cplx* v, const RingInvArgs& a, cons
 // Consecutive jobs of one kind within a launch: blocks [block0, ...) hold
 // blockDim / T rings each.
 struct RingSeg {
-  int body;      // log2 of the convolution (Bluestein), or kPow2Body + log2 n
+  int body;      // log2 of the convolution (Bluestein), kPow2Body + log2 n, or
+                 // kSubBody + log2 of the convolution whose threads it takes
   int job0, count, block0;
   int direct;    // forward: every residue has at most one column (ring_direct)
   int lds_ring;  // complex of LDS per ring
 };
-constexpr int kPow2Body = 32;
-constexpr int kMaxSegs = kBlueClasses + 1;
+constexpr int kPow2Body = 32, kSubBody = 64;
+constexpr int kMaxSegs = 2 * kBlueClasses + 1;
 constexpr int kRingLdsMax = 160 * 1024;
 struct RingSegs {
   RingSeg s[kMaxSegs];
@@ -721,14 +755,13 @@ struct RingSegs {
 };
 
 // the ring of this thread, and its place in it
-template <int T>
 struct RingOf {
   int t, sub;
   bool valid, two;
   int64_t b0;
   RingJob job;
   cplx* lds;
-  __device__ RingOf(const RingJob* jobs, const RingSeg& seg, int paired, int batch, void* raw) {
+  __device__ RingOf(const int T, const RingJob* jobs, const RingSeg& seg, int paired, int batch, void* raw) {
     t = threadIdx.x % T;
     sub = threadIdx.x / T;
     const int r = (blockIdx.x - seg.block0) * (blockDim.x / T) + sub;
@@ -745,7 +778,7 @@ __device__ __forceinline__ void blue_fwd(const RingFwdArgs& a, const RingSeg& se
                                          void* raw) {
   typedef Shape<LOGM> P;
   constexpr int T = P::T;
-  const RingOf<T> ring(a.jobs, seg, paired, a.batch, raw);
+  const RingOf ring(T, a.jobs, seg, paired, a.batch, raw);
   const RingJob& job = ring.job;
   cplx* lds = ring.lds;
   const int n = job.nphi;
@@ -755,7 +788,7 @@ __device__ __forceinline__ void blue_fwd(const RingFwdArgs& a, const RingSeg& se
   const cplx* __restrict__ phase = chirp + n;
 
   cplx v[16];
-  load_pixels<T, 8>(v, a, job, t, ring.b0, paired, ring.two);
+  load_pixels<8>(T, v, a, job, t, ring.b0, paired, ring.two);
   cplx c[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
@@ -776,13 +809,13 @@ __device__ __forceinline__ void blue_fwd(const RingFwdArgs& a, const RingSeg& se
   }
   const bool ph = ring_phase(a.apply_phase, job);
   if (seg.direct) {
-    if (ring.valid) store_direct<T, 8>(v, a, job, t, ring.b0, false);
+    if (ring.valid) store_direct<8>(T, v, a, job, t, ring.b0, false);
     return;
   }
-  residues_to_lds<T, 8>(v, lds, n, t, paired, [&](int e, cplx z) {
+  residues_to_lds<8>(T, v, lds, n, t, paired, [&](int e, cplx z) {
     return ph ? cmul(z, phase[t + T * e]) : z;
   });
-  if (ring.valid) store_columns<T>(lds, a, job, t, ring.b0, ring.two, ph);
+  if (ring.valid) store_columns(T, lds, a, job, t, ring.b0, ring.two, ph);
 }
 
 template <int LOGM>
@@ -790,7 +823,7 @@ __device__ __forceinline__ void blue_inv(const RingInvArgs& a, const RingSeg& se
                                          void* raw) {
   typedef Shape<LOGM> P;
   constexpr int T = P::T;
-  const RingOf<T> ring(a.jobs, seg, paired, a.batch, raw);
+  const RingOf ring(T, a.jobs, seg, paired, a.batch, raw);
   const RingJob& job = ring.job;
   cplx* lds = ring.lds;
   const int n = job.nphi;
@@ -801,19 +834,7 @@ __device__ __forceinline__ void blue_inv(const RingInvArgs& a, const RingSeg& se
   const FoldIn in(a, job, ring.b0, ring.two);
 
   cplx v[16];
-  cplx part = {0.0, 0.0};
-  if (n > T) {
-    in.template owned<T, 8>(v, t);
-  } else {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = {0.0, 0.0};
-    part = in.template shared<T>(t);
-  }
-  lds[t] = part;
-  __syncthreads();
-  if (n <= T && t < n) {
-    for (int g = 0; g < T / n; ++g) v[0] = cadd(v[0], lds[g * n + t]);
-  }
+  in.residues(T, v, lds, t);
   const double w = (a.apply_weight ? job.weight : 1.0) * ring_scale(a.norm_mode, n);
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
@@ -836,7 +857,111 @@ __device__ __forceinline__ void blue_inv(const RingInvArgs& a, const RingSeg& se
     const cplx z = cmul(v[e], p < n ? chirp[p] : cplx{0.0, 0.0});
     v[e] = {z.x, -z.y};
   }
-  store_pixels<T, 8>(v, a, job, t, ring.b0, paired, ring.two, in.herm);
+  store_pixels<8>(T, v, a, job, t, ring.b0, paired, ring.two, in.herm);
+}
+
+// Rings of another power of two, on the threads of a Bluestein ring (half of its points
+// at most): all T threads load, fold and store; the transform runs in self-sorting
+// passes through LDS, the first of radix 2, 4, 8 or 16 without twiddles, the others of
+// radix 16.  A HEALPix grid has two rings of each.
+template <int R, bool INV>
+__device__ __forceinline__ void sub_pass(const cplx* src, cplx* dst, const int T, int t, int n,
+                                         int Ns, const cplx* __restrict__ tw) {
+  const int nb = n / R;
+  for (int j = t; j < nb; j += T) {
+    cplx u[16];
+#pragma unroll
+    for (int r = 0; r < R; ++r) u[r] = src[j + r * nb];
+    const int jl = j & (Ns - 1);
+    if constexpr (R == 16) {
+      if (Ns > 1) twiddle16<INV>(u, load_tw16(tw, Ns, jl));
+      dft16<INV, false, false>(u);
+    }
+    if constexpr (R == 8) dft8<INV>(u);
+    if constexpr (R == 4) dft4<INV>(u[0], u[1], u[2], u[3]);
+    if constexpr (R == 2) dft2<INV>(u[0], u[1]);
+#pragma unroll
+    for (int k = 0; k < R; ++k) dst[(j - jl) * R + jl + k * Ns] = u[k];
+  }
+}
+// v[e] = x[t + T e] -> X[t + T e], e < 8, n <= 8 T <= 2048 points in 2 n of LDS.
+// Called by every thread; another barrier before lds is written again.
+template <bool INV>
+__device__ __forceinline__ void sub_fft(cplx* v, cplx* lds, const int T, int t, int n,
+                                        const cplx* __restrict__ tw) {
+#pragma unroll
+  for (int e = 0; e < 8; ++e)
+    if (t + T * e < n) lds[t + T * e] = v[e];
+  __syncthreads();
+  const int odd = (31 - __clz(n)) & 3;  // log2 of the first radix, 0: 16
+  cplx* src = lds;
+  cplx* dst = lds + n;
+  const int passes = T <= 32 ? 2 : 3;  // the same for every ring of the workgroup
+  int Ns = 1;
+#pragma unroll 1
+  for (int pass = 0; pass < passes; ++pass) {
+    if (Ns < n) {
+      const int lr = pass == 0 && odd ? odd : 4;
+      if (lr == 4)
+        sub_pass<16, INV>(src, dst, T, t, n, Ns, tw);
+      else if (lr == 3)
+        sub_pass<8, INV>(src, dst, T, t, n, Ns, tw);
+      else if (lr == 2)
+        sub_pass<4, INV>(src, dst, T, t, n, Ns, tw);
+      else
+        sub_pass<2, INV>(src, dst, T, t, n, Ns, tw);
+      cplx* x = src;
+      src = dst;
+      dst = x;
+      Ns <<= lr;
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int e = 0; e < 8; ++e) v[e] = t + T * e < n ? src[t + T * e] : cplx{0.0, 0.0};
+}
+
+__device__ __forceinline__ void sub_fwd(const RingFwdArgs& a, const RingSeg& seg, int paired,
+                                        void* raw) {
+  const int T = 1 << ((seg.body & (kPow2Body - 1)) - 4);
+  const RingOf ring(T, a.jobs, seg, paired, a.batch, raw);
+  const RingJob& job = ring.job;
+  const int n = job.nphi, t = ring.t;
+  const cplx* __restrict__ phase = a.chirp_pool + job.chirp_off;
+  cplx v[8];
+  load_pixels<8>(T, v, a, job, t, ring.b0, paired, ring.two);
+  sub_fft<false>(v, ring.lds, T, t, n, a.chirp_pool);
+  const double w = (a.apply_weight ? job.weight : 1.0) * ring_scale(a.norm_mode, n);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) v[e] = {w * v[e].x, w * v[e].y};
+  const bool ph = ring_phase(a.apply_phase, job);
+  residues_to_lds<8>(T, v, ring.lds, n, t, paired, [&](int e, cplx z) {
+    return ph ? cmul(z, phase[t + T * e]) : z;
+  });
+  if (ring.valid) store_columns(T, ring.lds, a, job, t, ring.b0, ring.two, ph);
+}
+
+__device__ __forceinline__ void sub_inv(const RingInvArgs& a, const RingSeg& seg, int paired,
+                                        void* raw) {
+  const int T = 1 << ((seg.body & (kPow2Body - 1)) - 4);
+  const RingOf ring(T, a.jobs, seg, paired, a.batch, raw);
+  const RingJob& job = ring.job;
+  const int n = job.nphi, t = ring.t;
+  const cplx* __restrict__ phase = a.chirp_pool + job.chirp_off;
+  const FoldIn in(a, job, ring.b0, ring.two);
+  cplx v[8], f[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const int p = t + T * e;
+    f[e] = in.ph && p < n ? phase[p] : cplx{1.0, 0.0};
+  }
+  in.residues(T, v, ring.lds, t);
+  const double w = (a.apply_weight ? job.weight : 1.0) * ring_scale(a.norm_mode, n);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) v[e] = tmul<true>(cplx{w * v[e].x, w * v[e].y}, f[e]);
+  __syncthreads();  // the partial sums are read
+  sub_fft<true>(v, ring.lds, T, t, n, a.chirp_pool);
+  if (ring.valid) store_pixels<8>(T, v, a, job, t, ring.b0, paired, ring.two, in.herm);
 }
 
 // e^{-i pi (t + T e) / N} of a power-of-two ring: e^{-i pi t / N} from the
@@ -852,19 +977,19 @@ __device__ __forceinline__ void pow2_fwd(const RingFwdArgs& a, const RingSeg& se
                                          void* raw) {
   typedef Pow2Shape<LOGN> P;
   constexpr int T = P::T, N = P::N;
-  const RingOf<T> ring(a.jobs, seg, paired, a.batch, raw);
+  const RingOf ring(T, a.jobs, seg, paired, a.batch, raw);
   const RingJob& job = ring.job;
   cplx* lds = ring.lds;
   const int t = ring.t;
   const cplx* __restrict__ tw = a.chirp_pool;
   cplx v[16];
-  load_pixels<T, 16>(v, a, job, t, ring.b0, paired, ring.two);
+  load_pixels<16>(T, v, a, job, t, ring.b0, paired, ring.two);
   pow2_fft<LOGN, false>(v, lds, t, tw);
   const double w = (a.apply_weight ? job.weight : 1.0) * ring_scale(a.norm_mode, N);
 #pragma unroll
   for (int e = 0; e < 16; ++e) v[e] = {w * v[e].x, w * v[e].y};
   const bool ph = ring_phase(a.apply_phase, job);
-  const cplx base = tw[t << (12 - LOGN)];
+  const cplx base = load_tw16(tw, 2 * T, t).w;
   if (seg.direct && paired) {
     // X and Y of the residues below N / 2 from z and the upper half's z'
     __syncthreads();
@@ -896,13 +1021,13 @@ __device__ __forceinline__ void pow2_fwd(const RingFwdArgs& a, const RingSeg& se
 #pragma unroll
       for (int e = 0; e < 16; ++e) v[e] = cmul(v[e], pow2_phase<LOGN>(base, e));
     }
-    if (ring.valid) store_direct<T, 16>(v, a, job, t, ring.b0, ph);
+    if (ring.valid) store_direct<16>(T, v, a, job, t, ring.b0, ph);
     return;
   }
-  residues_to_lds<T, 16>(v, lds, N, t, paired, [&](int e, cplx z) {
+  residues_to_lds<16>(T, v, lds, N, t, paired, [&](int e, cplx z) {
     return ph ? cmul(z, pow2_phase<LOGN>(base, e)) : z;
   });
-  if (ring.valid) store_columns<T>(lds, a, job, t, ring.b0, ring.two, ph);
+  if (ring.valid) store_columns(T, lds, a, job, t, ring.b0, ring.two, ph);
 }
 
 template <int LOGN>
@@ -910,24 +1035,24 @@ __device__ __forceinline__ void pow2_inv(const RingInvArgs& a, const RingSeg& se
                                          void* raw) {
   typedef Pow2Shape<LOGN> P;
   constexpr int T = P::T, N = P::N;
-  const RingOf<T> ring(a.jobs, seg, paired, a.batch, raw);
+  const RingOf ring(T, a.jobs, seg, paired, a.batch, raw);
   const RingJob& job = ring.job;
   cplx* lds = ring.lds;
   const int t = ring.t;
   const cplx* __restrict__ tw = a.chirp_pool;
   const FoldIn in(a, job, ring.b0, ring.two);
   cplx v[16];
-  in.template owned<T, 16>(v, t);
+  in.owned<16>(T, v, t);
   const double w = (a.apply_weight ? job.weight : 1.0) * ring_scale(a.norm_mode, N);
 #pragma unroll
   for (int e = 0; e < 16; ++e) v[e] = {w * v[e].x, w * v[e].y};
   if (in.ph) {
-    const cplx base = tw[t << (12 - LOGN)];
+    const cplx base = load_tw16(tw, 2 * T, t).w;
 #pragma unroll
     for (int e = 0; e < 16; ++e) v[e] = tmul<true>(v[e], pow2_phase<LOGN>(base, e));
   }
   pow2_fft<LOGN, true>(v, lds, t, tw);
-  if (ring.valid) store_pixels<T, 16>(v, a, job, t, ring.b0, paired, ring.two, in.herm);
+  if (ring.valid) store_pixels<16>(T, v, a, job, t, ring.b0, paired, ring.two, in.herm);
 }
 
 // Runs the body of this block's segment: those whose rings of T threads fit WG.
@@ -949,6 +1074,11 @@ __device__ __forceinline__ void ring_body(const Args& a, const RingSeg& seg, int
     }                                                                           \
     break;
   constexpr int kSpan = WG == 64 ? 16 : 8;
+  if (seg.body >= kSubBody) {
+    if constexpr (DIR == 0) sub_fwd(a, seg, paired, raw);
+    else sub_inv(a, seg, paired, raw);
+    return;
+  }
   switch (seg.body) {
     S2H_BLUE(6) S2H_BLUE(7) S2H_BLUE(8) S2H_BLUE(9) S2H_BLUE(10) S2H_BLUE(11) S2H_BLUE(12)
     S2H_BLUE(13)
@@ -1006,9 +1136,11 @@ RingSegs ring_segs(const JobSet& js) {
   RingSegs g{};
   int j0 = js.n_pow2;
   for (int c = kBlueClasses - 1; c >= 0; --c) {
-    if (!js.blue[c]) continue;
-    g.s[g.n++] = RingSeg{c + kBlueLogMin, j0, js.blue[c], 0, 0, shape_lds(c + kBlueLogMin)};
+    const int lg = c + kBlueLogMin;
+    if (js.blue[c]) g.s[g.n++] = RingSeg{lg, j0, js.blue[c], 0, 0, shape_lds(lg)};
     j0 += js.blue[c];
+    if (js.sub[c]) g.s[g.n++] = RingSeg{kSubBody + lg, j0, js.sub[c], 0, 0, shape_lds(lg)};
+    j0 += js.sub[c];
   }
   if (js.n_pow2)
     g.s[g.n++] = RingSeg{kPow2Body + js.log_pow2, 0, js.n_pow2, 0, 0, 1 << js.log_pow2};
@@ -1066,8 +1198,10 @@ hipError_t launch_rings(const Args& a, const RingSegs& g, unsigned gy, int paire
   const bool together = threads * gy <= (int64_t)kMergeBlocks * wg &&
                         narrow * (wg == 64 ? 16 : 8) >= wg && lds <= kRingLdsMax;
   if (together) return launch_segs<DIR>(a, g, 0, g.n, gy, paired, s);
-  for (int i = 0; i < g.n; ++i) {
-    const hipError_t e = launch_segs<DIR>(a, g, i, i + 1, gy, paired, s);
+  for (int i = 0, i1; i < g.n; i = i1) {
+    // the powers of two among the rings of one convolution length go with them
+    for (i1 = i + 1; i1 < g.n && g.s[i1].body == kSubBody + g.s[i].body;) ++i1;
+    const hipError_t e = launch_segs<DIR>(a, g, i, i1, gy, paired, s);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
@@ -1086,7 +1220,7 @@ unsigned grid_y(int batch, int paired) { return (unsigned)(paired ? (batch + 1) 
 
 hipError_t launch_ring_fft_forward(const RingFwdArgs& a0, const JobSet& js, int batch,
                                    hipStream_t s) {
-  if (batch == 0 || js.n_pow2 + js.n_blue == 0) return hipSuccess;
+  if (batch == 0 || js.n_pow2 + js.n_rest == 0) return hipSuccess;
   RingFwdArgs a = a0;
   a.jobs = js.jobs;
   a.batch = batch;
@@ -1094,11 +1228,11 @@ hipError_t launch_ring_fft_forward(const RingFwdArgs& a0, const JobSet& js, int 
   RingSegs g = ring_segs(js);
   for (int i = 0; i < g.n; ++i) {
     RingSeg& q = g.s[i];
-    if (q.body >= kPow2Body) {
+    if (q.body & kPow2Body) {
       q.direct = ring_direct(a, 1 << js.log_pow2, paired);
       if (!q.direct && paired) q.lds_ring *= 2;  // the residues of both maps
     } else {
-      q.direct = !paired && !a.apply_phase && ring_direct(a, js.min_blue, 0);
+      q.direct = !paired && !a.apply_phase && ring_direct(a, js.min_rest, 0);
     }
   }
   return launch_rings<0>(a, g, grid_y(batch, paired), paired, s);
@@ -1106,7 +1240,7 @@ hipError_t launch_ring_fft_forward(const RingFwdArgs& a0, const JobSet& js, int 
 
 hipError_t launch_ring_fft_inverse(const RingInvArgs& a0, const JobSet& js, int batch,
                                    hipStream_t s) {
-  if (batch == 0 || js.n_pow2 + js.n_blue == 0) return hipSuccess;
+  if (batch == 0 || js.n_pow2 + js.n_rest == 0) return hipSuccess;
   RingInvArgs a = a0;
   a.jobs = js.jobs;
   a.batch = batch;
