@@ -360,8 +360,10 @@ RingJob make_job(int64_t off, int nphi, int row, double phi0, double w, ChirpBui
   const bool direct = nphi == pow2 && (nphi & (nphi - 1)) == 0 && nphi >= 64;
   if (direct) return j;
   if ((nphi & (nphi - 1)) == 0) {
+    // on a ragged grid a whole wave at least: rings of several lengths in one wave would
+    // take the passes of each in turn (nside 16, one map, back: 13.6 -> 9.5 us)
     j.sub = 1;
-    j.conv_len = next_pow2(std::max(std::max(2 * nphi, 1 << kBlueLogMin), min_m));
+    j.conv_len = next_pow2(std::max({2 * nphi, 1 << kBlueLogMin, min_m ? std::max(min_m, 1024) : 0}));
     cb.add_sub(nphi, &j.chirp_off);
   } else {
     j.conv_len = cb.add_ring(nphi, &j.chirp_off, min_m);
