@@ -123,7 +123,11 @@ enum s2h_precision {
  * flags of s2h_inverse_ex: S2H_INV_REAL_OUTPUT writes float64 pixels for a
  * reality plan even where s2h_inverse_output_is_complex says complex (its
  * imaginary part is zero there); S2H_INV_SUBTRACT writes sub_from - I(flm)
- * (sub_from in the output layout, may alias f): a residual in one pass. */
+ * (sub_from in the output layout, may alias f): a residual in one pass.
+ * float64 pixels, and the input maps of reality plans, are transformed two at a
+ * time: a map 2k or 2k + 1 takes the rounding of the larger of the two, and a
+ * NaN or infinity reaches both.  Inverses that return complex128 transform every
+ * map alone. */
 enum { S2H_FWD_ACCUMULATE = 1 };
 enum { S2H_INV_REAL_OUTPUT = 1, S2H_INV_SUBTRACT = 2 };
 int s2h_forward_ex(const s2h_plan *plan, const void *f, int f_is_complex, void *flm,

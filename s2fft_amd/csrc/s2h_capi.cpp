@@ -311,9 +311,8 @@ int lat_forward_stage(const s2h_plan* p, const cplx* ftm, void* flm, int batch, 
     ProfScope prof(bf16 ? S2H_KERNEL_LAT_FORWARD_BF16
                         : mixed ? S2H_KERNEL_LAT_FORWARD_FP32 : S2H_KERNEL_LAT_FORWARD,
                    s);
-    // batches of 4 or more maps share each d-value across an 8-map MFMA tile;
-    // the mixed-precision projection always runs on the FP32 matrix cores
-    // multi-plane launches: the VALU kernel reads each map's own tables
+    // FP64: by valu_forward; the mixed-precision projection always runs on the FP32
+    // matrix cores; multi-plane launches: the VALU kernel reads each map's own tables
     if (valu)
       st = hip_status(launch_lat_forward(a, ps ? false : p->fwd_paired, s));
     else if (bf16)

@@ -8,10 +8,12 @@
 // data S (pair sum / difference of the ring Fourier coefficients, 8 maps x
 // re/im = 16 rows) sit in registers as A operands (A[i][k]: lane i + 16k).
 // The contraction over rings happens inside the MFMA; the waves of a
-// workgroup are summed through LDS in FP64 in a fixed order, workgroups of
-// one m with FP64 global atomics (2 per element at nside 1024, so the sum is
-// independent of their order).  Even and odd l (relative to m) form separate
-// 16-column tiles so that each uses one S (sum or difference).
+// workgroup are summed through LDS in FP64 in a fixed order.  The FP64 kernel
+// has one workgroup per m and adds its passes up by itself; the FP32 one adds
+// the workgroups of an m with FP64 global atomics (2 per element at nside
+// 1024, so the sum is independent of their order).  Even and odd l (relative
+// to m) form separate 16-column tiles so that each uses one S (sum or
+// difference).
 //
 // The recursion runs in its unit-c form (the plan's unit coefficients):
 // e_{l+1} = (a'_l x - b'_l) e_l - e_{l-1}, two FP64 operations per step,
@@ -19,8 +21,8 @@
 //
 // T = double: V_MFMA_F64_16X16X4F64, the plain FP64 transform.
 // T = float:  V_MFMA_F32_16X16X4F32 on FP32-rounded S and d with FP32
-//             accumulation over the ring pairs of a wave; the recursion and
-//             every sum beyond one wave stay FP64 (mixed precision).  This
+//             accumulation over 64 of a wave's rings; the recursion and every
+//             sum beyond stay FP64 (mixed precision).  This
 //             arithmetic has its own kernel, lat_forward_f32_kernel: 4 waves
 //             of 256 pairs, the d tiles double-buffered so that the recursion
 //             of one 64-pair set runs between the products of the previous
@@ -294,7 +296,7 @@ __global__ void __launch_bounds__(kFT, 2) lat_forward_f32_kernel(LatArgs a) {
   const Coef* __restrict__ cf = a.ucoef + (int64_t)am * L;  // unit-c: d_l = sigma_l e_l
   double* ctw = reinterpret_cast<double*>(&dt[0][wave][0][0]);
 
-  // recursion state and A operands as in lat_forward_mfma_kernel
+  // recursion state and A operands as in lat_forward_f64_kernel
   double x[kFSets], d[kFSets], dm1[kFSets];
   int ls[kFSets];
   float se[kFSets][16], so[kFSets][16];

@@ -41,15 +41,15 @@
 // 677 us from 2L + 1 rows (493 from L + 1; the column FFT chain 7.9 ms).
 //
 // What bounds it: 8 L^2 flops per complex element of the column on
-// V_MFMA_F64_16X16X4F64.  The operators are shared by every map, spin and
-// column of one parity, so they are stored packed in the A-operand order (a
-// wave's tile load is 512 contiguous bytes, resident in L2); the spectra are
-// the B operand, gathered straight into registers (16 lanes read 8 columns of
-// one parity; the wave of the other parity beside it uses the rest of the
-// lines).  No LDS; tile loads run ahead of the products by D K-steps.  At L =
-// 512, 64 spin-2 maps: 1.65 ms (42 TFLOP/s of products), and the projection of
-// half the rings 1.39 ms; the column FFT chain took 60.0 ms and the projection
-// 2.78 ms.  At L = 128, one map: 9.7 us (was 265 us).
+// V_MFMA_F64_16X16X4F64.  The operators are shared by every map, spin and column of one
+// parity, so they are stored packed in the A-operand order (a wave's tile load is 512
+// contiguous bytes, resident in L2).  Two kernels: theta_mix_kernel gathers the spectra
+// (the B operand) straight into registers, 16 lanes reading 8 columns of one parity while
+// the wave of the other parity beside it uses the rest of the lines, with loads D K-steps
+// ahead of the products (MW L = 128, one map: 9.7 us; the column FFT chain 265 us);
+// theta_mix_lds_kernel, for launches that fill the card, passes both through LDS (MW L =
+// 512, spin 2, 64 maps: 1.55 ms, 44 TFLOP/s of products, 1.69 from registers; the chain
+// 60.0 ms).  The projection of half the rings takes 1.03 ms there instead of 2.78.
 #include <map>
 #include <memory>
 #include <mutex>
@@ -537,7 +537,7 @@ __global__ void __launch_bounds__(256) theta_mix_kernel(MixKernelArgs a) {
 // column halves) share what they load and the matrix cores, not the L1's 64 bytes
 // per cycle, set the pace.  One workgroup: 64 rows of both parities x 64 columns;
 // a wave 4 row tiles x 2 column tiles; 16 input rows per LDS chunk, double-buffered
-// through registers (64 KB: two workgroups per CU).  The spectra are staged by
+// through registers (72 KB: two workgroups per CU).  The spectra are staged by
 // parity, (re, im) of 32 columns per input row, rows 640 bytes apart so that the two
 // rows of a half wave use all banks.  At MW L = 512, 64 maps the matrix cores are busy
 // for 68 % of its 1550 us (loads one chunk ahead instead of two: 2140 us).
